@@ -928,7 +928,6 @@ int fh_tune_set(fh_context* ctx, const char* name, int value) {
     if (!std::strcmp(name, "ntt_split") && value != 0 && !fh::ntt_split_ok(c.logN, value))
       throw fh::Error(FH_E_INVALID, "ntt_split " + std::to_string(value) + " is not built for logN " + std::to_string(c.logN));
     if (lo == 256 && value != 256 && value != 512) throw fh::Error(FH_E_INVALID, std::string(name) + " must be 256 or 512");
-    if (!std::strcmp(name, "ntt_split")) c.ensure_twists(value ? value : fh::ntt_default_split(c.logN));
     *slot = value;
   });
 }

@@ -27,6 +27,8 @@ struct PrimeConst {
   double ninv_d;      // N^-1 mod q, centred into (-q/2, q/2], as double
   uint64_t mont_ninv; // -q^-1 mod 2^64 (Montgomery reduction)
   uint64_t mont_r2;   // 2^128 mod q (to Montgomery form)
+  uint32_t lazy;      // 1 if q < 2^60 (the integer NTT keeps values up to 16 q)
+  float q32inv;       // 2^32 / q, rounded down
 };
 
 __device__ __forceinline__ uint64_t mulhi(uint64_t a, uint64_t b) { return __umul64hi(a, b); }

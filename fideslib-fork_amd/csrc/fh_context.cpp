@@ -346,45 +346,6 @@ static uint32_t bitrev(uint32_t x, int bits) {
   return r;
 }
 
-void Context::ensure_twists(int l1) {
-  if (l1 < 0 || l1 > 8 || l1 >= logN) throw Error(-1, "radix split out of range");
-  TwistSet& t = twists[l1];
-  if (t.tw) return;
-  // tau_r = psi^e_r, e_r = 1 + 2 brev_l1(r) - S1 (mod 2N)
-  const uint64_t m = 2ull * N;
-  const uint32_t S1 = 1u << l1, S2 = N >> l1;
-  std::vector<uint64_t> ts((size_t)np * N), tssh(ts.size()), its(ts.size()), itssh(ts.size());
-  std::vector<double> tsd(ts.size()), itsd(ts.size());
-  for (int i = 0; i < np; ++i) {
-    const uint64_t qi = q[i];
-    for (uint32_t r = 0; r < S1; ++r) {
-      const int64_t e = (1 + 2 * (int64_t)bitrev(r, l1) - (int64_t)S1) % (int64_t)m;
-      const uint64_t eu = (uint64_t)(e < 0 ? e + (int64_t)m : e);
-      const uint64_t step = h_powmod(psi[i], eu, qi), istep = h_powmod(psi[i], (m - eu) % m, qi);
-      uint64_t x = 1, xi = 1;
-      for (uint32_t c = 0; c < S2; ++c) {
-        const size_t o = (size_t)i * N + (size_t)r * S2 + c;
-        ts[o] = x;
-        its[o] = xi;
-        tssh[o] = h_shoup(x, qi);
-        itssh[o] = h_shoup(xi, qi);
-        tsd[o] = x > qi / 2 ? (double)x - (double)qi : (double)x;
-        itsd[o] = xi > qi / 2 ? (double)xi - (double)qi : (double)xi;
-        x = h_mulmod(x, step, qi);
-        xi = h_mulmod(xi, istep, qi);
-      }
-    }
-  }
-  TwistSet n;
-  n.tw = upload(ts);
-  n.tw_sh = upload(tssh);
-  n.itw = upload(its);
-  n.itw_sh = upload(itssh);
-  n.twd = upload(tsd);
-  n.itwd = upload(itsd);
-  t = n;
-}
-
 Context::Context(int logN_, int L1_, int K_, int dnum_, const std::vector<uint64_t>& primes)
     : logN(logN_), N(1u << logN_), L1(L1_), K(K_), dnum(dnum_) {
   if (logN < 10 || logN > 16) throw Error(-1, "logN must be in [10, 16]");
@@ -422,6 +383,10 @@ Context::Context(int logN_, int L1_, int K_, int dnum_, const std::vector<uint64
     // fp64 NTT: every intermediate stays below 2^53 when q < 2^50.2 (values are bounded by ~3.7q)
     P.fp64 = ((double)qi < 1.1487 * (double)(1ull << 50)) ? 1u : 0u;
     fp64[i] = (uint8_t)P.fp64;
+    P.lazy = qi < (1ull << 60) ? 1u : 0u;
+    // the quotient from it is never above the true one: the factor is rounded down by two ulps, more
+    // than the roundings of the converted high word and of the product take back
+    P.q32inv = (float)(4294967296.0 / (double)qi * (1.0 - 0x1p-22));
     P.ninv_d = P.ninv > qi / 2 ? (double)P.ninv - (double)qi : (double)P.ninv;
     P.mont_ninv = (uint64_t)0 - h_inv_odd(qi, 0);  // modulus 2^64: mask of m-1 = all ones
     P.mont_r2 = (uint64_t)(((((u128)1 << 64) % qi) * (((u128)1 << 64) % qi)) % qi);
@@ -448,7 +413,6 @@ Context::Context(int logN_, int L1_, int K_, int dnum_, const std::vector<uint64
   d_itw_sh = upload(itwsh);
   d_twd = upload(twd);
   d_itwd = upload(itwd);
-  ensure_twists(logN / 2);
 
   // ---- ModUp tables (OpenFHE PartQlHatInvModq / PartQlHatModp) ----
   const int E = L1 + K;

@@ -210,20 +210,6 @@ struct Context {
   uint64_t* d_itw_sh = nullptr;
   double* d_twd = nullptr;         // [np][N] twiddles as doubles (fp64 NTT path, q < 2^51)
   double* d_itwd = nullptr;
-  // Row twists of the two-pass NTT for radix split l1 (N = S1 x S2, S1 = 2^l1): after the column
-  // stages, row r is finished by a standard S2-point negacyclic transform of x_c tau_r^c, with
-  // tau_r = psi^(1 + 2 brev_l1(r) - S1); tw[r S2 + c] = tau_r^c, itw its inverse. Built at
-  // creation for the default split, on first use for another (ensure_twists).
-  struct TwistSet {
-    uint64_t* tw = nullptr;        // [np][N]
-    uint64_t* tw_sh = nullptr;
-    uint64_t* itw = nullptr;
-    uint64_t* itw_sh = nullptr;
-    double* twd = nullptr;         // centred doubles (fp64 path)
-    double* itwd = nullptr;
-  };
-  TwistSet twists[9];
-  void ensure_twists(int l1);
 
   // ModUp: for level l and digit d, source prescale [Qhat_i^-1]_{q_i} (+Shoup), and
   // [Qhat_i]_{p_j} for every extended position j of level l.

@@ -115,22 +115,12 @@ struct NttTables {
   const uint64_t* itw_sh;
   const double* twd;   // centred twiddles as doubles (fp64 path)
   const double* itwd;
-  const uint64_t* twist;     // row twists [np][N] and their inverses (Shoup companions, doubles)
-  const uint64_t* twist_sh;
-  const uint64_t* itwist;
-  const uint64_t* itwist_sh;
-  const double* twistd;
-  const double* itwistd;
   uint32_t N;
   uint32_t logN;
 };
 
-// tables of the two-pass NTT at radix split l1 (its row twists must have been built)
-inline NttTables ntt_tables(const Context& c, int l1) {
-  const Context::TwistSet& t = c.twists[l1];
-  if (!t.tw) throw Error(-1, "row twists of this radix split are not built");
-  return NttTables{c.d_prime, c.d_tw, c.d_tw_sh, c.d_itw, c.d_itw_sh, c.d_twd, c.d_itwd, t.tw, t.tw_sh,
-                   t.itw, t.itw_sh, t.twd, t.itwd, c.N, (uint32_t)c.logN};
+inline NttTables ntt_tables(const Context& c) {
+  return NttTables{c.d_prime, c.d_tw, c.d_tw_sh, c.d_itw, c.d_itw_sh, c.d_twd, c.d_itwd, c.N, (uint32_t)c.logN};
 }
 
 // NTT radix splits N = 2^l1 (column points) x 2^(logN - l1) (row points) the kernels are built

@@ -87,7 +87,6 @@ AutotuneResult autotune_ntt(Context& c, int polys) {
     constexpr double kGain = 0.95;
     for (int l1 = 4; l1 <= 8; ++l1) {
       if (l1 == l1d || !ntt_split_ok(c.logN, l1)) continue;
-      c.ensure_twists(l1);
       c.tune.ntt_split = l1;
       const double t = measure();
       if (t < best * kGain) best = t, best_split = l1;

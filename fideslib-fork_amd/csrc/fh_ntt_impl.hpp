@@ -10,10 +10,8 @@
 //  * N = S1 * S2 (S1 = 2^l1 "column" points, S2 = 2^l2 "row" points). The first
 //    l1 stages only couple elements of one column (stride S2), the last l2
 //    stages only elements of one row (contiguous), so a limb is transformed by
-//    two launches. Row rho's stages equal a standard S2-point negacyclic
-//    transform of x_c tau_rho^c (tau_rho = psi^(1 + 2 brev(rho) - S1)), so the row
-//    launch multiplies by a per-element twist table once and then uses the
-//    same S2 twiddles (kept in LDS) for every row, like the column launch. Each lane owns 16 elements of one sub-transform: four radix-2
+//    two launches: the column launch with the table's first S1 twiddles in LDS, the row launch with
+//    each row's own twiddles straight from the table. Each lane owns 16 elements of one sub-transform: four radix-2
 //    stages run in registers, one LDS exchange re-partitions the sub-transform,
 //    the remaining stages run in registers again. Global loads and stores are
 //    coalesced in both passes (rows are staged through LDS where the register
@@ -26,8 +24,8 @@
 //        three times the rate of a 64-bit Shoup product built from 32-bit
 //        multiplies. Values are re-centred into (-q/2, q/2] every few stages so
 //        every intermediate stays an exact integer below 2^53.
-//      - integer Harvey-lazy Shoup for the 60-bit primes: forward values in
-//        [0, 4q), inverse values in [0, 2q).
+//      - integer Shoup for the 60-bit primes, lazily reduced: up to 16 q below 2^60
+//        (IntL), up to 4 q below 2^62 (IntA).
 //    Both are exact, so the canonical outputs are identical.
 //  * Between the two launches the limb holds an internal form (lazy integers or
 //    doubles). A batch may be split into chunks of limbs (tunable "ntt_chunk_mb")
@@ -38,6 +36,7 @@
 #pragma once
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "fh_kernels.hpp"
 
@@ -48,34 +47,100 @@ namespace {
 // workgroup sizes the passes are built for (the default and the wide tile)
 constexpr int kNttThreads = 256, kNttWide = 512;
 
+// Every arithmetic's butterflies and settling steps carry the bound of each value, in units of the
+// prime, in an int the caller keeps per register (b: |x| or x < b q). The loops are fully unrolled
+// and start from constants, so the bounds fold away; only IntL acts on them.
+
 // ------------------------------------------------------------------------------- integer arithmetic
+// Primes below 2^60: sixteen multiples of q fit a word, so a value is reduced only where its bound
+// would pass 16 q instead of in every butterfly. The quotient product is exact (Shoup), the low words
+// are formed as y w + h (-q) mod 2^64, and a multiple of q that keeps a difference positive is
+// shifted in with the same add. A forward butterfly costs 22 VALU instructions instead of 29.
+struct IntL {
+  using T = uint64_t;
+  static constexpr int kMid = 16;   // bound of a value between the passes of a forward transform
+  uint64_t q, nq;                   // nq = -q mod 2^64
+  float q32inv;                     // 2^32 / q, rounded down: the quotient of a value below 16 q
+  struct W {
+    uint64_t w, sh;
+  };
+  __device__ __forceinline__ T from_canon(uint64_t v) const { return v; }
+  __device__ __forceinline__ T from_mid(uint64_t v) const { return v; }
+  __device__ __forceinline__ uint64_t to_mid(T v) const { return v; }
+  // x w mod q in [0, 2q) for any x < 2^64
+  __device__ __forceinline__ T mul(T x, W w) const { return x * w.w + mulhi(x, w.sh) * nq; }
+  __device__ __forceinline__ void sub8(T& x, int& b) const {
+    const uint64_t m = q << 3;
+    x = x >= m ? x - m : x;
+    b = b - 8 > 8 ? b - 8 : 8;
+  }
+  // x mod q up to one q, for b <= 16: the quotient (< 16) from the high word in fp32, rounded down
+  // by at most one
+  __device__ __forceinline__ T below2(T x) const {
+    const uint32_t h = (uint32_t)((float)(uint32_t)(x >> 32) * q32inv);
+    return x + (uint64_t)h * nq;
+  }
+  __device__ __forceinline__ void fwd(T& X, T& Y, W w, int& bx, int& by) const {
+    if (bx + 2 > 16) sub8(X, bx);
+    const uint64_t t = mul(Y, w), x2 = X + (q << 1);
+    X = X + t;
+    Y = x2 - t;
+    bx = by = bx + 2;
+  }
+  static __device__ __forceinline__ constexpr int log2_up(int b) { return b <= 1 ? 0 : b <= 2 ? 1 : b <= 4 ? 2 : b <= 8 ? 3 : 4; }
+  __device__ __forceinline__ void inv(T& X, T& Y, W w, int& bx, int& by) const {
+    if (bx + (1 << log2_up(by)) > 16) {
+      if (bx > 8) sub8(X, bx);
+      if (by > 8) sub8(Y, by);
+    }
+    const uint64_t v = X + (q << log2_up(by)) - Y;
+    X = X + Y;
+    Y = mul(v, w);
+    bx = bx + by;
+    by = 2;
+  }
+  __device__ __forceinline__ void settle_fwd(T&, int&) const {}
+  __device__ __forceinline__ void settle_mid(T&, int&) const {}
+  __device__ __forceinline__ void settle_inv(T& x, int& b) const {
+    if (b > 2) x = below2(x);
+    b = 2;
+  }
+  __device__ __forceinline__ uint64_t canon(T x, int b) const {
+    if (b > 2) x = below2(x);
+    return x >= q ? x - q : x;
+  }
+};
+
+// Primes from 2^60 to 2^62: only four multiples of q fit, forward values stay in [0, 4q), inverse
+// values in [0, 2q), reduced in every butterfly.
 struct IntA {
   using T = uint64_t;
+  static constexpr int kMid = 1;
   uint64_t q, q2;
   struct W {
     uint64_t w, sh;
   };
-  __device__ __forceinline__ W tw(const uint64_t* t, const uint64_t* tsh, uint32_t i) const { return W{t[i], tsh[i]}; }
   __device__ __forceinline__ T from_canon(uint64_t v) const { return v; }
   __device__ __forceinline__ T from_mid(uint64_t v) const { return v; }
   __device__ __forceinline__ uint64_t to_mid(T v) const { return v; }
-  __device__ __forceinline__ void fwd(T& X, T& Y, W w) const {
+  __device__ __forceinline__ T mul(T x, W w) const { return shoup_lazy(x, w.w, w.sh, q); }
+  __device__ __forceinline__ void fwd(T& X, T& Y, W w, int&, int&) const {
     uint64_t x = X >= q2 ? X - q2 : X;         // [0, 2q)
     uint64_t t = shoup_lazy(Y, w.w, w.sh, q);  // [0, 2q)
     X = x + t;                                 // [0, 4q)
     Y = x - t + q2;                            // [0, 4q)
   }
-  __device__ __forceinline__ void inv(T& X, T& Y, W w) const {
+  __device__ __forceinline__ void inv(T& X, T& Y, W w, int&, int&) const {
     uint64_t u = X + Y;                        // X, Y in [0, 2q)
     u = u >= q2 ? u - q2 : u;
     uint64_t v = X - Y + q2;                   // [0, 4q)
     X = u;
     Y = shoup_lazy(v, w.w, w.sh, q);           // [0, 2q)
   }
-  __device__ __forceinline__ void recenter(T&) const {}
-  // x * w for any x < 2^64, result in [0, 2q)
-  __device__ __forceinline__ T mul(T x, W w) const { return shoup_lazy(x, w.w, w.sh, q); }
-  __device__ __forceinline__ uint64_t canon(T x) const {
+  __device__ __forceinline__ void settle_fwd(T&, int&) const {}
+  __device__ __forceinline__ void settle_mid(T&, int&) const {}
+  __device__ __forceinline__ void settle_inv(T&, int&) const {}
+  __device__ __forceinline__ uint64_t canon(T x, int) const {
     x = x >= q2 ? x - q2 : x;
     return x >= q ? x - q : x;
   }
@@ -85,10 +150,10 @@ struct IntA {
 struct FpA {
   using T = double;
   using W = double;
+  static constexpr int kMid = 1;
   double q, qinv, half;
-  __device__ __forceinline__ W tw(const double* t, const double*, uint32_t i) const { return t[i]; }
   // y * w mod q for |y| < 4q, |w| <= q/2: exact, result in about (-1.3q, 1.3q)
-  __device__ __forceinline__ double mulmod(double y, double w) const {
+  __device__ __forceinline__ double mul(double y, double w) const {
     const double h = y * w;
     const double l = fma(y, w, -h);
     const double c = rint(h * qinv);
@@ -101,30 +166,65 @@ struct FpA {
   }
   __device__ __forceinline__ T from_mid(uint64_t v) const { return __longlong_as_double((long long)v); }
   __device__ __forceinline__ uint64_t to_mid(T v) const { return (uint64_t)__double_as_longlong(v); }
-  __device__ __forceinline__ void fwd(T& X, T& Y, W w) const {
-    const double t = mulmod(Y, w);
+  __device__ __forceinline__ void fwd(T& X, T& Y, W w, int&, int&) const {
+    const double t = mul(Y, w);
     Y = X - t;
     X = X + t;
   }
-  __device__ __forceinline__ void inv(T& X, T& Y, W w) const {
+  __device__ __forceinline__ void inv(T& X, T& Y, W w, int&, int&) const {
     const double u = X + Y, v = X - Y;
     X = u;
-    Y = mulmod(v, w);
+    Y = mul(v, w);
   }
   __device__ __forceinline__ void recenter(T& x) const { x = fma(-rint(x * qinv), q, x); }
-  // x * w re-centred into [-q/2, q/2]
-  __device__ __forceinline__ T mul(T x, W w) const {
-    T r = mulmod(x, w);
-    recenter(r);
-    return r;
-  }
-  __device__ __forceinline__ uint64_t canon(T x) const {
+  // forward values are re-centred after every four stages, inverse values (whose sums double) after
+  // every second
+  __device__ __forceinline__ void settle_fwd(T& x, int&) const { recenter(x); }
+  __device__ __forceinline__ void settle_mid(T& x, int&) const { recenter(x); }
+  __device__ __forceinline__ void settle_inv(T& x, int&) const { recenter(x); }
+  __device__ __forceinline__ uint64_t canon(T x, int) const {
     recenter(x);
     x = x < 0 ? x + q : x;
     x = x >= q ? x - q : x;
     return (uint64_t)x;
   }
 };
+
+// twiddle i of a table (and of its Shoup companion)
+__device__ __forceinline__ double tw_at(const FpA&, const double* t, const double*, uint32_t i) { return t[i]; }
+template <class A>
+__device__ __forceinline__ typename A::W tw_at(const A&, const uint64_t* t, const uint64_t* tsh, uint32_t i) {
+  return typename A::W{t[i], tsh[i]};
+}
+
+// CNT consecutive twiddles from index i (a multiple of CNT, tables 16-byte aligned), 16 bytes a load
+template <int CNT>
+__device__ __forceinline__ void tw_load(const FpA&, double* w, const double* t, const double*, size_t i) {
+  if constexpr (CNT == 1) {
+    w[0] = t[i];
+  } else {
+#pragma unroll
+    for (int k = 0; k < CNT; k += 2) {
+      const double2 v = *reinterpret_cast<const double2*>(t + i + k);
+      w[k] = v.x;
+      w[k + 1] = v.y;
+    }
+  }
+}
+template <int CNT, class A>
+__device__ __forceinline__ void tw_load(const A&, typename A::W* w, const uint64_t* t, const uint64_t* tsh, size_t i) {
+  if constexpr (CNT == 1) {
+    w[0] = typename A::W{t[i], tsh[i]};
+  } else {
+#pragma unroll
+    for (int k = 0; k < CNT; k += 2) {
+      const ulonglong2 v = *reinterpret_cast<const ulonglong2*>(t + i + k);
+      const ulonglong2 h = *reinterpret_cast<const ulonglong2*>(tsh + i + k);
+      w[k] = typename A::W{v.x, h.x};
+      w[k + 1] = typename A::W{v.y, h.y};
+    }
+  }
+}
 
 // Loads of the second pass. PlainLd: ordinary loads (the two-launch form: the first launch's
 // stores are visible to the next launch). L2Ld: loads that skip the CU's L1 (sc0) and are served by
@@ -140,30 +240,47 @@ struct L2Ld {
 };
 
 // per-limb arithmetic selection
+enum : int { kArithFp = 0, kArithLazy = 1, kArithWide = 2 };
 struct Sel {
-  bool fp;
-  IntA ia;
+  int kind;
   FpA fa;
+  IntL il;
+  IntA ia;
   const uint64_t *tw, *twsh;
   const double* twd;
-  const uint64_t *ts, *tssh;   // row twists of the limb's prime (forward: tau^c, inverse: tau^-c)
-  const double* tsd;
 };
 
 __device__ __forceinline__ Sel select(const NttTables& tb, int pid, bool inverse) {
   const PrimeConst& P = tb.prime[pid];
   Sel s;
-  s.fp = P.fp64 != 0;
-  s.ia = IntA{P.q, 2 * P.q};
+  s.kind = P.fp64 ? kArithFp : P.lazy ? kArithLazy : kArithWide;
   s.fa = FpA{P.qd, P.qinv, 0.5 * P.qd};
+  s.il = IntL{P.q, 0 - P.q, P.q32inv};
+  s.ia = IntA{P.q, 2 * P.q};
   const size_t o = (size_t)pid * tb.N;
   s.tw = (inverse ? tb.itw : tb.tw) + o;
   s.twsh = (inverse ? tb.itw_sh : tb.tw_sh) + o;
   s.twd = (inverse ? tb.itwd : tb.twd) + o;
-  s.ts = (inverse ? tb.itwist : tb.twist) + o;
-  s.tssh = (inverse ? tb.itwist_sh : tb.twist_sh) + o;
-  s.tsd = (inverse ? tb.itwistd : tb.twistd) + o;
   return s;
+}
+
+// f(arithmetic, twiddle table, its Shoup companion) with the limb's arithmetic; the choice is
+// uniform over the workgroup
+template <class F>
+__device__ __forceinline__ void with_arith(const Sel& s, F&& f) {
+  if (s.kind == kArithFp) f(s.fa, s.twd, s.twd);
+  else if (s.kind == kArithLazy) f(s.il, s.tw, s.twsh);
+  else f(s.ia, s.tw, s.twsh);
+}
+
+// the first n twiddles of the table into LDS (w; Shoup companions into wsh)
+template <class A, class TwT>
+__device__ __forceinline__ void stage_tw(const A&, uint64_t* w, uint64_t* wsh, const TwT* t, const TwT* tsh, int n) {
+  TwT* d = reinterpret_cast<TwT*>(w);
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    d[i] = t[i];
+    if constexpr (sizeof(typename A::W) == 16) wsh[i] = tsh[i];
+  }
 }
 
 // Thread index policies of the pass bodies. Inside a loop (the team kernels run their limbs in
@@ -182,18 +299,14 @@ struct OpaqueTid {
 };
 
 // ------------------------------------------------------------------------------- forward, columns
-// First l1 stages. Input: canonical (in place or out of place), output: internal form.
-template <int LS, class Tid = PlainTid, class A, class TwT>
-__device__ __forceinline__ void fwd_cols_body(const A& ar, const TwT* sw, const TwT* swp, const uint64_t* p, uint64_t* po,
-                                              uint64_t* tile, uint32_t N2, int C, uint32_t bx) {
-  constexpr int S = 1 << LS, T = S / 16, PADS = S + 1;
-  const int tid = Tid::get();
-  const int cc = tid % C, r0 = tid / C;
-  const uint32_t col = bx * C + cc;
-  typename A::T x[16];
+// The l1 stages of one column held by T = S / 16 threads, 16 elements each: in: element k at row
+// r0 + T k (bound 1), out: at row 16 r0 + k (LS > 4, through the column's LDS slot t) or r0 + T k.
+template <int LS, class A, class TwT>
+__device__ __forceinline__ void fwd_cols_stages(const A& ar, typename A::T (&x)[16], const TwT* sw, const TwT* swp, uint64_t* t, int r0) {
+  constexpr int S = 1 << LS, T = S / 16;
+  int b[16];
 #pragma unroll
-  for (int k = 0; k < 16; ++k) x[k] = ar.from_canon(p[(size_t)(r0 + T * k) * N2 + col]);
-  __syncthreads();
+  for (int k = 0; k < 16; ++k) b[k] = 1;
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
     const int h = 8 >> s;
@@ -201,13 +314,12 @@ __device__ __forceinline__ void fwd_cols_body(const A& ar, const TwT* sw, const 
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const int idx = (1 << s) + (k >> (4 - s));
-      ar.fwd(x[k], x[k + h], ar.tw(sw, swp, idx));
+      ar.fwd(x[k], x[k + h], tw_at(ar, sw, swp, idx), b[k], b[k + h]);
     }
   }
 #pragma unroll
-  for (int k = 0; k < 16; ++k) ar.recenter(x[k]);
+  for (int k = 0; k < 16; ++k) ar.settle_fwd(x[k], b[k]);
   if constexpr (LS > 4) {
-    uint64_t* t = tile + cc * PADS;
 #pragma unroll
     for (int k = 0; k < 16; ++k) t[r0 + T * k] = ar.to_mid(x[k]);
     __syncthreads();
@@ -220,14 +332,31 @@ __device__ __forceinline__ void fwd_cols_body(const A& ar, const TwT* sw, const 
       for (int k = 0; k < 16; ++k) {
         if (k & h) continue;
         const int idx = (1 << s) + ((16 * r0 + k) >> (LS - s));
-        ar.fwd(x[k], x[k + h], ar.tw(sw, swp, idx));
+        ar.fwd(x[k], x[k + h], tw_at(ar, sw, swp, idx), b[k], b[k + h]);
       }
     }
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      ar.recenter(x[k]);
-      po[(size_t)(16 * r0 + k) * N2 + col] = ar.to_mid(x[k]);
-    }
+    for (int k = 0; k < 16; ++k) ar.settle_fwd(x[k], b[k]);
+  }
+}
+
+// First l1 stages. Input: canonical (in place or out of place), output: internal form.
+template <int LS, class Tid = PlainTid, class A, class TwT>
+__device__ __forceinline__ void fwd_cols_body(const A& ar, const TwT* tw, const TwT* twsh, uint64_t* sw, uint64_t* swp, const uint64_t* p,
+                                              uint64_t* po, uint64_t* tile, uint32_t N2, int C, uint32_t bx) {
+  constexpr int S = 1 << LS, T = S / 16, PADS = S + 1;
+  const int tid = Tid::get();
+  const int cc = tid % C, r0 = tid / C;
+  const uint32_t col = bx * C + cc;
+  typename A::T x[16];
+  stage_tw(ar, sw, swp, tw, twsh, S);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) x[k] = ar.from_canon(p[(size_t)(r0 + T * k) * N2 + col]);
+  __syncthreads();
+  fwd_cols_stages<LS>(ar, x, (const TwT*)sw, (const TwT*)swp, tile + cc * PADS, r0);
+  if constexpr (LS > 4) {
+#pragma unroll
+    for (int k = 0; k < 16; ++k) po[(size_t)(16 * r0 + k) * N2 + col] = ar.to_mid(x[k]);
   } else {
 #pragma unroll
     for (int k = 0; k < 16; ++k) po[(size_t)(r0 + T * k) * N2 + col] = ar.to_mid(x[k]);
@@ -246,14 +375,9 @@ __global__ __launch_bounds__(TH) void k_ntt_fwd_cols(Addr ad, AddrOut ao, NttTab
   const Sel sel = select(tb, pid, false);
   const int C = blockDim.x / T;
   const uint32_t N2 = tb.N >> LS;
-  if (sel.fp) {
-    double* swd = reinterpret_cast<double*>(sw);
-    for (int i = threadIdx.x; i < S; i += blockDim.x) swd[i] = sel.twd[i];
-    fwd_cols_body<LS>(sel.fa, (const double*)swd, (const double*)swd, p, po, tile, N2, C, blockIdx.x);
-  } else {
-    for (int i = threadIdx.x; i < S; i += blockDim.x) { sw[i] = sel.tw[i]; swp[i] = sel.twsh[i]; }
-    fwd_cols_body<LS>(sel.ia, (const uint64_t*)sw, (const uint64_t*)swp, p, po, tile, N2, C, blockIdx.x);
-  }
+  with_arith(sel, [&](const auto& ar, const auto* tw, const auto* twsh) {
+    fwd_cols_body<LS>(ar, tw, twsh, sw, swp, p, po, tile, N2, C, blockIdx.x);
+  });
 }
 
 // ------------------------------------------------------------------------------- row tiles in LDS
@@ -270,80 +394,159 @@ struct RowTile {
 };
 
 // ------------------------------------------------------------------------------- forward, rows
-// Last l2 stages. Row rho of the intermediate is finished by a standard S2-point negacyclic
-// transform of x_c tau_rho^c (c = position in the row): one coalesced twist multiply per element,
-// then stages whose twiddles are the first S2 entries of the table, the same for every row, read
-// from LDS. Input: internal form, output: canonical residues handed to the epilogue.
+// Last l2 stages. Stage s of row rho uses the 2^s table entries from 2^(l1 + s) + rho 2^s on. Over a
+// row's stages every lane needs 15 of them that its row shares and up to 15 that are its own, each
+// group contiguous, so they are read straight from the table in 16-byte loads (the table's words
+// each once per limb) and cost neither LDS space nor a staging barrier. Input: internal form, output:
+// canonical residues handed to the epilogue. Against one coalesced twist multiply per element and
+// shared twiddles from LDS, the inverse row passes of one rotation (25 and 18 limbs, N=2^16) went
+// from 43 to 30 us; with thousands of limbs the pass is bound by HBM and the two forms tie.
 //
-// fwd_rows_core: the stages of one row (at `row`, its first word at limb position rbase) by the T
-// threads of row slot rr of the tile. With LS > 4 the canonical outputs end in the LDS tile (word
-// rsw(c0 + T k) of the slot holds position c0 + T k) after a barrier, where the row pass's store
-// phase and the fused key inner product read them; with LS <= 4 (no LDS exchange) they go to the
-// epilogue directly.
-template <int LS, class Ld = PlainLd, class A, class TwT, class Epi>
-__device__ __forceinline__ void fwd_rows_core(const A& ar, const TwT* sw, const TwT* swp, const TwT* ts, const TwT* tsp, const uint64_t* row,
-                                              uint32_t rbase, uint64_t* tile, int rr, int c0, const Epi& epi) {
+// Twiddles of a row's stages: `shared` for stage s < 4 (2^s entries, the same for the row's lanes),
+// `own` for stage s >= 4 (this lane's 16 >> (LS - s)). The fp64 path requests a phase's 15 words
+// together, ahead of the barrier or the data they meet; the integer paths (two words each) load
+// stage by stage, which keeps four waves per SIMD.
+template <int LS, class A>
+struct RowTw {
+  using W = typename A::W;
+  static constexpr bool kAhead = sizeof(W) == 8;
+  static constexpr int kOwn4 = LS > 4 ? 16 >> (LS - 4) : 0;
+  W w[kAhead ? 15 : 8];
+  template <int s, class TwT>
+  __device__ __forceinline__ void load_shared(const A& ar, const TwT* tw, const TwT* twsh, int l1, uint32_t rho) {
+    tw_load<(1 << s)>(ar, w + (kAhead ? (1 << s) - 1 : 0), tw, twsh, ((size_t)1 << (l1 + s)) + ((size_t)rho << s));
+  }
+  template <int s, class TwT>
+  __device__ __forceinline__ void load_own(const A& ar, const TwT* tw, const TwT* twsh, int l1, uint32_t rho, int c0) {
+    if constexpr (s >= 4 && s < LS)
+      tw_load<(16 >> (LS - s))>(ar, w + (kAhead ? kOwn4 * ((1 << (s - 4)) - 1) : 0), tw, twsh,
+                                ((size_t)1 << (l1 + s)) + ((size_t)rho << s) + ((16u * c0) >> (LS - s)));
+  }
+  template <class TwT>
+  __device__ __forceinline__ void ahead_shared(const A& ar, const TwT* tw, const TwT* twsh, int l1, uint32_t rho) {
+    if constexpr (kAhead) {
+      load_shared<0>(ar, tw, twsh, l1, rho);
+      load_shared<1>(ar, tw, twsh, l1, rho);
+      load_shared<2>(ar, tw, twsh, l1, rho);
+      load_shared<3>(ar, tw, twsh, l1, rho);
+    }
+  }
+  template <class TwT>
+  __device__ __forceinline__ void ahead_own(const A& ar, const TwT* tw, const TwT* twsh, int l1, uint32_t rho, int c0) {
+    if constexpr (kAhead) {
+      load_own<4>(ar, tw, twsh, l1, rho, c0);
+      load_own<5>(ar, tw, twsh, l1, rho, c0);
+      load_own<6>(ar, tw, twsh, l1, rho, c0);
+      load_own<7>(ar, tw, twsh, l1, rho, c0);
+    }
+  }
+  template <int s, class TwT>
+  __device__ __forceinline__ const W* shared(const A& ar, const TwT* tw, const TwT* twsh, int l1, uint32_t rho) {
+    if constexpr (kAhead) return w + (1 << s) - 1;
+    load_shared<s>(ar, tw, twsh, l1, rho);
+    return w;
+  }
+  template <int s, class TwT>
+  __device__ __forceinline__ const W* own(const A& ar, const TwT* tw, const TwT* twsh, int l1, uint32_t rho, int c0) {
+    if constexpr (kAhead) return w + kOwn4 * ((1 << (s - 4)) - 1);
+    load_own<s>(ar, tw, twsh, l1, rho, c0);
+    return w;
+  }
+};
+
+// fwd_rows_core: the stages of row rho (its first word at `row`) by the T threads of row slot rr of
+// the tile. With LS > 4 the canonical outputs end in the LDS tile (word rsw(c0 + T k) of the slot
+// holds position c0 + T k) after a barrier, where the row pass's store phase and the fused key inner
+// product read them; with LS <= 4 (no LDS exchange) they stay in x (position c0 + T k).
+// `before_barrier` runs ahead of the last barrier (the epilogue's loads are issued there).
+template <int LS, class Ld = PlainLd, class A, class TwT, class F>
+__device__ __forceinline__ void fwd_rows_core(const A& ar, const TwT* tw, const TwT* twsh, int l1, const uint64_t* row, uint32_t rho,
+                                              uint64_t* tile, int rr, int c0, uint64_t (&out)[16], F&& before_barrier) {
   constexpr int S = 1 << LS, T = S / 16, PADS = RowTile<LS>::PAD;
   typename A::T x[16];
+  int b[16];
+  RowTw<LS, A> rt;
 #pragma unroll
-  for (int k = 0; k < 16; ++k) x[k] = ar.from_mid(Ld::ld(row + c0 + T * k));
-#pragma unroll
-  for (int k = 0; k < 16; ++k) x[k] = ar.mul(x[k], ar.tw(ts + rbase, tsp + rbase, c0 + T * k));
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    const int h = 8 >> s;
+  for (int k = 0; k < 16; ++k) {
+    x[k] = ar.from_mid(Ld::ld(row + c0 + T * k));
+    b[k] = A::kMid;
+  }
+  rt.ahead_shared(ar, tw, twsh, l1, rho);
+  auto stage = [&](auto sc) {
+    constexpr int s = decltype(sc)::value, h = 8 >> s;
+    const typename A::W* w = rt.template shared<s>(ar, tw, twsh, l1, rho);
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
-      const int idx = (1 << s) + (k >> (4 - s));
-      ar.fwd(x[k], x[k + h], ar.tw(sw, swp, idx));
+      ar.fwd(x[k], x[k + h], w[k >> (4 - s)], b[k], b[k + h]);
     }
-  }
+  };
+  stage(std::integral_constant<int, 0>{});
+  stage(std::integral_constant<int, 1>{});
+  stage(std::integral_constant<int, 2>{});
+  stage(std::integral_constant<int, 3>{});
   if constexpr (LS > 4) {
     uint64_t* t = tile + rr * PADS;
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
-      ar.recenter(x[k]);
+      ar.settle_fwd(x[k], b[k]);
       t[rsw(c0 + T * k)] = ar.to_mid(x[k]);
     }
+    rt.ahead_own(ar, tw, twsh, l1, rho, c0);
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 16; ++k) x[k] = ar.from_mid(t[rsw(16 * c0 + k)]);
+    auto own = [&](auto sc) {
+      constexpr int s = decltype(sc)::value;
+      if constexpr (s < LS) {
+        constexpr int h = S >> (s + 1);
+        const typename A::W* w = rt.template own<s>(ar, tw, twsh, l1, rho, c0);
 #pragma unroll
-    for (int s = 4; s < LS; ++s) {
-      const int h = S >> (s + 1);
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        if (k & h) continue;
-        const int idx = (1 << s) + ((16 * c0 + k) >> (LS - s));
-        ar.fwd(x[k], x[k + h], ar.tw(sw, swp, idx));
+        for (int k = 0; k < 16; ++k) {
+          if (k & h) continue;
+          ar.fwd(x[k], x[k + h], w[k >> (LS - s)], b[k], b[k + h]);
+        }
       }
-    }
+    };
+    own(std::integral_constant<int, 4>{});
+    own(std::integral_constant<int, 5>{});
+    own(std::integral_constant<int, 6>{});
+    own(std::integral_constant<int, 7>{});
     // each thread rewrites exactly the LDS words it read: no barrier needed before the store
 #pragma unroll
-    for (int k = 0; k < 16; ++k) t[rsw(16 * c0 + k)] = ar.canon(x[k]);
+    for (int k = 0; k < 16; ++k) t[rsw(16 * c0 + k)] = ar.canon(x[k], b[k]);
+    before_barrier();
     __syncthreads();
-  } else {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) epi.store(const_cast<uint64_t*>(row), rbase, c0 + T * k, ar.canon(x[k]));
+    for (int k = 0; k < 16; ++k) out[k] = t[rsw(c0 + T * k)];
+  } else {
+    before_barrier();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) out[k] = ar.canon(x[k], b[k]);
   }
 }
 
+// The epilogue's operands are loaded together before any result is stored: a store in between would
+// make every following load wait for it, since the compiler cannot rule out that they overlap
+// (N=2^16, ModDown epilogue, with the change of the twiddles: 3200 limbs 1229 -> 1029 us, 50 limbs
+// 29.9 -> 21.6 us).
 template <int LS, class Ld = PlainLd, class A, class TwT, class Epi>
-__device__ __forceinline__ void fwd_rows_body(const A& ar, const TwT* sw, const TwT* swp, const TwT* ts, const TwT* tsp, uint64_t* p,
-                                              uint64_t* tile, int R, const Epi& epi, uint32_t bx) {
-  constexpr int S = 1 << LS, T = S / 16, PADS = RowTile<LS>::PAD;
+__device__ __forceinline__ void fwd_rows_body(const A& ar, const TwT* tw, const TwT* twsh, int l1, uint64_t* p, uint64_t* tile, int R,
+                                              const Epi& epi, uint32_t bx) {
+  constexpr int S = 1 << LS, T = S / 16;
   const int tid = threadIdx.x;
   const int rr = tid / T, c0 = tid % T;
   const uint32_t rho = bx * R + rr;
   uint64_t* row = p + (size_t)rho * S;
   const uint32_t rbase = rho * S;
-  fwd_rows_core<LS, Ld>(ar, sw, swp, ts, tsp, row, rbase, tile, rr, c0, epi);
-  if constexpr (LS > 4) {
-    const uint64_t* t = tile + rr * PADS;
+  uint64_t v[16];
+  typename Epi::In in[16];
+  fwd_rows_core<LS, Ld>(ar, tw, twsh, l1, row, rho, tile, rr, c0, v, [&] {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) epi.store(row, rbase, c0 + T * k, t[rsw(c0 + T * k)]);
-  }
+    for (int k = 0; k < 16; ++k) in[k] = epi.load(rbase + c0 + T * k);
+  });
+#pragma unroll
+  for (int k = 0; k < 16; ++k) epi.store(row, rbase, c0 + T * k, v[k], in[k]);
 }
 
 // ------------------------------------------------------------------------------- forward epilogues
@@ -353,8 +556,10 @@ __device__ __forceinline__ void fwd_rows_body(const A& ar, const TwT* sw, const 
 // combination x_i * [q_l^-1]_{q_i} + v (src/NTTfusions.cuh:214-235). Job y addresses
 // (poly, limb) = (y % npolys, y / npolys), the order of SetAddr.
 struct EpiStore {
+  struct In {};
   __device__ __forceinline__ void init(uint32_t, uint32_t, const PrimeConst*) {}
-  __device__ __forceinline__ void store(uint64_t* row, uint32_t, uint32_t j, uint64_t v) const { row[j] = v; }
+  __device__ __forceinline__ In load(uint32_t) const { return In{}; }
+  __device__ __forceinline__ void store(uint64_t* row, uint32_t, uint32_t j, uint64_t v, In) const { row[j] = v; }
 };
 
 struct EpiModDown {
@@ -377,8 +582,10 @@ struct EpiModDown {
     wi = w[i];
     wish = wsh[i];
   }
-  __device__ __forceinline__ void store(uint64_t*, uint32_t rbase, uint32_t j, uint64_t v) const {
-    oi[rbase + j] = shoup(sub_mod(xi[rbase + j], v, q), wi, wish, q);
+  using In = uint64_t;
+  __device__ __forceinline__ In load(uint32_t j) const { return xi[j]; }
+  __device__ __forceinline__ void store(uint64_t*, uint32_t rbase, uint32_t j, uint64_t v, In x) const {
+    oi[rbase + j] = shoup(sub_mod(x, v, q), wi, wish, q);
   }
 };
 
@@ -399,136 +606,149 @@ struct EpiRescale {
     wi = w[i];
     wish = wsh[i];
   }
-  __device__ __forceinline__ void store(uint64_t*, uint32_t rbase, uint32_t j, uint64_t v) const {
-    oi[rbase + j] = add_mod(shoup(xi[rbase + j], wi, wish, q), v, q);
+  using In = uint64_t;
+  __device__ __forceinline__ In load(uint32_t j) const { return xi[j]; }
+  __device__ __forceinline__ void store(uint64_t*, uint32_t rbase, uint32_t j, uint64_t v, In x) const {
+    oi[rbase + j] = add_mod(shoup(x, wi, wish, q), v, q);
   }
 };
 
 template <int LS, int TH, class Addr, class Epi>
-__global__ __launch_bounds__(TH) void k_ntt_fwd_rows(Addr ad, NttTables tb, Epi epi) {
+__global__ __launch_bounds__(TH) __attribute__((amdgpu_waves_per_eu(4))) void k_ntt_fwd_rows(Addr ad, NttTables tb, Epi epi) {
   constexpr int S = 1 << LS, T = S / 16, PADS = RowTile<LS>::PAD, RMAX = TH / T;
   __shared__ uint64_t tile[RMAX * PADS];
-  __shared__ uint64_t sw[S], swp[S];
   uint64_t* p;
   int pid;
   ad.at(blockIdx.y, tb.N, p, pid);
   epi.init(blockIdx.y, tb.N, tb.prime);
   const Sel sel = select(tb, pid, false);
   const int R = blockDim.x / T;
-  if (sel.fp) {
-    double* swd = reinterpret_cast<double*>(sw);
-    for (int i = threadIdx.x; i < S; i += blockDim.x) swd[i] = sel.twd[i];
-    __syncthreads();
-    fwd_rows_body<LS>(sel.fa, (const double*)swd, (const double*)swd, sel.tsd, sel.tsd, p, tile, R, epi, blockIdx.x);
-  } else {
-    for (int i = threadIdx.x; i < S; i += blockDim.x) { sw[i] = sel.tw[i]; swp[i] = sel.twsh[i]; }
-    __syncthreads();
-    fwd_rows_body<LS>(sel.ia, (const uint64_t*)sw, (const uint64_t*)swp, sel.ts, sel.tssh, p, tile, R, epi, blockIdx.x);
-  }
+  with_arith(sel, [&](const auto& ar, const auto* tw, const auto* twsh) {
+    fwd_rows_body<LS>(ar, tw, twsh, (int)tb.logN - LS, p, tile, R, epi, blockIdx.x);
+  });
 }
 
 // ------------------------------------------------------------------------------- inverse, rows
-// First launch of the INTT: the inverse of the forward row transform, i.e. the standard S2-point
-// Gentleman-Sande stages (first S2 entries of the inverse table, from LDS) followed by one
-// coalesced multiply by tau_rho^-c. Input: canonical, output: internal form. fp64 values are
-// re-centred after every second stage (Gentleman-Sande sums double per stage).
+// First launch of the INTT: the inverse of the forward row pass (Gentleman-Sande stages with the
+// inverse table's entries at the same indices). Input: canonical, output: internal form.
 template <int LS, class A, class TwT>
-__device__ __forceinline__ void inv_rows_body(const A& ar, const TwT* sw, const TwT* swp, const TwT* ts, const TwT* tsp, const uint64_t* p,
-                                              uint64_t* po, uint64_t* tile, int R, uint32_t bx) {
+__device__ __forceinline__ void inv_rows_body(const A& ar, const TwT* tw, const TwT* twsh, int l1, const uint64_t* p, uint64_t* po,
+                                              uint64_t* tile, int R, uint32_t bx) {
   constexpr int S = 1 << LS, T = S / 16, PADS = RowTile<LS>::PAD;
   const int tid = threadIdx.x;
   const int rr = tid / T, c0 = tid % T;
   const uint32_t rho = bx * R + rr;
   const uint64_t* row = p + (size_t)rho * S;
   uint64_t* rowo = po + (size_t)rho * S;
-  const uint32_t rbase = rho * S;
   uint64_t* t = tile + rr * PADS;
   typename A::T x[16];
-  if constexpr (LS > 4) {
+  int b[16];
+  RowTw<LS, A> rt;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) t[rsw(c0 + T * k)] = row[c0 + T * k];
+  for (int k = 0; k < 16; ++k) b[k] = 1;
+  if constexpr (LS > 4) {
+    uint64_t in[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) in[k] = row[c0 + T * k];
+    rt.ahead_own(ar, tw, twsh, l1, rho, c0);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) t[rsw(c0 + T * k)] = in[k];
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 16; ++k) x[k] = ar.from_canon(t[rsw(16 * c0 + k)]);
+    auto own = [&](auto sc) {
+      constexpr int s = decltype(sc)::value;
+      if constexpr (s < LS) {
+        constexpr int h = S >> (s + 1);
+        const typename A::W* w = rt.template own<s>(ar, tw, twsh, l1, rho, c0);
 #pragma unroll
-    for (int s = LS - 1; s >= 4; --s) {
-      const int h = S >> (s + 1);
+        for (int k = 0; k < 16; ++k) {
+          if (k & h) continue;
+          ar.inv(x[k], x[k + h], w[k >> (LS - s)], b[k], b[k + h]);
+        }
+        if (((LS - s) & 1) == 0 && s != 4) {
 #pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        if (k & h) continue;
-        const int idx = (1 << s) + ((16 * c0 + k) >> (LS - s));
-        ar.inv(x[k], x[k + h], ar.tw(sw, swp, idx));
+          for (int k = 0; k < 16; ++k) ar.settle_mid(x[k], b[k]);
+        }
       }
-      if (((LS - s) & 1) == 0) {
-#pragma unroll
-        for (int k = 0; k < 16; ++k) ar.recenter(x[k]);
-      }
-    }
+    };
+    own(std::integral_constant<int, 7>{});
+    own(std::integral_constant<int, 6>{});
+    own(std::integral_constant<int, 5>{});
+    own(std::integral_constant<int, 4>{});
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
-      ar.recenter(x[k]);
+      ar.settle_inv(x[k], b[k]);
       t[rsw(16 * c0 + k)] = ar.to_mid(x[k]);
     }
+    rt.ahead_shared(ar, tw, twsh, l1, rho);
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; ++k) x[k] = ar.from_mid(t[rsw(c0 + T * k)]);
+    for (int k = 0; k < 16; ++k) {
+      x[k] = ar.from_mid(t[rsw(c0 + T * k)]);
+      b[k] = 2;
+    }
   } else {
 #pragma unroll
     for (int k = 0; k < 16; ++k) x[k] = ar.from_canon(row[c0 + T * k]);
+    rt.ahead_shared(ar, tw, twsh, l1, rho);
   }
-#pragma unroll
-  for (int s = 3; s >= 0; --s) {
-    const int h = 8 >> s;
+  auto stage = [&](auto sc) {
+    constexpr int s = decltype(sc)::value, h = 8 >> s;
+    const typename A::W* w = rt.template shared<s>(ar, tw, twsh, l1, rho);
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
-      const int idx = (1 << s) + (k >> (4 - s));
-      ar.inv(x[k], x[k + h], ar.tw(sw, swp, idx));
+      ar.inv(x[k], x[k + h], w[k >> (4 - s)], b[k], b[k + h]);
     }
-    if ((s & 1) == 0) {
+    if (s == 2) {
 #pragma unroll
-      for (int k = 0; k < 16; ++k) ar.recenter(x[k]);
+      for (int k = 0; k < 16; ++k) ar.settle_mid(x[k], b[k]);
     }
+  };
+  stage(std::integral_constant<int, 3>{});
+  stage(std::integral_constant<int, 2>{});
+  stage(std::integral_constant<int, 1>{});
+  stage(std::integral_constant<int, 0>{});
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    ar.settle_inv(x[k], b[k]);
+    rowo[c0 + T * k] = ar.to_mid(x[k]);
   }
-#pragma unroll
-  for (int k = 0; k < 16; ++k) rowo[c0 + T * k] = ar.to_mid(ar.mul(x[k], ar.tw(ts + rbase, tsp + rbase, c0 + T * k)));
 }
 
 template <int LS, int TH, class Addr, class AddrOut>
-__global__ __launch_bounds__(TH) void k_ntt_inv_rows(Addr ad, AddrOut ao, NttTables tb) {
+__global__ __launch_bounds__(TH) __attribute__((amdgpu_waves_per_eu(4))) void k_ntt_inv_rows(Addr ad, AddrOut ao, NttTables tb) {
   constexpr int S = 1 << LS, T = S / 16, PADS = RowTile<LS>::PAD, RMAX = TH / T;
   __shared__ uint64_t tile[RMAX * PADS];
-  __shared__ uint64_t sw[S], swp[S];
   uint64_t *p, *po;
   int pid, pido;
   ad.at(blockIdx.y, tb.N, p, pid);
   ao.at(blockIdx.y, tb.N, po, pido);
   const Sel sel = select(tb, pid, true);
   const int R = blockDim.x / T;
-  if (sel.fp) {
-    double* swd = reinterpret_cast<double*>(sw);
-    for (int i = threadIdx.x; i < S; i += blockDim.x) swd[i] = sel.twd[i];
-    __syncthreads();
-    inv_rows_body<LS>(sel.fa, (const double*)swd, (const double*)swd, sel.tsd, sel.tsd, p, po, tile, R, blockIdx.x);
-  } else {
-    for (int i = threadIdx.x; i < S; i += blockDim.x) { sw[i] = sel.tw[i]; swp[i] = sel.twsh[i]; }
-    __syncthreads();
-    inv_rows_body<LS>(sel.ia, (const uint64_t*)sw, (const uint64_t*)swp, sel.ts, sel.tssh, p, po, tile, R, blockIdx.x);
-  }
+  with_arith(sel, [&](const auto& ar, const auto* tw, const auto* twsh) {
+    inv_rows_body<LS>(ar, tw, twsh, (int)tb.logN - LS, p, po, tile, R, blockIdx.x);
+  });
 }
 
 // ------------------------------------------------------------------------------- inverse, columns
 // Second launch of the INTT (first l1 stages, reversed) with the N^-1 scaling. Input: internal
 // form, output: canonical residues.
-template <int LS, class Ld = PlainLd, class Tid = PlainTid, class A, class TwT, class Fin>
-__device__ __forceinline__ void inv_cols_body(const A& ar, const TwT* sw, const TwT* swp, uint64_t* p, uint64_t* tile, uint32_t N2,
-                                              int C, const Fin& fin, uint32_t bx) {
+template <int LS, class Ld = PlainLd, class Tid = PlainTid, class A, class TwT>
+__device__ __forceinline__ void inv_cols_body(const A& ar, const TwT* tw, const TwT* twsh, uint64_t* swb, uint64_t* swpb, uint64_t* p,
+                                              uint64_t* tile, uint32_t N2, int C, typename A::W fin, uint32_t bx) {
   constexpr int S = 1 << LS, T = S / 16, PADS = S + 1;
   const int tid = Tid::get();
   const int cc = tid % C, r0 = tid / C;
   const uint32_t col = bx * C + cc;
+  stage_tw(ar, swb, swpb, tw, twsh, S);
+  const TwT *sw = (const TwT*)swb, *swp = (const TwT*)swpb;
   typename A::T x[16];
+  int b[16];
   uint64_t* t = tile + cc * PADS;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) b[k] = 2;
   if constexpr (LS > 4) {
 #pragma unroll
     for (int k = 0; k < 16; ++k) x[k] = ar.from_mid(Ld::ld(p + (size_t)(16 * r0 + k) * N2 + col));
@@ -540,21 +760,24 @@ __device__ __forceinline__ void inv_cols_body(const A& ar, const TwT* sw, const 
       for (int k = 0; k < 16; ++k) {
         if (k & h) continue;
         const int idx = (1 << s) + ((16 * r0 + k) >> (LS - s));
-        ar.inv(x[k], x[k + h], ar.tw(sw, swp, idx));
+        ar.inv(x[k], x[k + h], tw_at(ar, sw, swp, idx), b[k], b[k + h]);
       }
-      if (((LS - s) & 1) == 0) {
+      if (((LS - s) & 1) == 0 && s != 4) {
 #pragma unroll
-        for (int k = 0; k < 16; ++k) ar.recenter(x[k]);
+        for (int k = 0; k < 16; ++k) ar.settle_mid(x[k], b[k]);
       }
     }
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
-      ar.recenter(x[k]);
+      ar.settle_inv(x[k], b[k]);
       t[16 * r0 + k] = ar.to_mid(x[k]);
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; ++k) x[k] = ar.from_mid(t[r0 + T * k]);
+    for (int k = 0; k < 16; ++k) {
+      x[k] = ar.from_mid(t[r0 + T * k]);
+      b[k] = 2;
+    }
   } else {
 #pragma unroll
     for (int k = 0; k < 16; ++k) x[k] = ar.from_mid(Ld::ld(p + (size_t)(r0 + T * k) * N2 + col));
@@ -567,33 +790,27 @@ __device__ __forceinline__ void inv_cols_body(const A& ar, const TwT* sw, const 
     for (int k = 0; k < 16; ++k) {
       if (k & h) continue;
       const int idx = (1 << s) + (k >> (4 - s));
-      ar.inv(x[k], x[k + h], ar.tw(sw, swp, idx));
+      ar.inv(x[k], x[k + h], tw_at(ar, sw, swp, idx), b[k], b[k + h]);
     }
-    if ((s & 1) == 0) {
+    if (s == 2) {
 #pragma unroll
-      for (int k = 0; k < 16; ++k) ar.recenter(x[k]);
+      for (int k = 0; k < 16; ++k) ar.settle_mid(x[k], b[k]);
     }
   }
+  // N^-1: a product by a constant, which takes what the last two stages leave unsettled
 #pragma unroll
-  for (int k = 0; k < 16; ++k) p[(size_t)(r0 + T * k) * N2 + col] = fin(x[k]);
+  for (int k = 0; k < 16; ++k) p[(size_t)(r0 + T * k) * N2 + col] = ar.canon(ar.mul(x[k], fin), 2);
 }
 
-struct IntFin {
-  IntA a;
-  uint64_t s, ssh;
-  __device__ __forceinline__ uint64_t operator()(uint64_t v) const {
-    uint64_t r = shoup_lazy(v, s, ssh, a.q);
-    return r >= a.q ? r - a.q : r;
-  }
-};
-struct FpFin {
-  FpA a;
-  double s;
-  __device__ __forceinline__ uint64_t operator()(double v) const { return a.canon(a.mulmod(v, s)); }
-};
+// N^-1 mod the prime as the arithmetic's twiddle
+__device__ __forceinline__ double ninv_of(const FpA&, const PrimeConst& P) { return P.ninv_d; }
+template <class A>
+__device__ __forceinline__ typename A::W ninv_of(const A&, const PrimeConst& P) {
+  return typename A::W{P.ninv, P.ninv_sh};
+}
 
 template <int LS, int TH, class Addr>
-__global__ __launch_bounds__(TH) void k_ntt_inv_cols(Addr ad, NttTables tb) {
+__global__ __launch_bounds__(TH) __attribute__((amdgpu_waves_per_eu(4))) void k_ntt_inv_cols(Addr ad, NttTables tb) {
   constexpr int S = 1 << LS, T = S / 16, PADS = S + 1, CMAX = TH / T;
   __shared__ uint64_t tile[CMAX * PADS];
   __shared__ uint64_t sw[S], swp[S];
@@ -601,17 +818,11 @@ __global__ __launch_bounds__(TH) void k_ntt_inv_cols(Addr ad, NttTables tb) {
   int pid;
   ad.at(blockIdx.y, tb.N, p, pid);
   const Sel sel = select(tb, pid, true);
-  const PrimeConst& P = tb.prime[pid];
   const int C = blockDim.x / T;
   const uint32_t N2 = tb.N >> LS;
-  if (sel.fp) {
-    double* swd = reinterpret_cast<double*>(sw);
-    for (int i = threadIdx.x; i < S; i += blockDim.x) swd[i] = sel.twd[i];
-    inv_cols_body<LS>(sel.fa, (const double*)swd, (const double*)swd, p, tile, N2, C, FpFin{sel.fa, P.ninv_d}, blockIdx.x);
-  } else {
-    for (int i = threadIdx.x; i < S; i += blockDim.x) { sw[i] = sel.tw[i]; swp[i] = sel.twsh[i]; }
-    inv_cols_body<LS>(sel.ia, (const uint64_t*)sw, (const uint64_t*)swp, p, tile, N2, C, IntFin{sel.ia, P.ninv, P.ninv_sh}, blockIdx.x);
-  }
+  with_arith(sel, [&](const auto& ar, const auto* tw, const auto* twsh) {
+    inv_cols_body<LS>(ar, tw, twsh, sw, swp, p, tile, N2, C, ninv_of(ar, tb.prime[pid]), blockIdx.x);
+  });
 }
 
 // ------------------------------------------------------------------------------- team form
@@ -703,6 +914,14 @@ __device__ __forceinline__ bool team_setup(const TeamArgs& ta, uint32_t& team, u
   return true;
 }
 
+// f with the limb's arithmetic, in a kernel of one class (FP: the fp64 path, else the integer paths)
+template <bool FP, class F>
+__device__ __forceinline__ void team_arith(const Sel& s, F&& f) {
+  if constexpr (FP) f(s.fa, s.twd, s.twd);
+  else if (s.kind == kArithLazy) f(s.il, s.tw, s.twsh);
+  else f(s.ia, s.tw, s.twsh);
+}
+
 // Each workgroup runs its limbs software-pipelined: the first pass of the team's next limb is done
 // before waiting for the current limb's team barrier, so the barrier's latency hides behind a pass
 // of work; two limbs per team are in flight (two alternating counter slots, targets W per use).
@@ -739,16 +958,9 @@ __global__ __launch_bounds__(TH) __attribute__((amdgpu_waves_per_eu(3))) void k_
     ao.at(y, tb.N, po, pido);
     const Sel sel = select(tb, pid, false);
     __syncthreads();   // earlier readers of sw / tile are done
-    if constexpr (FP) {
-      double* swd = reinterpret_cast<double*>(sw);
-      for (int i = threadIdx.x; i < S; i += TH) swd[i] = sel.twd[i];
-      __syncthreads();
-      fwd_cols_body<LS, OpaqueTid>(sel.fa, (const double*)swd, (const double*)swd, p, po, tile, N2, C, opaque(m));
-    } else {
-      for (int i = threadIdx.x; i < S; i += TH) { sw[i] = sel.tw[i]; swp[i] = sel.twsh[i]; }
-      __syncthreads();
-      fwd_cols_body<LS, OpaqueTid>(sel.ia, (const uint64_t*)sw, (const uint64_t*)swp, p, po, tile, N2, C, opaque(m));
-    }
+    team_arith<FP>(sel, [&](const auto& ar, const auto* tw, const auto* twsh) {
+      fwd_cols_body<LS, OpaqueTid>(ar, tw, twsh, sw, swp, p, po, tile, N2, C, opaque(m));
+    });
     team_arrive(slot + (k & 1), formal);
   };
   auto pass2 = [&](uint32_t y) {
@@ -760,16 +972,9 @@ __global__ __launch_bounds__(TH) __attribute__((amdgpu_waves_per_eu(3))) void k_
     e.init(y, tb.N, tb.prime);
     const Sel sel = select(tb, pid, false);
     __syncthreads();
-    if constexpr (FP) {
-      double* swd = reinterpret_cast<double*>(sw);
-      for (int i = threadIdx.x; i < S; i += TH) swd[i] = sel.twd[i];
-      __syncthreads();
-      fwd_rows_body<LS, L2Ld>(sel.fa, (const double*)swd, (const double*)swd, sel.tsd, sel.tsd, po, tile, C, e, opaque(m));
-    } else {
-      for (int i = threadIdx.x; i < S; i += TH) { sw[i] = sel.tw[i]; swp[i] = sel.twsh[i]; }
-      __syncthreads();
-      fwd_rows_body<LS, L2Ld>(sel.ia, (const uint64_t*)sw, (const uint64_t*)swp, sel.ts, sel.tssh, po, tile, C, e, opaque(m));
-    }
+    team_arith<FP>(sel, [&](const auto& ar, const auto* tw, const auto* twsh) {
+      fwd_rows_body<LS, L2Ld>(ar, tw, twsh, (int)tb.logN - LS, po, tile, C, e, opaque(m));
+    });
   };
   uint32_t y = team < ta.njobs && mine(team) ? team : next(team);
   uint32_t k = 0;
@@ -815,16 +1020,9 @@ __global__ __launch_bounds__(TH) __attribute__((amdgpu_waves_per_eu(3))) void k_
     ao.at(y, tb.N, po, pido);
     const Sel sel = select(tb, pid, true);
     __syncthreads();
-    if constexpr (FP) {
-      double* swd = reinterpret_cast<double*>(sw);
-      for (int i = threadIdx.x; i < S; i += TH) swd[i] = sel.twd[i];
-      __syncthreads();
-      inv_rows_body<LS>(sel.fa, (const double*)swd, (const double*)swd, sel.tsd, sel.tsd, p, po, tile, C, opaque(m));
-    } else {
-      for (int i = threadIdx.x; i < S; i += TH) { sw[i] = sel.tw[i]; swp[i] = sel.twsh[i]; }
-      __syncthreads();
-      inv_rows_body<LS>(sel.ia, (const uint64_t*)sw, (const uint64_t*)swp, sel.ts, sel.tssh, p, po, tile, C, opaque(m));
-    }
+    team_arith<FP>(sel, [&](const auto& ar, const auto* tw, const auto* twsh) {
+      inv_rows_body<LS>(ar, tw, twsh, (int)tb.logN - LS, p, po, tile, C, opaque(m));
+    });
     team_arrive(slot + (k & 1), formal);
   };
   auto pass2 = [&](uint32_t y) {
@@ -833,19 +1031,10 @@ __global__ __launch_bounds__(TH) __attribute__((amdgpu_waves_per_eu(3))) void k_
     ad.at(y, tb.N, p, pid);
     ao.at(y, tb.N, po, pido);
     const Sel sel = select(tb, pid, true);
-    const PrimeConst& P = tb.prime[pid];
     __syncthreads();
-    if constexpr (FP) {
-      double* swd = reinterpret_cast<double*>(sw);
-      for (int i = threadIdx.x; i < S; i += TH) swd[i] = sel.twd[i];
-      __syncthreads();
-      inv_cols_body<LS, L2Ld, OpaqueTid>(sel.fa, (const double*)swd, (const double*)swd, po, tile, N2, C, FpFin{sel.fa, P.ninv_d}, opaque(m));
-    } else {
-      for (int i = threadIdx.x; i < S; i += TH) { sw[i] = sel.tw[i]; swp[i] = sel.twsh[i]; }
-      __syncthreads();
-      inv_cols_body<LS, L2Ld, OpaqueTid>(sel.ia, (const uint64_t*)sw, (const uint64_t*)swp, po, tile, N2, C, IntFin{sel.ia, P.ninv, P.ninv_sh},
-                              opaque(m));
-    }
+    team_arith<FP>(sel, [&](const auto& ar, const auto* tw, const auto* twsh) {
+      inv_cols_body<LS, L2Ld, OpaqueTid>(ar, tw, twsh, sw, swp, po, tile, N2, C, ninv_of(ar, tb.prime[pid]), opaque(m));
+    });
   };
   uint32_t y = team < ta.njobs && mine(team) ? team : next(team);
   uint32_t k = 0;
@@ -905,10 +1094,12 @@ struct EpiModDownJobs {
     wi = w[j.pid];
     wish = wsh[j.pid];
   }
-  __device__ __forceinline__ void store(uint64_t*, uint32_t rbase, uint32_t jj, uint64_t v) const {
-    uint64_t r = shoup(sub_mod(xi[rbase + jj], v, q), wi, wish, q);
-    if (ai) r = add_mod(ai[rbase + jj], r, q);
-    oi[rbase + jj] = r;
+  struct In {
+    uint64_t x, a;
+  };
+  __device__ __forceinline__ In load(uint32_t j) const { return In{xi[j], ai ? ai[j] : 0}; }
+  __device__ __forceinline__ void store(uint64_t*, uint32_t rbase, uint32_t jj, uint64_t v, In e) const {
+    oi[rbase + jj] = add_mod(e.a, shoup(sub_mod(e.x, v, q), wi, wish, q), q);
   }
 };
 
@@ -935,9 +1126,12 @@ struct EpiRescaleJobs {
     wi = w[o];
     wish = wsh[o];
   }
-  __device__ __forceinline__ void store(uint64_t*, uint32_t rbase, uint32_t jj, uint64_t v) const {
-    uint64_t x = xi[rbase + jj];
-    if (pti) x = mul_mod(x, pti[rbase + jj], P);
+  struct In {
+    uint64_t x, pt;
+  };
+  __device__ __forceinline__ In load(uint32_t j) const { return In{xi[j], pti ? pti[j] : 0}; }
+  __device__ __forceinline__ void store(uint64_t*, uint32_t rbase, uint32_t jj, uint64_t v, In e) const {
+    const uint64_t x = pti ? mul_mod(e.x, e.pt, P) : e.x;
     oi[rbase + jj] = add_mod(shoup(x, wi, wish, P.q), v, P.q);
   }
 };
@@ -947,7 +1141,9 @@ struct ShiftEpi {
   Epi e;
   uint32_t base;
   __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime) { e.init(y + base, N, prime); }
-  __device__ __forceinline__ void store(uint64_t* row, uint32_t rbase, uint32_t j, uint64_t v) const { e.store(row, rbase, j, v); }
+  using In = typename Epi::In;
+  __device__ __forceinline__ In load(uint32_t j) const { return e.load(j); }
+  __device__ __forceinline__ void store(uint64_t* row, uint32_t rbase, uint32_t j, uint64_t v, In in) const { e.store(row, rbase, j, v, in); }
 };
 
 // limbs per chunk: the intermediate of one chunk stays MALL-resident between the two launches
@@ -1100,7 +1296,7 @@ struct ChunkStreams {
 
 template <class Addr, class AddrOut, int L1S, int L2S, bool WIDE, class Epi>
 void fwd_impl(const Context& c, const Addr& ad, const AddrOut& ao, uint32_t nlimbs, hipStream_t st0, const Epi& epi, const char* rows_name) {
-  NttTables tb = ntt_tables(c, L1S);
+  NttTables tb = ntt_tables(c);
   if constexpr (L1S == L2S && L1S >= 6) {
     if (team_ok<L1S, L2S>(c, st0) && launch_fwd_team<L1S>(c, ad, ao, nlimbs, tb, st0, epi, rows_name)) return;
   }
@@ -1128,7 +1324,7 @@ void fwd_impl(const Context& c, const Addr& ad, const AddrOut& ao, uint32_t nlim
 
 template <class Addr, class AddrOut, int L1S, int L2S, bool WIDE>
 void inv_impl(const Context& c, const Addr& ad, const AddrOut& ao, uint32_t nlimbs, hipStream_t st0) {
-  NttTables tb = ntt_tables(c, L1S);
+  NttTables tb = ntt_tables(c);
   if constexpr (L1S == L2S && L1S >= 6) {
     if (team_ok<L1S, L2S>(c, st0) && launch_inv_team<L1S>(c, ad, ao, nlimbs, tb, st0)) return;
   }

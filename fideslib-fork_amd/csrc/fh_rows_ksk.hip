@@ -55,7 +55,6 @@ __global__ __launch_bounds__(TH) void k_ntt_rows_ksk(RowsKskParams kp, RowsKskIt
   constexpr int S = 1 << LS, T = S / 16, PADS = RowTile<LS>::PAD, RMAX = TH / T;
   static_assert(LS > 4, "the fused row pass reads its outputs from the LDS tile");
   __shared__ uint64_t tile[RMAX * PADS];
-  __shared__ uint64_t sw[S], swp[S];
   const uint32_t per = (kp.total + 7) / 8;
   const uint32_t J = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
   if (J >= kp.total) return;  // the whole workgroup: J is uniform
@@ -68,20 +67,9 @@ __global__ __launch_bounds__(TH) void k_ntt_rows_ksk(RowsKskParams kp, RowsKskIt
   const int tid = threadIdx.x, rr = tid / T, c0 = tid % T;
   const int R = blockDim.x / T;
   const uint32_t rbase = (tl * (uint32_t)R + (uint32_t)rr) * S;
-  if (sel.fp) {
-    double* swd = reinterpret_cast<double*>(sw);
-    for (int k = tid; k < S; k += blockDim.x) swd[k] = sel.twd[k];
-  } else {
-    for (int k = tid; k < S; k += blockDim.x) {
-      sw[k] = sel.tw[k];
-      swp[k] = sel.twsh[k];
-    }
-  }
-  __syncthreads();
   const size_t N = kp.N, E = (size_t)kp.L1 + kp.K;
   const uint32_t own_d = pos < kp.lq ? pos / kp.alpha : ~0u;
   const uint64_t* key = it.key[g];
-  const uint64_t* t = tile + rr * PADS;
   uint64_t a0[16], a1[16];
 #pragma unroll
   for (int k = 0; k < 16; ++k) a0[k] = a1[k] = 0;
@@ -95,12 +83,9 @@ __global__ __launch_bounds__(TH) void k_ntt_rows_ksk(RowsKskParams kp, RowsKskIt
       // every thread reads back only the tile words it wrote last (positions c0 + T k of its row
       // slot), so the next digit's first LDS writes need no barrier
       const uint64_t* row = kp.digits + b * kp.dig_stride + ((size_t)d * kp.ext + pos) * N + rbase;
-      if (sel.fp)
-        fwd_rows_core<LS>(sel.fa, (const double*)sw, (const double*)sw, sel.tsd, sel.tsd, row, rbase, tile, rr, c0, EpiStore{});
-      else
-        fwd_rows_core<LS>(sel.ia, (const uint64_t*)sw, (const uint64_t*)swp, sel.ts, sel.tssh, row, rbase, tile, rr, c0, EpiStore{});
-#pragma unroll
-      for (int k = 0; k < 16; ++k) x[k] = t[rsw(c0 + T * k)];
+      with_arith(sel, [&](const auto& ar, const auto* tw, const auto* twsh) {
+        fwd_rows_core<LS>(ar, tw, twsh, (int)tb.logN - LS, row, rbase / S, tile, rr, c0, x, [] {});
+      });
     }
     const uint64_t* kb = key + ((size_t)(2 * d) * E + pid) * N + rbase;
     const uint64_t* ka = kb + E * N;
@@ -132,7 +117,7 @@ int split_of(const Context& c) { return c.tune.ntt_split ? c.tune.ntt_split : nt
 // the column pass alone over the ModUp targets (up to 65535 limbs per launch)
 template <int L1S, bool WIDE>
 void modup_cols(const Context& c, const ModUpAddr& m, uint32_t n, hipStream_t st) {
-  const NttTables tb = ntt_tables(c, L1S);
+  const NttTables tb = ntt_tables(c);
   for (uint32_t base = 0; base < n; base += 65535) {
     const uint32_t cnt = std::min<uint32_t>(65535, n - base);
     const Shift<ModUpAddr> sa{m, base};
@@ -144,7 +129,7 @@ void modup_cols(const Context& c, const ModUpAddr& m, uint32_t n, hipStream_t st
 template <int L1S, int L2S>
 void rows_ksk_launch(const Context& c, const RowsKskParams& kp0, const RowsKskItems& it, hipStream_t st) {
   if constexpr (L2S > 4 && L2S <= 8) {
-    const NttTables tb = ntt_tables(c, L1S);
+    const NttTables tb = ntt_tables(c);
     const dim3 blk = row_block<L2S, kNttThreads>(c.N);
     const uint32_t R = blk.x / ((1u << L2S) / 16);
     RowsKskParams kp = kp0;
