@@ -16,6 +16,7 @@
 #include <tuple>
 
 #include "fh_batch.hpp"
+#include "fh_keyswitch.hpp"
 
 namespace fh {
 
@@ -38,7 +39,9 @@ struct TensorJob {
 
 // (a0 b0, a0 b1 + a1 b0, a1 b1) for one limb (src/CKKS/ElemenwiseBatchKernels.cu:1363-1400)
 __global__ __launch_bounds__(kT) void k_tensor_jobs(const TensorJob* __restrict__ jobs, const PrimeConst* __restrict__ prime, uint32_t N) {
-  const TensorJob j = jobs[blockIdx.y];
+  TensorJob j = jobs[blockIdx.y];
+  j.a0 = as_global(j.a0), j.a1 = as_global(j.a1), j.b0 = as_global(j.b0), j.b1 = as_global(j.b1);
+  j.o0 = as_global(j.o0), j.o1 = as_global(j.o1), j.o2 = as_global(j.o2);
   const PrimeConst P = prime[j.pid];
   for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < N; n += gridDim.x * blockDim.x) {
     const uint64_t a0 = j.a0[n], a1 = j.a1[n], b0 = j.b0[n], b1 = j.b1[n];
@@ -57,7 +60,8 @@ struct AddJob {
 
 // out = a + b, or out = a when b is null (level reduction, the untouched component of AddPlain)
 __global__ __launch_bounds__(kT) void k_add_jobs(const AddJob* __restrict__ jobs, const PrimeConst* __restrict__ prime, uint32_t N) {
-  const AddJob j = jobs[blockIdx.y];
+  AddJob j = jobs[blockIdx.y];
+  j.a = as_global(j.a), j.b = as_global(j.b), j.out = as_global(j.out);
   const uint64_t q = prime[j.pid].q;
   if (j.b) {
     for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < N; n += gridDim.x * blockDim.x) j.out[n] = add_mod(j.a[n], j.b[n], q);
@@ -74,7 +78,8 @@ struct MulPtJob {
 
 // (a0 pt, a1 pt) for one limb: ciphertext times plaintext (src/CKKS/LimbPartition.cu:588-682 multElement)
 __global__ __launch_bounds__(kT) void k_mulpt_jobs(const MulPtJob* __restrict__ jobs, const PrimeConst* __restrict__ prime, uint32_t N) {
-  const MulPtJob j = jobs[blockIdx.y];
+  MulPtJob j = jobs[blockIdx.y];
+  j.a0 = as_global(j.a0), j.a1 = as_global(j.a1), j.pt = as_global(j.pt), j.o0 = as_global(j.o0), j.o1 = as_global(j.o1);
   const PrimeConst P = prime[j.pid];
   for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < N; n += gridDim.x * blockDim.x) {
     const uint64_t w = j.pt[n];
@@ -84,13 +89,6 @@ __global__ __launch_bounds__(kT) void k_mulpt_jobs(const MulPtJob* __restrict__ 
 }
 
 // ------------------------------------------------------------------------------ ModUp conversion
-struct ModUpJob {
-  const uint64_t* coef;   // INTT of the key-switched polynomial (l+1 limbs)
-  const uint64_t* eval;   // the polynomial itself (l+1 limbs), copied to the digit's own limbs; null: not copied
-  uint64_t* out;          // digit d's block: l+1+K limbs
-  uint32_t l, d;
-};
-
 struct ConvConst {
   uint32_t N, L1, K, alpha, dnum;
   const PrimeConst* prime;
@@ -111,7 +109,8 @@ __global__ __launch_bounds__(kT) void k_modup_conv_jobs(const ModUpJob* __restri
   __shared__ Op s_qhat[SZ * kMaxPrimes];
   __shared__ uint64_t s_pq[kMaxPrimes], s_pn[kMaxPrimes];
   __shared__ uint64_t inv[SZ], invsh[SZ], qs[SZ];
-  const ModUpJob j = jobs[blockIdx.y];
+  ModUpJob j = jobs[blockIdx.y];
+  j.coef = as_global(j.coef), j.eval = as_global(j.eval), j.out = as_global(j.out);
   const uint32_t N = cc.N, lq = j.l + 1, ext = lq + cc.K, E = cc.L1 + cc.K;
   const uint32_t start = j.d * cc.alpha;
   const uint32_t sz = min(cc.alpha, lq - start);
@@ -211,7 +210,8 @@ template <class M>
 __global__ __launch_bounds__(kT) void k_ksk_jobs(const KskItem* __restrict__ items, const KskGroup* __restrict__ groups, KskConst kc) {
   using Op = typename M::Op;
   const uint32_t p = blockIdx.y;
-  const KskGroup g = groups[blockIdx.z];
+  KskGroup g = groups[blockIdx.z];
+  g.key = as_global(g.key);
   if (p < kc.L1 && p >= g.max_lq) return;
   const PrimeConst P = kc.prime[p];
   const uint32_t E = kc.L1 + kc.K;
@@ -235,7 +235,8 @@ __global__ __launch_bounds__(kT) void k_ksk_jobs(const KskItem* __restrict__ ite
     const uint32_t j0 = g.gal_inv != 1 ? auto_src(n, g.gal_inv, kc.logN) : n;
     const uint32_t j1 = g.gal_inv != 1 ? auto_src(n + 1, g.gal_inv, kc.logN) : n + 1;
     for (uint32_t t = 0; t < g.count; ++t) {
-      const KskItem it = items[g.first + t];
+      KskItem it = items[g.first + t];
+      it.dig = as_global(it.dig), it.c0 = as_global(it.c0), it.ext = as_global(it.ext), it.own = as_global(it.own);
       const uint32_t lq = it.l + 1;
       if (qprime && p >= lq) continue;
       const uint32_t ext = lq + kc.K;
@@ -283,12 +284,6 @@ __global__ __launch_bounds__(kT) void k_ksk_jobs(const KskItem* __restrict__ ite
 }
 
 // ------------------------------------------------------------------------------ ModDown conversion
-struct MdJob {
-  const uint64_t* pc;     // INTT of the K special limbs of one polynomial
-  uint64_t* conv;         // l+1 limbs, coefficient form
-  uint32_t lq, pad;
-};
-
 // k_moddown_conv_r of fh_keyswitch.hip with l+1 read from the job
 template <int KK, class M, bool RN>
 __global__ __launch_bounds__(kT) void k_moddown_conv_jobs(const MdJob* __restrict__ jobs, ConvConst cc) {
@@ -296,7 +291,8 @@ __global__ __launch_bounds__(kT) void k_moddown_conv_jobs(const MdJob* __restric
   __shared__ Op s_phat[KK * kMaxPrimes];
   __shared__ uint64_t s_q[kMaxPrimes], s_n[kMaxPrimes];
   __shared__ uint64_t inv[KK], invsh[KK], ps[KK];
-  const MdJob j = jobs[blockIdx.y];
+  MdJob j = jobs[blockIdx.y];
+  j.pc = as_global(j.pc), j.conv = as_global(j.conv);
   const uint32_t N = cc.N, lq = j.lq, K = cc.K;
   for (uint32_t i = threadIdx.x; i < KK * lq; i += blockDim.x) {
     const uint32_t k = i / lq, t = i % lq;
@@ -368,7 +364,8 @@ struct RsJob {
 __global__ __launch_bounds__(kT) void k_rescale_expand_jobs(const RsJob* __restrict__ jobs, const PrimeConst* __restrict__ prime,
                                                            const uint64_t* __restrict__ QlQl, const uint64_t* __restrict__ QlQl_sh,
                                                            uint32_t L1, uint32_t N) {
-  const RsJob j = jobs[blockIdx.y];
+  RsJob j = jobs[blockIdx.y];
+  j.top = as_global(j.top), j.e = as_global(j.e);
   const uint64_t ql = prime[j.l].q, qi = prime[j.i].q;
   const uint64_t half = ql >> 1;
   const size_t o = (size_t)j.l * L1 + j.i;
@@ -953,16 +950,19 @@ void launch_all(Context& c, BatchPlan& P, hipStream_t st) {
   }
   if (P.n_ks_intt) {
     ntt_inv_jobs(c, P.t_ks_in, P.t_ks_out, P.n_ks_intt, st);
+    const bool fused = conv_cols_usable(c, c.alpha), fused_down = conv_cols_usable(c, c.K);
     ConvConst cc{N, (uint32_t)c.L1, (uint32_t)c.K, (uint32_t)c.alpha, (uint32_t)c.dnum, c.d_prime, c.d_modup_qhinv, c.d_modup_qhinv_sh,
                  c.d_modup_qhat_m, c.d_md_phinv, c.d_md_phinv_sh, c.d_md_phat_m, c.reduced_noise ? c.d_modup_negq_m : nullptr,
                  c.reduced_noise ? c.d_md_negp_m : nullptr};
-    {
+    if (fused) {
+      conv_cols_modup_jobs(c, P.t_modup, P.n_modup, st);
+    } else {
       ProfScope ps_(c, "modup_conv", st);
       const dim3 g = grid_tiles(N, P.n_modup, 2);
       FH_CONV_DISPATCH(c, c.alpha, k_modup_conv_jobs, (g, kT, 0, st), (P.t_modup, cc))
     }
     FH_HIP(hipGetLastError());
-    ntt_fwd_jobs(c, P.t_modup_ntt, P.n_modup_ntt, st);
+    ntt_fwd_jobs(c, P.t_modup_ntt, P.n_modup_ntt, st, !fused);
     {
       ProfScope ps_(c, "ksk_batch", st);
       KskConst kc{N, (uint32_t)c.L1, (uint32_t)c.K, (uint32_t)c.alpha, (uint32_t)c.dnum, (uint32_t)c.logN, c.d_prime, c.d_pmod, c.d_pmod_sh};
@@ -972,13 +972,15 @@ void launch_all(Context& c, BatchPlan& P, hipStream_t st) {
     }
     FH_HIP(hipGetLastError());
     ntt_inv_jobs(c, P.t_md_in, P.t_md_out, P.n_md_intt, st);
-    {
+    if (fused_down) {
+      conv_cols_moddown_jobs(c, P.t_md, P.n_md, st);
+    } else {
       ProfScope ps_(c, "moddown_conv", st);
       const dim3 g = grid_tiles(N, P.n_md, 2);
       FH_CONV_DISPATCH(c, c.K, k_moddown_conv_jobs, (g, kT, 0, st), (P.t_md, cc))
     }
     FH_HIP(hipGetLastError());
-    ntt_fwd_jobs_moddown(c, P.t_md_ntt, P.t_md_epi, P.n_md_ntt, st);
+    ntt_fwd_jobs_moddown(c, P.t_md_ntt, P.t_md_epi, P.n_md_ntt, st, !fused_down);
   }
   if (P.n_rs_intt) {
     ntt_inv_jobs(c, P.t_rs_in, P.t_rs_out, P.n_rs_intt, st);

@@ -514,6 +514,7 @@ Context::Context(int logN_, int L1_, int K_, int dnum_, const std::vector<uint64
     d_modup_negq_m = upload(negq);
     d_md_negp_m = upload(negp);
   }
+  build_conv_cols(phat);
   d_md_pinv = upload(h_pinv);
   d_md_pinv_sh = upload(pinv_sh);
   d_pmod = upload(h_pmod);
@@ -549,6 +550,110 @@ Context::Context(int logN_, int L1_, int K_, int dnum_, const std::vector<uint64
   }
   FH_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
   ensure_aux_stream();
+}
+
+namespace {
+
+// digits[8] of v < 2^60 in base 256, each in [-128, 127]
+void signed_digits(uint64_t v, int8_t* out, size_t stride) {
+  int carry = 0;
+  for (int b = 0; b < 8; ++b) {
+    int d = (int)((v >> (8 * b)) & 255) + carry;
+    carry = d >= 128;
+    if (carry) d -= 256;
+    out[b * stride] = (int8_t)d;
+  }
+}
+
+// rows of one target prime p for the source factors f[0..n): digit row b, byte 8 i + a = digit b of
+// [2^8a f_i]_p; and the target's constant
+ConvTarget conv_rows(const std::vector<uint64_t>& f, uint64_t p, int kb, int8_t* rows) {
+  u128 sum = 0;
+  for (size_t i = 0; i < f.size(); ++i) {
+    uint64_t v = f[i] % p;
+    for (int a = 0; a < 8; ++a) {
+      signed_digits(v, rows + 8 * i + a, (size_t)kb);
+      sum += v;
+      v = h_mulmod(v, 256, p);
+    }
+  }
+  const uint64_t off = (uint64_t)((sum * 128) % p);
+  const u128 c = (u128)off + ((u128)p << 14);
+  ConvTarget t{};
+  t.lo = (uint64_t)c;
+  t.q = (float)((double)off / (double)p + 16384.0 - 0.375);
+  return t;
+}
+
+int conv_row_bytes(int sources) { return sources <= 8 ? 64 : sources <= 12 ? 96 : 128; }
+
+// group the targets by NTT arithmetic in fours, padding with repeats
+void conv_order(const std::vector<int>& targets, const std::vector<uint8_t>& fp64, uint8_t* ord) {
+  std::vector<uint8_t> slots;
+  int groups[2] = {0, 0};
+  for (int cls = 0; cls < 2; ++cls) {
+    int n = 0;
+    for (int t : targets)
+      if ((fp64[t] ? 0 : 1) == cls) {
+        slots.push_back((uint8_t)t);
+        ++n;
+      }
+    for (; n & 3; ++n) slots.push_back((uint8_t)(slots.back() | 0x80));
+    groups[cls] = n / 4;
+  }
+  ord[0] = (uint8_t)(groups[0] + groups[1]);
+  ord[1] = (uint8_t)groups[0];
+  std::copy(slots.begin(), slots.end(), ord + 4);
+}
+
+}  // namespace
+
+void Context::build_conv_cols(const std::vector<uint64_t>& phat) {
+  conv_cols_ok = K >= 1 && K <= 16 && alpha <= 16 && logN >= 12;
+  for (uint64_t v : q) conv_cols_ok = conv_cols_ok && v > (1ull << 48) && v < (1ull << 60);
+  if (!conv_cols_ok) return;
+  conv_kb_up = conv_row_bytes(alpha);
+  conv_kb_dn = conv_row_bytes(K);
+  std::vector<int8_t> up((size_t)L1 * np * 8 * conv_kb_up, 0), dn((size_t)L1 * 8 * conv_kb_dn, 0);
+  std::vector<ConvTarget> up_t((size_t)L1 * np), dn_t(L1);
+  std::vector<uint8_t> up_ord((size_t)L1 * dnum * kConvOrd, 0), dn_ord((size_t)L1 * kConvOrd, 0);
+  for (int l = 0; l < L1; ++l) {
+    // the digit whose last member is l, towards every other prime (a full digit's targets may lie
+    // above l at higher levels)
+    const int d = l / alpha, start = d * alpha, sz = l - start + 1;
+    for (int t = 0; t < np; ++t) {
+      if (t >= start && t <= l) continue;
+      const uint64_t p = q[t];
+      std::vector<uint64_t> f(sz);
+      for (int i = 0; i < sz; ++i) {
+        uint64_t pr = 1;
+        for (int j = 0; j < sz; ++j)
+          if (j != i) pr = h_mulmod(pr, q[start + j] % p, p);
+        f[i] = pr;
+      }
+      up_t[(size_t)l * np + t] = conv_rows(f, p, conv_kb_up, &up[((size_t)l * np + t) * 8 * conv_kb_up]);
+    }
+    for (int dd = 0; dd < num_digits(l); ++dd) {
+      const int s0 = dd * alpha, e0 = std::min(s0 + alpha, l + 1);
+      std::vector<int> targets;
+      for (int t = 0; t <= l; ++t)
+        if (t < s0 || t >= e0) targets.push_back(t);
+      for (int k = 0; k < K; ++k) targets.push_back(L1 + k);
+      conv_order(targets, fp64, &up_ord[((size_t)l * dnum + dd) * kConvOrd]);
+    }
+    std::vector<uint64_t> f(K);
+    for (int k = 0; k < K; ++k) f[k] = phat[(size_t)k * L1 + l];
+    dn_t[l] = conv_rows(f, q[l], conv_kb_dn, &dn[(size_t)l * 8 * conv_kb_dn]);
+    std::vector<int> targets;
+    for (int t = 0; t <= l; ++t) targets.push_back(t);
+    conv_order(targets, fp64, &dn_ord[(size_t)l * kConvOrd]);
+  }
+  d_cv_up = upload(up);
+  d_cv_up_t = upload(up_t);
+  d_cv_up_ord = upload(up_ord);
+  d_cv_dn = upload(dn);
+  d_cv_dn_t = upload(dn_t);
+  d_cv_dn_ord = upload(dn_ord);
 }
 
 void Context::ensure_aux_stream() {

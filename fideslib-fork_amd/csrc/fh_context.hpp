@@ -183,6 +183,17 @@ struct Tune {
   int ntt_team_per_xcd = 4;
 };
 
+// Per target of a matrix-instruction conversion: the constant that turns the sum over the sources'
+// bytes less 128 into the sum over the bytes, plus 2^14 p (which keeps every sum positive).
+struct ConvTarget {
+  uint64_t lo;   // its low word
+  float q;       // its quotient by p, less 0.375
+  uint32_t pad;
+};
+// target order of one conversion: groups of four of one NTT arithmetic. Bytes: number of groups, number
+// of fp64 groups (first), 2 unused, then 4 prime indices per group (bit 7: padding, not written)
+constexpr int kConvSlots = 84, kConvOrd = 4 + kConvSlots;
+
 struct Context;
 // Records an event pair around the launches issued in its scope when profiling is on.
 struct ProfScope {
@@ -227,6 +238,18 @@ struct Context {
   uint64_t* d_modup_negq_m = nullptr;    // [L1][dnum][L1+K] Montgomery form of [-Q_d]_{p_j}
   uint64_t* d_md_negp_m = nullptr;       // [L1] Montgomery form of [-P]_{q_i}
   bool mac30_ok() const { return split_mac_ok && (!reduced_noise || (alpha < 16 && K < 16)); }
+  // Matrix-instruction form of both conversions (conv_cols, fh_conv_cols.hip): the products
+  // [2^8a Qhat_i]_p (a: byte of the source) as signed base-256 digits, one row of digits per (target
+  // prime, output byte). A digit's matrix depends on its members alone, so it is kept under the level
+  // its last member has.
+  bool conv_cols_ok = false;             // primes in (2^48, 2^60), alpha and K <= 16
+  int conv_kb_up = 0, conv_kb_dn = 0;    // bytes per row: 8 per source, padded to 64, 96 or 128
+  int8_t* d_cv_up = nullptr;             // [L1][np][8][conv_kb_up]
+  ConvTarget* d_cv_up_t = nullptr;       // [L1][np]
+  uint8_t* d_cv_up_ord = nullptr;        // [L1][dnum][kConvOrd]
+  int8_t* d_cv_dn = nullptr;             // [L1][8][conv_kb_dn]
+  ConvTarget* d_cv_dn_t = nullptr;       // [L1]
+  uint8_t* d_cv_dn_ord = nullptr;        // [L1][kConvOrd]
   // ModDown
   uint64_t* d_md_phinv = nullptr;        // [K]     [P^_k^-1]_{p_k}
   uint64_t* d_md_phinv_sh = nullptr;     // [K]
@@ -285,6 +308,7 @@ struct Context {
  private:
   template <class T>
   T* upload(const std::vector<T>& v);
+  void build_conv_cols(const std::vector<uint64_t>& phat);
 };
 
 // A hook run at the start of every engine call this thread makes on a context (before the call

@@ -123,7 +123,7 @@ __device__ __forceinline__ void wsum_body(const WSumIn& in, int n, const uint64_
     uint64_t r0 = a0, r1 = a0;
     for (int k = 0; k < n; ++k) {
       const uint64_t wk = w[(size_t)k * towers + limb];
-      const V2 x = ld2(in.p[k] + ((size_t)comp * in.limbs[k] + limb) * N + i);
+      const V2 x = ld2(as_global(in.p[k]) + ((size_t)comp * in.limbs[k] + limb) * N + i);
       r0 = add_mod(r0, mul_mod(x.x, wk, P), P.q);
       r1 = add_mod(r1, mul_mod(x.y, wk, P), P.q);
     }

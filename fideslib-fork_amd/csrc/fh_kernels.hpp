@@ -49,6 +49,16 @@ struct EpiJob {
   uint32_t l;
 };
 
+// A buffer pointer that a kernel reads from a job table, for accesses through the global address space.
+// To the compiler such a pointer is generic: it issues flat accesses, which count as LDS accesses as
+// well, wait on both counters and take no scalar base. The pointer must be uniform over the wave.
+template <class T>
+__device__ __forceinline__ T* as_global(T* p) {
+  const uint64_t v = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return (T*)(__attribute__((address_space(1))) T*)((uint64_t)hi << 32 | lo);
+}
+
 struct SetAddr {
   LimbSet s;
   // limb-major job order: consecutive blocks work on the same prime (its twiddles stay in L2)
@@ -62,7 +72,7 @@ struct SetAddr {
 struct JobAddr {
   const LimbJob* jobs;
   __device__ __forceinline__ void at(uint32_t y, uint32_t, uint64_t*& p, int& pid) const {
-    p = jobs[y].ptr;
+    p = as_global(jobs[y].ptr);
     pid = (int)jobs[y].pid;
   }
 };
@@ -173,7 +183,8 @@ void ntt_fwd(const Context& c, const LimbSet& s, hipStream_t st);
 void ntt_inv(const Context& c, const LimbSet& s, hipStream_t st);
 void ntt_fwd(const Context& c, const LimbSet& in, const LimbSet& out, hipStream_t st);  // out-of-place
 void ntt_inv(const Context& c, const LimbSet& in, const LimbSet& out, hipStream_t st);
-void ntt_fwd_modup(const Context& c, const ModUpAddr& a, uint32_t n, hipStream_t st);
+// cols false (here and below): the limbs have had their column pass, only the row pass runs
+void ntt_fwd_modup(const Context& c, const ModUpAddr& a, uint32_t n, hipStream_t st, bool cols = true);
 // the column pass alone over the ModUp targets: their row stages then run in the fused key inner
 // product (rows_ksk, fh_rows_ksk.hip)
 void ntt_fwd_modup_cols(const Context& c, const ModUpAddr& a, uint32_t n, hipStream_t st);
@@ -191,11 +202,11 @@ struct AutotuneResult {
   double ms_best;       // forward + inverse at the chosen shape
 };
 AutotuneResult autotune_ntt(Context& c, int polys);
-void ntt_fwd_jobs(const Context& c, const LimbJob* d_jobs, uint32_t njobs, hipStream_t st);
+void ntt_fwd_jobs(const Context& c, const LimbJob* d_jobs, uint32_t njobs, hipStream_t st, bool cols = true);
 // Forward NTT of the ModDown conversion (conv: npolys x lq limbs over Q_l, coefficient form, used as
 // scratch) fused with the ModDown combination: out_i = (x_i - NTT(conv)_i) * [P^-1]_{q_i}.
 void ntt_fwd_moddown(const Context& c, const LimbSet& conv, const uint64_t* x, uint64_t x_stride, uint64_t* out, uint64_t out_stride,
-                     hipStream_t st);
+                     hipStream_t st, bool cols = true);
 // Forward NTT of the Rescale correction e (npolys x l limbs, coefficient form, scratch) fused with
 // the Rescale combination: out_i = x_i * [q_l^-1]_{q_i} + NTT(e)_i.
 void ntt_fwd_rescale(const Context& c, const LimbSet& e, const uint64_t* x, uint32_t l, uint64_t* out, hipStream_t st);
@@ -204,7 +215,7 @@ void ntt_inv_jobs(const Context& c, const LimbJob* d_jobs, uint32_t njobs, hipSt
 void ntt_fwd_jobs(const Context& c, const LimbJob* d_in, const LimbJob* d_out, uint32_t njobs, hipStream_t st);
 void ntt_inv_jobs(const Context& c, const LimbJob* d_in, const LimbJob* d_out, uint32_t njobs, hipStream_t st);
 // in-place forward NTTs of the job limbs (scratch) with the ModDown / Rescale epilogue of d_epi[y]
-void ntt_fwd_jobs_moddown(const Context& c, const LimbJob* d_jobs, const EpiJob* d_epi, uint32_t njobs, hipStream_t st);
+void ntt_fwd_jobs_moddown(const Context& c, const LimbJob* d_jobs, const EpiJob* d_epi, uint32_t njobs, hipStream_t st, bool cols = true);
 void ntt_fwd_jobs_rescale(const Context& c, const LimbJob* d_jobs, const EpiJob* d_epi, uint32_t njobs, hipStream_t st);
 
 }  // namespace fh

@@ -544,7 +544,16 @@ void modup_batch(Context& c, const uint64_t* x, int l, int npolys, uint64_t x_st
                  x_stride, c.d_prime, c.d_modup_qhinv, c.d_modup_qhinv_sh, c.d_modup_qhat, c.d_modup_qhat_m,
                  c.reduced_noise ? c.d_modup_negq_m : nullptr};
   if (c.reduced_noise && (!c.rn_conv_ok || c.alpha > 16)) throw Error(-3, "ReducedNoise conversions need (alpha + 1) * max prime <= 2^64");
-  {
+  const bool fused = conv_cols_usable(c, c.alpha);
+  if (fused) {
+    conv_cols_modup(c, tmp.p, l, npolys, digits, st);
+    // the digits' own limbs (contiguous in the input and in each digit)
+    for (uint32_t d = 0; copy_own && d < beta; ++d) {
+      const size_t start = (size_t)d * c.alpha, sz = std::min<size_t>(c.alpha, lq - start);
+      FH_HIP(hipMemcpy2DAsync(digits + ((size_t)d * ext + start) * c.N, (size_t)beta * ext * c.N * 8, x + start * c.N, x_stride * 8, sz * c.N * 8,
+                              npolys, hipMemcpyDeviceToDevice, st));
+    }
+  } else {
     ProfScope ps_(c, "modup_conv", st);
     const dim3 g2 = grid_n(c.N, beta * npolys, 2);
     const uint64_t* own = copy_own ? x : nullptr;
@@ -553,8 +562,8 @@ void modup_batch(Context& c, const uint64_t* x, int l, int npolys, uint64_t x_st
   }
   FH_HIP(hipGetLastError());
   ModUpAddr a{digits, ext, lq, (uint32_t)c.alpha, (uint32_t)c.L1, beta, (uint32_t)npolys, (uint64_t)beta * ext * c.N};
-  if (rows) ntt_fwd_modup(c, a, a.count(), st);
-  else ntt_fwd_modup_cols(c, a, a.count(), st);
+  if (rows) ntt_fwd_modup(c, a, a.count(), st, !fused);
+  else if (!fused) ntt_fwd_modup_cols(c, a, a.count(), st);
 }
 
 void ksk_inner(Context& c, const uint64_t* digits, int l, const uint64_t* key, uint64_t* out0, uint64_t* out1,
@@ -604,7 +613,10 @@ void moddown(Context& c, const uint64_t* x, int l, uint64_t* out, int npolys, ui
   ModDownParams mp{c.N, lq, ext, (uint32_t)c.L1, K, c.d_prime, c.d_md_phinv, c.d_md_phinv_sh, c.d_md_phat, c.d_md_phat_m,
                    c.d_md_pinv, c.d_md_pinv_sh, c.reduced_noise ? c.d_md_negp_m : nullptr};
   if (c.reduced_noise && (!c.rn_conv_ok || K > 16)) throw Error(-3, "ReducedNoise conversions need (K + 1) * max prime <= 2^64");
-  {
+  const bool fused = conv_cols_usable(c, (int)K);
+  if (fused) {
+    conv_cols_moddown(c, pc.p, l, npolys, conv.p, st);
+  } else {
     ProfScope ps_(c, "moddown_conv", st);
     const dim3 g2 = grid_n(c.N, npolys, 2);
     if (!c.redc_conv_ok || K > 16) k_moddown_conv<<<grid_n(c.N, npolys), kT, 0, st>>>(pc.p, conv.p, mp);
@@ -612,7 +624,7 @@ void moddown(Context& c, const uint64_t* x, int l, uint64_t* out, int npolys, ui
   }
   FH_HIP(hipGetLastError());
   // forward NTT of the conversion with (x_i - conv_i) * P^-1 fused into its last launch
-  ntt_fwd_moddown(c, make_set(conv.p, lq, qids.data(), npolys, (uint64_t)lq * c.N), x, x_stride, out, out_stride, st);
+  ntt_fwd_moddown(c, make_set(conv.p, lq, qids.data(), npolys, (uint64_t)lq * c.N), x, x_stride, out, out_stride, st, !fused);
 }
 
 void rescale(Context& c, const uint64_t* x, int l, int ncomp, uint64_t* out, hipStream_t st) {

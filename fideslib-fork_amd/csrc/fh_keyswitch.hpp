@@ -6,6 +6,31 @@
 
 namespace fh {
 
+// Conversion jobs of a mixed-level batch (device tables).
+struct ModUpJob {
+  const uint64_t* coef;   // INTT of the key-switched polynomial (l+1 limbs)
+  const uint64_t* eval;   // the polynomial itself (l+1 limbs), copied to the digit's own limbs; null: not copied
+  uint64_t* out;          // digit d's block: l+1+K limbs
+  uint32_t l, d;
+};
+struct MdJob {
+  const uint64_t* pc;     // INTT of the K special limbs of one polynomial
+  uint64_t* conv;         // l+1 limbs, coefficient form
+  uint32_t lq, pad;
+};
+
+// Conversion and column pass of the targets' forward NTT in one launch (fh_conv_cols.hip). usable: the
+// context's primes, the default radix split, the exact (not ReducedNoise) conversion and three
+// sources (alpha for ModUp, K for ModDown) or more; otherwise the conversion kernels of
+// fh_keyswitch.hip / fh_batch.hip run, followed by both NTT passes.
+bool conv_cols_usable(const Context& c, int sources);
+// coef: npolys x (l+1) limbs (INTT of the inputs) -> the target limbs of npolys x beta digits, after their column pass
+void conv_cols_modup(const Context& c, const uint64_t* coef, int l, int npolys, uint64_t* digits, hipStream_t st);
+// pcoef: npolys x K limbs (INTT of the special limbs) -> npolys x (l+1) limbs, after their column pass
+void conv_cols_moddown(const Context& c, const uint64_t* pcoef, int l, int npolys, uint64_t* conv, hipStream_t st);
+void conv_cols_modup_jobs(const Context& c, const ModUpJob* jobs, uint32_t n, hipStream_t st);
+void conv_cols_moddown_jobs(const Context& c, const MdJob* jobs, uint32_t n, hipStream_t st);
+
 // digits: beta x (l+1+K) limbs (EVAL)
 void modup(Context& c, const uint64_t* x, int l, uint64_t* digits, hipStream_t st);
 // npolys inputs x_stride words apart (0 = packed) -> npolys packed digit blocks. copy_own false

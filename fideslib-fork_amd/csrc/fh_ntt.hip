@@ -16,9 +16,9 @@ void ntt_inv(const Context& c, const LimbSet& in, const LimbSet& out, hipStream_
   dispatch(c, SetAddr{in}, SetAddr{out}, in.nlimbs * in.npolys, st, false);
 }
 void ntt_fwd_moddown(const Context& c, const LimbSet& conv, const uint64_t* x, uint64_t x_stride, uint64_t* out, uint64_t out_stride,
-                     hipStream_t st) {
+                     hipStream_t st, bool cols) {
   EpiModDown e{x, x_stride, out, out_stride, c.d_md_pinv, c.d_md_pinv_sh, conv.npolys, nullptr, nullptr, 0, 0, 0};
-  dispatch(c, SetAddr{conv}, SetAddr{conv}, conv.nlimbs * conv.npolys, st, true, e, "ntt_fwd_rows_moddown");
+  dispatch(c, SetAddr{conv}, SetAddr{conv}, conv.nlimbs * conv.npolys, st, true, e, "ntt_fwd_rows_moddown", cols);
 }
 
 void ntt_fwd_rescale(const Context& c, const LimbSet& e, const uint64_t* x, uint32_t l, uint64_t* out, hipStream_t st) {

@@ -52,13 +52,15 @@ constexpr int kNttThreads = 256, kNttWide = 512;
 // and start from constants, so the bounds fold away; only IntL acts on them.
 
 // ------------------------------------------------------------------------------- integer arithmetic
-// Primes below 2^60: sixteen multiples of q fit a word, so a value is reduced only where its bound
-// would pass 16 q instead of in every butterfly. The quotient product is exact (Shoup), the low words
-// are formed as y w + h (-q) mod 2^64, and a multiple of q that keeps a difference positive is
-// shifted in with the same add. A forward butterfly costs 22 VALU instructions instead of 29.
+// Primes below 2^60: sixteen multiples of q fit a word, so a product is left anywhere below 4 q and a
+// value is reduced only where its bound would pass 16 q, to below 2 q with a quotient taken in fp32.
+// A multiple of q that keeps a difference positive is shifted in with the same add. A forward
+// butterfly takes 17 VALU instructions and the reductions 1.5 more on average, where Harvey's (a
+// reduction in each) took 29.
 struct IntL {
   using T = uint64_t;
-  static constexpr int kMid = 16;   // bound of a value between the passes of a forward transform
+  static constexpr int kMid = 14;   // largest bound of a value between the passes of a forward transform
+  static constexpr int kMidInv = 4; // and of an inverse one
   uint64_t q, nq;                   // nq = -q mod 2^64
   float q32inv;                     // 2^32 / q, rounded down: the quotient of a value below 16 q
   struct W {
@@ -67,43 +69,40 @@ struct IntL {
   __device__ __forceinline__ T from_canon(uint64_t v) const { return v; }
   __device__ __forceinline__ T from_mid(uint64_t v) const { return v; }
   __device__ __forceinline__ uint64_t to_mid(T v) const { return v; }
-  // x w mod q in [0, 2q) for any x < 2^64
-  __device__ __forceinline__ T mul(T x, W w) const { return x * w.w + mulhi(x, w.sh) * nq; }
-  __device__ __forceinline__ void sub8(T& x, int& b) const {
-    const uint64_t m = q << 3;
-    x = x >= m ? x - m : x;
-    b = b - 8 > 8 ? b - 8 : 8;
-  }
+  __device__ __forceinline__ T mul(T x, W w) const { return shoup_lazy4(x, w.w, w.sh, nq); }
   // x mod q up to one q, for b <= 16: the quotient (< 16) from the high word in fp32, rounded down
   // by at most one
   __device__ __forceinline__ T below2(T x) const {
     const uint32_t h = (uint32_t)((float)(uint32_t)(x >> 32) * q32inv);
-    return x + (uint64_t)h * nq;
+    const uint64_t p = (uint64_t)h * (uint32_t)nq + x;
+    return (uint64_t)((uint32_t)(p >> 32) + h * (uint32_t)(nq >> 32)) << 32 | (uint32_t)p;
+  }
+  __device__ __forceinline__ void lower(T& x, int& b) const {
+    x = below2(x);
+    b = 2;
   }
   __device__ __forceinline__ void fwd(T& X, T& Y, W w, int& bx, int& by) const {
-    if (bx + 2 > 16) sub8(X, bx);
-    const uint64_t t = mul(Y, w), x2 = X + (q << 1);
+    if (bx + 4 > 16) lower(X, bx);
+    const uint64_t t = mul(Y, w), x4 = X + (q << 2);
     X = X + t;
-    Y = x2 - t;
-    bx = by = bx + 2;
+    Y = x4 - t;
+    bx = by = bx + 4;
   }
   static __device__ __forceinline__ constexpr int log2_up(int b) { return b <= 1 ? 0 : b <= 2 ? 1 : b <= 4 ? 2 : b <= 8 ? 3 : 4; }
   __device__ __forceinline__ void inv(T& X, T& Y, W w, int& bx, int& by) const {
-    if (bx + (1 << log2_up(by)) > 16) {
-      if (bx > 8) sub8(X, bx);
-      if (by > 8) sub8(Y, by);
-    }
+    if (bx + (1 << log2_up(by)) > 16 && by > 2) lower(Y, by);
+    if (bx + (1 << log2_up(by)) > 16) lower(X, bx);
     const uint64_t v = X + (q << log2_up(by)) - Y;
     X = X + Y;
     Y = mul(v, w);
     bx = bx + by;
-    by = 2;
+    by = 4;
   }
   __device__ __forceinline__ void settle_fwd(T&, int&) const {}
   __device__ __forceinline__ void settle_mid(T&, int&) const {}
   __device__ __forceinline__ void settle_inv(T& x, int& b) const {
-    if (b > 2) x = below2(x);
-    b = 2;
+    if (b > kMidInv) lower(x, b);
+    b = kMidInv;
   }
   __device__ __forceinline__ uint64_t canon(T x, int b) const {
     if (b > 2) x = below2(x);
@@ -115,7 +114,7 @@ struct IntL {
 // values in [0, 2q), reduced in every butterfly.
 struct IntA {
   using T = uint64_t;
-  static constexpr int kMid = 1;
+  static constexpr int kMid = 1, kMidInv = 1;
   uint64_t q, q2;
   struct W {
     uint64_t w, sh;
@@ -150,7 +149,7 @@ struct IntA {
 struct FpA {
   using T = double;
   using W = double;
-  static constexpr int kMid = 1;
+  static constexpr int kMid = 1, kMidInv = 1;
   double q, qinv, half;
   // y * w mod q for |y| < 4q, |w| <= q/2: exact, result in about (-1.3q, 1.3q)
   __device__ __forceinline__ double mul(double y, double w) const {
@@ -299,14 +298,11 @@ struct OpaqueTid {
 };
 
 // ------------------------------------------------------------------------------- forward, columns
-// The l1 stages of one column held by T = S / 16 threads, 16 elements each: in: element k at row
-// r0 + T k (bound 1), out: at row 16 r0 + k (LS > 4, through the column's LDS slot t) or r0 + T k.
+// The l1 stages of one column held by T = S / 16 threads, 16 elements each. First half (lo): stages
+// 0..3 on element k at row r0 + T k. Second half (hi, LS > 4): the rest on element k at row
+// 16 r0 + k. b: the values' bounds. sw / swp: the table's first S twiddles.
 template <int LS, class A, class TwT>
-__device__ __forceinline__ void fwd_cols_stages(const A& ar, typename A::T (&x)[16], const TwT* sw, const TwT* swp, uint64_t* t, int r0) {
-  constexpr int S = 1 << LS, T = S / 16;
-  int b[16];
-#pragma unroll
-  for (int k = 0; k < 16; ++k) b[k] = 1;
+__device__ __forceinline__ void fwd_cols_lo(const A& ar, typename A::T (&x)[16], int (&b)[16], const TwT* sw, const TwT* swp) {
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
     const int h = 8 >> s;
@@ -319,25 +315,22 @@ __device__ __forceinline__ void fwd_cols_stages(const A& ar, typename A::T (&x)[
   }
 #pragma unroll
   for (int k = 0; k < 16; ++k) ar.settle_fwd(x[k], b[k]);
-  if constexpr (LS > 4) {
+}
+template <int LS, class A, class TwT>
+__device__ __forceinline__ void fwd_cols_hi(const A& ar, typename A::T (&x)[16], int (&b)[16], const TwT* sw, const TwT* swp, int r0) {
+  constexpr int S = 1 << LS;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) t[r0 + T * k] = ar.to_mid(x[k]);
-    __syncthreads();
+  for (int s = 4; s < LS; ++s) {
+    const int h = S >> (s + 1);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) x[k] = ar.from_mid(t[16 * r0 + k]);
-#pragma unroll
-    for (int s = 4; s < LS; ++s) {
-      const int h = S >> (s + 1);
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        if (k & h) continue;
-        const int idx = (1 << s) + ((16 * r0 + k) >> (LS - s));
-        ar.fwd(x[k], x[k + h], tw_at(ar, sw, swp, idx), b[k], b[k + h]);
-      }
+    for (int k = 0; k < 16; ++k) {
+      if (k & h) continue;
+      const int idx = (1 << s) + ((16 * r0 + k) >> (LS - s));
+      ar.fwd(x[k], x[k + h], tw_at(ar, sw, swp, idx), b[k], b[k + h]);
     }
-#pragma unroll
-    for (int k = 0; k < 16; ++k) ar.settle_fwd(x[k], b[k]);
   }
+#pragma unroll
+  for (int k = 0; k < 16; ++k) ar.settle_fwd(x[k], b[k]);
 }
 
 // First l1 stages. Input: canonical (in place or out of place), output: internal form.
@@ -353,8 +346,18 @@ __device__ __forceinline__ void fwd_cols_body(const A& ar, const TwT* tw, const 
 #pragma unroll
   for (int k = 0; k < 16; ++k) x[k] = ar.from_canon(p[(size_t)(r0 + T * k) * N2 + col]);
   __syncthreads();
-  fwd_cols_stages<LS>(ar, x, (const TwT*)sw, (const TwT*)swp, tile + cc * PADS, r0);
+  int b[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) b[k] = 1;
+  fwd_cols_lo<LS>(ar, x, b, (const TwT*)sw, (const TwT*)swp);
   if constexpr (LS > 4) {
+    uint64_t* t = tile + cc * PADS;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) t[r0 + T * k] = ar.to_mid(x[k]);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) x[k] = ar.from_mid(t[16 * r0 + k]);
+    fwd_cols_hi<LS>(ar, x, b, (const TwT*)sw, (const TwT*)swp, r0);
 #pragma unroll
     for (int k = 0; k < 16; ++k) po[(size_t)(16 * r0 + k) * N2 + col] = ar.to_mid(x[k]);
   } else {
@@ -686,7 +689,7 @@ __device__ __forceinline__ void inv_rows_body(const A& ar, const TwT* tw, const 
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       x[k] = ar.from_mid(t[rsw(c0 + T * k)]);
-      b[k] = 2;
+      b[k] = A::kMidInv;
     }
   } else {
 #pragma unroll
@@ -748,7 +751,7 @@ __device__ __forceinline__ void inv_cols_body(const A& ar, const TwT* tw, const 
   int b[16];
   uint64_t* t = tile + cc * PADS;
 #pragma unroll
-  for (int k = 0; k < 16; ++k) b[k] = 2;
+  for (int k = 0; k < 16; ++k) b[k] = A::kMidInv;
   if constexpr (LS > 4) {
 #pragma unroll
     for (int k = 0; k < 16; ++k) x[k] = ar.from_mid(Ld::ld(p + (size_t)(16 * r0 + k) * N2 + col));
@@ -776,7 +779,7 @@ __device__ __forceinline__ void inv_cols_body(const A& ar, const TwT* tw, const 
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       x[k] = ar.from_mid(t[r0 + T * k]);
-      b[k] = 2;
+      b[k] = A::kMidInv;
     }
   } else {
 #pragma unroll
@@ -799,7 +802,7 @@ __device__ __forceinline__ void inv_cols_body(const A& ar, const TwT* tw, const 
   }
   // N^-1: a product by a constant, which takes what the last two stages leave unsettled
 #pragma unroll
-  for (int k = 0; k < 16; ++k) p[(size_t)(r0 + T * k) * N2 + col] = ar.canon(ar.mul(x[k], fin), 2);
+  for (int k = 0; k < 16; ++k) p[(size_t)(r0 + T * k) * N2 + col] = ar.canon(ar.mul(x[k], fin), 4);
 }
 
 // N^-1 mod the prime as the arithmetic's twiddle
@@ -1087,9 +1090,9 @@ struct EpiModDownJobs {
   uint64_t q, wi, wish;
   __device__ __forceinline__ void init(uint32_t y, uint32_t, const PrimeConst* prime) {
     const EpiJob j = jobs[y];
-    xi = j.x;
-    oi = j.out;
-    ai = j.add;
+    xi = as_global(j.x);
+    oi = as_global(j.out);
+    ai = as_global(j.add);
     q = prime[j.pid].q;
     wi = w[j.pid];
     wish = wsh[j.pid];
@@ -1118,9 +1121,9 @@ struct EpiRescaleJobs {
   PrimeConst P;
   __device__ __forceinline__ void init(uint32_t y, uint32_t, const PrimeConst* prime) {
     const EpiJob j = jobs[y];
-    xi = j.x;
-    pti = j.add;
-    oi = j.out;
+    xi = as_global(j.x);
+    pti = as_global(j.add);
+    oi = as_global(j.out);
     P = prime[j.pid];
     const size_t o = (size_t)j.l * L1 + j.pid;
     wi = w[o];
@@ -1294,11 +1297,13 @@ struct ChunkStreams {
   }
 };
 
+// cols false: the limbs have had their column pass (conv_cols), only the row pass runs
 template <class Addr, class AddrOut, int L1S, int L2S, bool WIDE, class Epi>
-void fwd_impl(const Context& c, const Addr& ad, const AddrOut& ao, uint32_t nlimbs, hipStream_t st0, const Epi& epi, const char* rows_name) {
+void fwd_impl(const Context& c, const Addr& ad, const AddrOut& ao, uint32_t nlimbs, hipStream_t st0, const Epi& epi, const char* rows_name,
+              bool cols) {
   NttTables tb = ntt_tables(c);
   if constexpr (L1S == L2S && L1S >= 6) {
-    if (team_ok<L1S, L2S>(c, st0) && launch_fwd_team<L1S>(c, ad, ao, nlimbs, tb, st0, epi, rows_name)) return;
+    if (cols && team_ok<L1S, L2S>(c, st0) && launch_fwd_team<L1S>(c, ad, ao, nlimbs, tb, st0, epi, rows_name)) return;
   }
   const bool wc = WIDE && c.tune.ntt_threads[0] == kNttWide, wr = WIDE && c.tune.ntt_threads[1] == kNttWide;
   const uint32_t chunk = chunk_limbs(c);
@@ -1310,12 +1315,12 @@ void fwd_impl(const Context& c, const Addr& ad, const AddrOut& ao, uint32_t nlim
     Shift<AddrOut> so{ao, base};
     ShiftEpi<Epi> se{epi, base};
     if constexpr (WIDE) {
-      if (wc) launch_fwd_cols<L1S, kNttWide>(c, sa, so, n, tb, st);
-      else launch_fwd_cols<L1S, kNttThreads>(c, sa, so, n, tb, st);
+      if (cols && wc) launch_fwd_cols<L1S, kNttWide>(c, sa, so, n, tb, st);
+      else if (cols) launch_fwd_cols<L1S, kNttThreads>(c, sa, so, n, tb, st);
       if (wr) launch_fwd_rows<L2S, kNttWide>(c, so, n, tb, st, se, rows_name);
       else launch_fwd_rows<L2S, kNttThreads>(c, so, n, tb, st, se, rows_name);
     } else {
-      launch_fwd_cols<L1S, kNttThreads>(c, sa, so, n, tb, st);
+      if (cols) launch_fwd_cols<L1S, kNttThreads>(c, sa, so, n, tb, st);
       launch_fwd_rows<L2S, kNttThreads>(c, so, n, tb, st, se, rows_name);
     }
   }
@@ -1351,13 +1356,13 @@ void inv_impl(const Context& c, const Addr& ad, const AddrOut& ao, uint32_t nlim
 
 template <class Addr, class AddrOut, class Epi = EpiStore>
 void dispatch(const Context& c, const Addr& ad, const AddrOut& ao, uint32_t nlimbs, hipStream_t st, bool fwd, const Epi& epi = Epi{},
-              const char* rows_name = "ntt_fwd_rows") {
+              const char* rows_name = "ntt_fwd_rows", bool cols = true) {
   if (nlimbs == 0) return;
   const int l1 = c.tune.ntt_split ? c.tune.ntt_split : ntt_default_split(c.logN);
   // (logN, l1) pairs accepted by ntt_split_ok; the default split of each logN also has wide tiles
 #define FH_NTT_CASE(LN, A, WIDE)                                                                     \
   case LN * 16 + A:                                                                                  \
-    if (fwd) fwd_impl<Addr, AddrOut, A, LN - A, WIDE, Epi>(c, ad, ao, nlimbs, st, epi, rows_name);   \
+    if (fwd) fwd_impl<Addr, AddrOut, A, LN - A, WIDE, Epi>(c, ad, ao, nlimbs, st, epi, rows_name, cols); \
     else inv_impl<Addr, AddrOut, A, LN - A, WIDE>(c, ad, ao, nlimbs, st);                            \
     break;
   switch (c.logN * 16 + l1) {
