@@ -104,6 +104,12 @@ __global__ __launch_bounds__(kT) void k_lt_sum(LimbSet acc, const uint64_t* __re
   }
 }
 
+void lt_sum(Context& c, const LimbSet& acc, const uint64_t* T, uint64_t t_stride, int nt, hipStream_t st) {
+  ProfScope ps_(c, "lt_sum", st);
+  k_lt_sum<<<grid_n(c.N, 2 * acc.nlimbs), kT, 0, st>>>(acc, T, t_stride, nt, c.N, c.d_prime);
+  FH_HIP(hipGetLastError());
+}
+
 // k_extend_p for B ciphertexts: blockIdx.y = (b, comp, pos)
 __global__ __launch_bounds__(kT) void k_extend_p_b(const uint64_t* __restrict__ x, uint64_t x_stride, uint64_t* __restrict__ out,
                                                     uint64_t out_stride, uint32_t N, uint32_t lq, uint32_t ext, const PrimeConst* prime,
@@ -251,8 +257,8 @@ void lt_finish(Context& c, uint64_t* acc, int l, int offset, const uint64_t* off
   if (offset != 0) {
     DBuf c1q(c.pool, (size_t)lq * N), dig(c.pool, (size_t)beta * E), t(c.pool, 2 * E);
     moddown(c, acc + E, l, c1q.p, 1, 0, 0, st);
-    modup(c, c1q.p, l, dig.p, st);
-    ksk_inner(c, dig.p, l, off_key, t.p, t.p + E, acc, off_gal, st, true);
+    modup_batch(c, c1q.p, l, 1, 0, dig.p, st, false);
+    ksk_inner(c, dig.p, l, off_key, t.p, t.p + E, acc, off_gal, st, true, c1q.p);
     moddown(c, t.p, l, out, 2, 0, 0, st);
   } else {
     moddown(c, acc, l, out, 2, 0, 0, st);
@@ -285,8 +291,8 @@ void linear_transform(Context& c, const uint64_t* ct, int l, int rowSize, int bS
     uint64_t* Rp = Rj - 2 * E;
     if (giant) {
       moddown(c, Rj + E, l, c1q.p, 1, 0, 0, st);
-      modup(c, c1q.p, l, dig.p, st);
-      ksk_inner(c, dig.p, l, giant_key, Rp, Rp + E, Rj, giant_gal, st, true, nullptr, true);
+      modup_batch(c, c1q.p, l, 1, 0, dig.p, st, false);
+      ksk_inner(c, dig.p, l, giant_key, Rp, Rp + E, Rj, giant_gal, st, true, c1q.p, true);
     } else {
       LimbSet a = make_set(Rp, ext, epids.data(), 2, E), b = make_set(Rj, ext, epids.data(), 2, E);
       ew_binary(c, 0, a, b, a, st);
@@ -336,13 +342,10 @@ void linear_transform_flat(Context& c, const uint64_t* ct, int l, int rowSize, i
       src = gathered.p;
     }
     moddown(c, src + E, l, c1q.p, nr, 2 * E, (uint64_t)lq * N, st);
-    modup_batch(c, c1q.p, l, nr, (uint64_t)lq * N, dig.p, st, true);
-    ksk_items(c, nr, 1, dig.p, (uint64_t)beta * E, src, 2 * E, true, true, l, keys.data(), gals.data(), T.p, 2 * E, st);
-    {
-      ProfScope ps_(c, "lt_sum", st);
-      k_lt_sum<<<grid_n(c.N, 2 * ext), kT, 0, st>>>(acc, T.p, 2 * E, nr, c.N, c.d_prime);
-      FH_HIP(hipGetLastError());
-    }
+    modup_batch(c, c1q.p, l, nr, (uint64_t)lq * N, dig.p, st, false);
+    ksk_items(c, nr, 1, dig.p, (uint64_t)beta * E, src, 2 * E, true, true, l, keys.data(), gals.data(), T.p, 2 * E, st, c1q.p,
+              (uint64_t)lq * N);
+    lt_sum(c, acc, T.p, 2 * E, nr, st);
   }
   for (int j = 1; j < gStep; ++j)
     if (((long long)j * bStep * stride) % slots == 0) ew_binary(c, 0, acc, make_set(R.p + (size_t)j * 2 * E, ext, epids.data(), 2, E), acc, st);
@@ -397,7 +400,7 @@ void linear_transform_batch(Context& c, int count, const uint64_t* cts, uint64_t
   }
   if (nrot) {
     rot = DBuf(c.pool, (size_t)B * nrot * 2 * E);
-    modup_batch(c, cts + (size_t)lq * N, l, (int)B, ct_stride, dig.p, st);
+    modup_batch(c, cts + (size_t)lq * N, l, (int)B, ct_stride, dig.p, st, false);
     std::vector<const uint64_t*> ks((size_t)B * nrot);
     std::vector<uint32_t> gs((size_t)B * nrot);
     for (uint32_t b = 0; b < B; ++b)
@@ -406,7 +409,7 @@ void linear_transform_batch(Context& c, int count, const uint64_t* cts, uint64_t
         gs[(size_t)b * nrot + r] = baby_gal[rot_idx[r]];
       }
     ksk_items(c, (int)(B * nrot), (int)nrot, dig.p, (uint64_t)beta * E, cts, ct_stride, true, false, l, ks.data(), gs.data(), rot.p, 2 * E,
-              st);
+              st, cts + (size_t)lq * N, ct_stride);
   }
 
   // ---- giant-step partial sums: diagonals read once for the batch ----
@@ -441,9 +444,9 @@ void linear_transform_batch(Context& c, int count, const uint64_t* cts, uint64_t
       uint64_t* Rp = Rj - 2 * E;  // every ciphertext's R_{j-1} += rot_giant(R_j)
       if (giant) {
         moddown(c, Rj + E, l, c1q.p, (int)B, rstride, (uint64_t)lq * N, st);
-        modup_batch(c, c1q.p, l, (int)B, (uint64_t)lq * N, dig.p, st);
+        modup_batch(c, c1q.p, l, (int)B, (uint64_t)lq * N, dig.p, st, false);
         ksk_items(c, (int)B, 1, dig.p, (uint64_t)beta * E, Rj, rstride, true, true, l, gk.data(), gg.data(), Rp, rstride, st,
-                  nullptr, 0, true);
+                  c1q.p, (uint64_t)lq * N, true);
       } else {
         for (int comp = 0; comp < 2; ++comp) {
           LimbSet a = make_set(Rp + comp * E, ext, epids.data(), B, rstride), b = make_set(Rj + comp * E, ext, epids.data(), B, rstride);
@@ -452,9 +455,10 @@ void linear_transform_batch(Context& c, int count, const uint64_t* cts, uint64_t
       }
     } else if (offset != 0) {
       moddown(c, Rj + E, l, c1q.p, (int)B, rstride, (uint64_t)lq * N, st);
-      modup_batch(c, c1q.p, l, (int)B, (uint64_t)lq * N, dig.p, st);
+      modup_batch(c, c1q.p, l, (int)B, (uint64_t)lq * N, dig.p, st, false);
       DBuf t(c.pool, (size_t)B * 2 * E);
-      ksk_items(c, (int)B, 1, dig.p, (uint64_t)beta * E, Rj, rstride, true, true, l, okv.data(), og.data(), t.p, 2 * E, st);
+      ksk_items(c, (int)B, 1, dig.p, (uint64_t)beta * E, Rj, rstride, true, true, l, okv.data(), og.data(), t.p, 2 * E, st, c1q.p,
+                (uint64_t)lq * N);
       moddown(c, t.p, l, out, (int)(2 * B), E, (uint64_t)lq * N, st);
     } else {
       moddown(c, Rj, l, out, (int)B, rstride, 2ull * lq * N, st);
@@ -488,10 +492,7 @@ void accumulate_cascade(Context& c, const uint64_t* ct, int l, int radix, int si
     }
     rotate_hoisted(c, out, l, n, keys + used, galois + used, true, false, fast.p + 2 * E, st);
     LimbSet a = make_set(fast.p, ext, epids.data(), 2, E);
-    for (int i = 1; i <= n; ++i) {
-      LimbSet b = make_set(fast.p + (size_t)i * 2 * E, ext, epids.data(), 2, E);
-      ew_binary(c, 0, a, b, a, st);
-    }
+    lt_sum(c, a, fast.p + 2 * E, 2 * E, n, st);
     moddown(c, fast.p, l, out, 2, 0, 0, st);
     used += n;
   }
@@ -534,10 +535,7 @@ void accumulate_sum(Context& c, const uint64_t* ct, int l, int radix, int size, 
       FH_HIP(hipGetLastError());
     }
     LimbSet a = make_set(fast.p, ext, epids.data(), 2, E);
-    for (int i = 1; i <= n; ++i) {
-      LimbSet b = make_set(fast.p + (size_t)i * 2 * E, ext, epids.data(), 2, E);
-      ew_binary(c, 0, a, b, a, st);
-    }
+    lt_sum(c, a, fast.p + 2 * E, 2 * E, n, st);
     moddown(c, fast.p + E, l, out + Q, 1, 0, 0, st);
     c0_ext = true;
     used += n;
