@@ -353,32 +353,6 @@ __global__ __launch_bounds__(kT) void k_moddown_conv_jobs(const MdJob* __restric
   }
 }
 
-// ------------------------------------------------------------------------------ Rescale expansion
-struct RsJob {
-  const uint64_t* top;    // INTT of limb l of one component
-  uint64_t* e;            // limb i of the correction
-  uint32_t l, i;
-};
-
-// k_rescale_expand of fh_keyswitch.hip with (l, i) read from the job
-__global__ __launch_bounds__(kT) void k_rescale_expand_jobs(const RsJob* __restrict__ jobs, const PrimeConst* __restrict__ prime,
-                                                           const uint64_t* __restrict__ QlQl, const uint64_t* __restrict__ QlQl_sh,
-                                                           uint32_t L1, uint32_t N) {
-  RsJob j = jobs[blockIdx.y];
-  j.top = as_global(j.top), j.e = as_global(j.e);
-  const uint64_t ql = prime[j.l].q, qi = prime[j.i].q;
-  const uint64_t half = ql >> 1;
-  const size_t o = (size_t)j.l * L1 + j.i;
-  const uint64_t f = QlQl[o], fsh = QlQl_sh[o];
-  const uint64_t diff = ql > qi ? qi - (ql % qi) : qi - ql;
-  for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < N; n += gridDim.x * blockDim.x) {
-    uint64_t v = j.top[n];
-    if (v > half) v += diff;
-    if (v >= qi) v %= qi;
-    j.e[n] = shoup(v, f, fsh, qi);
-  }
-}
-
 // Reorder NTT job lists prime-major (stable), permuting a companion list the same way:
 // consecutive workgroups then share one prime's twiddle table in L2.
 template <class T>
@@ -511,8 +485,6 @@ struct BatchPlan {
   uint32_t n_md_ntt = 0;
   const LimbJob *t_rs_in = nullptr, *t_rs_out = nullptr;
   uint32_t n_rs_intt = 0;
-  const RsJob* t_rs = nullptr;
-  uint32_t n_rs = 0;
   const LimbJob* t_rs_ntt = nullptr;
   const EpiJob* t_rs_epi = nullptr;
   uint32_t n_rs_ntt = 0;
@@ -762,7 +734,6 @@ void Batch::finalize() {
   std::vector<ModUpJob> mj;
   std::vector<MdJob> mdj;
   std::vector<EpiJob> md_epi, rs_epi;
-  std::vector<RsJob> rj;
   for (const auto& k : ks) {
     const uint32_t lq = k.l + 1, ext = lq + K, beta = c.num_digits(k.l);
     uint64_t* coef = A + k.coef;
@@ -792,7 +763,7 @@ void Batch::finalize() {
       for (uint32_t i = 0; i < lq; ++i) {
         md_ntt.push_back(LimbJob{conv + ((size_t)poly * lq + i) * N, i, 0});
         md_epi.push_back(EpiJob{ex + ((size_t)poly * ext + i) * N, k.out + ((size_t)poly * lq + i) * N, add ? add + (size_t)i * N : nullptr, i,
-                                (uint32_t)k.l});
+                                (uint32_t)k.l, nullptr});
       }
     }
   }
@@ -845,12 +816,13 @@ void Batch::finalize() {
       rs_in.push_back(LimbJob{R + ((size_t)comp * lq + l) * N, l, 0});
       rs_out.push_back(LimbJob{top + (size_t)comp * N, l, 0});
       for (uint32_t ii = 0; ii < l; ++ii) {
-        rj.push_back(RsJob{top + (size_t)comp * N, e + ((size_t)comp * l + ii) * N, l, ii});
         rs_ntt.push_back(LimbJob{e + ((size_t)comp * l + ii) * N, ii, 0});
         if (rs.a)
-          rs_epi.push_back(EpiJob{rs.a + ((size_t)comp * lq + ii) * N, rout + ((size_t)comp * l + ii) * N, rs.pt + (size_t)ii * N, ii, l});
+          rs_epi.push_back(EpiJob{rs.a + ((size_t)comp * lq + ii) * N, rout + ((size_t)comp * l + ii) * N, rs.pt + (size_t)ii * N, ii, l,
+                                  top + (size_t)comp * N});
         else
-          rs_epi.push_back(EpiJob{R + ((size_t)comp * lq + ii) * N, rout + ((size_t)comp * l + ii) * N, nullptr, ii, l});
+          rs_epi.push_back(EpiJob{R + ((size_t)comp * lq + ii) * N, rout + ((size_t)comp * l + ii) * N, nullptr, ii, l,
+                                  top + (size_t)comp * N});
       }
     }
   }
@@ -875,7 +847,7 @@ void Batch::finalize() {
   const size_t o_tensor = tb.put(tj), o_add = tb.put(aj), o_ks_in = tb.put(ks_in), o_ks_out = tb.put(ks_out), o_modup = tb.put(mj),
                o_modup_ntt = tb.put(modup_ntt), o_ki = tb.put(ki), o_kg = tb.put(kg), o_md_in = tb.put(md_in), o_md_out = tb.put(md_out),
                o_md = tb.put(mdj), o_md_ntt = tb.put(md_ntt), o_md_epi = tb.put(md_epi), o_rs_in = tb.put(rs_in), o_rs_out = tb.put(rs_out),
-               o_rs = tb.put(rj), o_rs_ntt = tb.put(rs_ntt), o_rs_epi = tb.put(rs_epi);
+               o_rs_ntt = tb.put(rs_ntt), o_rs_epi = tb.put(rs_epi);
   if (P.tables_cap < tb.bytes.size() || !P.d_tables) {
     // a run on another stream may still read the old tables; runs on the context stream are
     // ordered before any later use of the block returned to the pool
@@ -921,12 +893,10 @@ void Batch::finalize() {
   P.t_rs_in = reinterpret_cast<const LimbJob*>(D + o_rs_in);
   P.t_rs_out = reinterpret_cast<const LimbJob*>(D + o_rs_out);
   P.n_rs_intt = (uint32_t)rs_in.size();
-  P.t_rs = reinterpret_cast<const RsJob*>(D + o_rs);
-  P.n_rs = (uint32_t)rj.size();
   P.t_rs_ntt = reinterpret_cast<const LimbJob*>(D + o_rs_ntt);
   P.t_rs_epi = reinterpret_cast<const EpiJob*>(D + o_rs_epi);
   P.n_rs_ntt = (uint32_t)rs_ntt.size();
-  if (P.n_modup > 65535 || P.n_md > 65535 || P.n_rs > 65535 || P.n_tensor > 65535 || P.n_add > 65535 || P.n_ksk_groups > 65535 ||
+  if (P.n_modup > 65535 || P.n_md > 65535 || P.n_rs_ntt > 65535 || P.n_tensor > 65535 || P.n_add > 65535 || P.n_ksk_groups > 65535 ||
       P.n_mulpt > 65535)
     throw Error(-3, "batch too large for one launch per stage");
   P.final = true;
@@ -984,11 +954,6 @@ void launch_all(Context& c, BatchPlan& P, hipStream_t st) {
   }
   if (P.n_rs_intt) {
     ntt_inv_jobs(c, P.t_rs_in, P.t_rs_out, P.n_rs_intt, st);
-    {
-      ProfScope ps_(c, "rescale_expand", st);
-      k_rescale_expand_jobs<<<grid_tiles(N, P.n_rs, 1), kT, 0, st>>>(P.t_rs, c.d_prime, c.d_rs_QlQl, c.d_rs_QlQl_sh, (uint32_t)c.L1, N);
-    }
-    FH_HIP(hipGetLastError());
     ntt_fwd_jobs_rescale(c, P.t_rs_ntt, P.t_rs_epi, P.n_rs_ntt, st);
   }
   FH_HIP(hipGetLastError());

@@ -100,35 +100,12 @@ __device__ __forceinline__ int64_t coeff_at(const D2* work, uint32_t j, uint32_t
   return (int64_t)llround(v * scale);
 }
 
-__device__ __forceinline__ uint64_t signed_residue(int64_t v, const PrimeConst& P) {
-  if (v >= 0) return barrett128(0, (uint64_t)v, P);
-  uint64_t r = barrett128(0, (uint64_t)(-(v + 1)), P) + 1;
-  if (r == P.q) r = 0;
-  return r ? P.q - r : 0;
-}
-
-// job y = (limb, plaintext) of the output set: the residues of the rounded coefficients
-__global__ __launch_bounds__(kEncThreads) void k_encode_finish(const D2* __restrict__ work, LimbSet out, const PrimeConst* pr, uint32_t N, uint32_t n,
-                                                               int logn, int loggap, double scale) {
-  uint64_t* p;
-  int pid;
-  SetAddr{out}.at(blockIdx.y, N, p, pid);
-  const uint32_t poly = blockIdx.y % out.npolys;
-  const PrimeConst P = pr[pid];
-  const D2* wk = work + (size_t)poly * n;
-  for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < N; j += gridDim.x * blockDim.x)
-    p[j] = signed_residue(coeff_at(wk, j, N, n, logn, loggap, scale), P);
-}
-
-// integer coefficients (count x N, device) -> residues of every limb of the output set
-__global__ __launch_bounds__(kEncThreads) void k_encode_coeffs(const int64_t* __restrict__ m, LimbSet out, const PrimeConst* pr, uint32_t N) {
-  uint64_t* p;
-  int pid;
-  SetAddr{out}.at(blockIdx.y, N, p, pid);
-  const uint32_t poly = blockIdx.y % out.npolys;
-  const PrimeConst P = pr[pid];
-  const int64_t* mp = m + (size_t)poly * N;
-  for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < N; j += gridDim.x * blockDim.x) p[j] = signed_residue(mp[j], P);
+// the rounded coefficients of every plaintext (blockIdx.y), N each
+__global__ __launch_bounds__(kEncThreads) void k_encode_round(const D2* __restrict__ work, int64_t* __restrict__ m, uint32_t N, uint32_t n, int logn,
+                                                              int loggap, double scale) {
+  const D2* wk = work + (size_t)blockIdx.y * n;
+  int64_t* o = m + (size_t)blockIdx.y * N;
+  for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < N; j += gridDim.x * blockDim.x) o[j] = coeff_at(wk, j, N, n, logn, loggap, scale);
 }
 
 inline dim3 enc_grid(uint32_t N, uint32_t jobs) {
@@ -190,7 +167,7 @@ void encode_slots(Context& c, const double* values, int count, uint32_t slots, d
   int logn = 0;
   while ((1u << logn) < n) ++logn;
   const int logM = c.logN + 1, loggap = c.logN - 1 - logn;
-  DBuf vals(c.pool, (size_t)count * n * 2), work(c.pool, (size_t)count * n * 2);
+  DBuf vals(c.pool, (size_t)count * n * 2), work(c.pool, (size_t)count * n * 2), coef(c.pool, (size_t)count * c.N);
   const double2* tw = reinterpret_cast<const double2*>(c.d_ifft_w);
   // chunks of about 8 MB of slot values: the upload of one chunk (synchronous for pageable host
   // memory) overlaps the transforms of the previous one
@@ -200,9 +177,6 @@ void encode_slots(Context& c, const double* values, int count, uint32_t slots, d
     double* v = reinterpret_cast<double*>(vals.p) + (size_t)b0 * n * 2;
     D2* wk = reinterpret_cast<D2*>(work.p) + (size_t)b0 * n;
     FH_HIP(hipMemcpyAsync(v, values + (size_t)b0 * n * 2, (size_t)nb * n * 2 * sizeof(double), hipMemcpyHostToDevice, st));
-    LimbSet part = out;
-    part.base = out.base + (size_t)b0 * out.poly_stride;
-    part.npolys = (uint32_t)nb;
     ProfScope ps_(c, "encode", st);
     k_ifft_load<<<dim3((n + kEncThreads - 1) / kEncThreads, nb), kEncThreads, 0, st>>>(v, wk, n);
     FH_HIP(hipGetLastError());
@@ -215,10 +189,12 @@ void encode_slots(Context& c, const double* values, int count, uint32_t slots, d
       k_ifft_stages_lds<<<dim3(n >> loglen, nb), kEncThreads, 0, st>>>(wk, c.d_ifft_rot, tw, logM, n, loglen);
       FH_HIP(hipGetLastError());
     }
-    k_encode_finish<<<enc_grid(c.N, part.nlimbs * part.npolys), kEncThreads, 0, st>>>(wk, part, c.d_prime, c.N, n, logn, loggap, scale);
+    k_encode_round<<<enc_grid(c.N, (uint32_t)nb), kEncThreads, 0, st>>>(wk, reinterpret_cast<int64_t*>(coef.p) + (size_t)b0 * c.N, c.N, n, logn, loggap,
+                                                                       scale);
     FH_HIP(hipGetLastError());
   }
-  ntt_fwd(c, out, st);
+  // residues modulo every limb's prime in the transform's first launch
+  ntt_fwd_signed(c, reinterpret_cast<const int64_t*>(coef.p), out, st);
 }
 
 void encode_coeffs(Context& c, const int64_t* coeffs, int count, const LimbSet& out, hipStream_t st) {
@@ -227,12 +203,7 @@ void encode_coeffs(Context& c, const int64_t* coeffs, int count, const LimbSet& 
   if (count > 65535 || (size_t)out.nlimbs * count > 65535) throw Error(-1, "encode: too many plaintexts in one call");
   DBuf m(c.pool, (size_t)count * c.N);
   FH_HIP(hipMemcpyAsync(m.p, coeffs, (size_t)count * c.N * sizeof(int64_t), hipMemcpyHostToDevice, st));
-  {
-  ProfScope ps_(c, "encode", st);
-  k_encode_coeffs<<<enc_grid(c.N, out.nlimbs * out.npolys), kEncThreads, 0, st>>>(reinterpret_cast<const int64_t*>(m.p), out, c.d_prime, c.N);
-  FH_HIP(hipGetLastError());
-  }
-  ntt_fwd(c, out, st);
+  ntt_fwd_signed(c, reinterpret_cast<const int64_t*>(m.p), out, st);
 }
 
 }  // namespace fh

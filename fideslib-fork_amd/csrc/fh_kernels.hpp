@@ -40,13 +40,15 @@ __device__ __forceinline__ uint32_t auto_src(uint32_t j, uint32_t k, int logN) {
 }
 
 // Epilogue entry of a fused forward NTT over a job table (same index as the NTT job):
-// ModDown: out = (x - v) [P^-1]_{q_pid} (+ add); Rescale: out = x [q_l^-1]_{q_pid} + v.
+// ModDown: out = (x - v) [P^-1]_{q_pid} (+ add); Rescale: out = x [q_l^-1]_{q_pid} + v, v the transform
+// of the correction formed from `top` (the INTT of limb l).
 struct EpiJob {
   const uint64_t* x;
   uint64_t* out;
   const uint64_t* add;
   uint32_t pid;
   uint32_t l;
+  const uint64_t* top;
 };
 
 // A buffer pointer that a kernel reads from a job table, for accesses through the global address space.
@@ -204,12 +206,18 @@ struct AutotuneResult {
 AutotuneResult autotune_ntt(Context& c, int polys);
 void ntt_fwd_jobs(const Context& c, const LimbJob* d_jobs, uint32_t njobs, hipStream_t st, bool cols = true);
 // Forward NTT of the ModDown conversion (conv: npolys x lq limbs over Q_l, coefficient form, used as
-// scratch) fused with the ModDown combination: out_i = (x_i - NTT(conv)_i) * [P^-1]_{q_i}.
+// scratch) fused with the ModDown combination: out_i = (x_i - NTT(conv)_i) * [P^-1]_{q_i} (+ add_i,
+// polynomial b's at add + (b / 2) add_pair + (b % 2) lq N when add is set).
 void ntt_fwd_moddown(const Context& c, const LimbSet& conv, const uint64_t* x, uint64_t x_stride, uint64_t* out, uint64_t out_stride,
-                     hipStream_t st, bool cols = true);
-// Forward NTT of the Rescale correction e (npolys x l limbs, coefficient form, scratch) fused with
-// the Rescale combination: out_i = x_i * [q_l^-1]_{q_i} + NTT(e)_i.
-void ntt_fwd_rescale(const Context& c, const LimbSet& e, const uint64_t* x, uint32_t l, uint64_t* out, hipStream_t st);
+                     hipStream_t st, bool cols = true, const uint64_t* add = nullptr, uint64_t add_pair = 0);
+// Forward NTT of the Rescale correction e (scratch: npolys x l limbs), formed from the dropped limbs
+// top (npolys limbs, coefficient form), fused with the Rescale combination: out_i = x_i * [q_l^-1]_{q_i}
+// + NTT(e)_i.
+void ntt_fwd_rescale(const Context& c, const LimbSet& e, const uint64_t* top, const uint64_t* x, uint32_t l, uint64_t* out, hipStream_t st);
+// forward NTT of tower 0 (x0: npolys limbs, coefficient form) lifted to every limb of out
+void ntt_fwd_mod_raise(const Context& c, const uint64_t* x0, const LimbSet& out, hipStream_t st);
+// forward NTT of npolys x N signed integer coefficients modulo every limb of out
+void ntt_fwd_signed(const Context& c, const int64_t* m, const LimbSet& out, hipStream_t st);
 void ntt_inv_jobs(const Context& c, const LimbJob* d_jobs, uint32_t njobs, hipStream_t st);
 // out-of-place job forms: job y reads in[y].ptr and writes out[y].ptr (same prime)
 void ntt_fwd_jobs(const Context& c, const LimbJob* d_in, const LimbJob* d_out, uint32_t njobs, hipStream_t st);

@@ -459,56 +459,6 @@ __global__ __launch_bounds__(kT) void k_moddown_conv_r(const uint64_t* __restric
   }
 }
 
-// ----------------------------------------------------------------------------------- Rescale
-struct RescaleParams {
-  uint32_t N, l, L1;
-  const PrimeConst* prime;
-  const uint64_t* qlinv;     // [L1][L1]
-  const uint64_t* qlinv_sh;
-  const uint64_t* QlQl;      // [L1][L1]
-  const uint64_t* QlQl_sh;
-};
-
-// blockIdx.y = comp * l + i: e_i = SwitchModulus_{q_l -> q_i}(top) * QlQl[l][i] (coefficient form)
-__global__ __launch_bounds__(kT) void k_rescale_expand(const uint64_t* __restrict__ top, uint64_t* __restrict__ e, RescaleParams rp) {
-  const uint32_t comp = blockIdx.y / rp.l, i = blockIdx.y % rp.l;
-  const uint64_t ql = rp.prime[rp.l].q, qi = rp.prime[i].q;
-  const uint64_t half = ql >> 1;
-  const size_t o = (size_t)rp.l * rp.L1 + i;
-  const uint64_t f = rp.QlQl[o], fsh = rp.QlQl_sh[o];
-  // OpenFHE NativeVector::SwitchModulus, old modulus q_l > or < q_i
-  const uint64_t diff = ql > qi ? qi - (ql % qi) : qi - ql;
-  const uint64_t* t = top + (size_t)comp * rp.N;
-  uint64_t* ei = e + ((size_t)comp * rp.l + i) * rp.N;
-  for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < rp.N; n += gridDim.x * blockDim.x) {
-    uint64_t v = t[n];
-    if (v > half) v += diff;
-    if (v >= qi) v %= qi;
-    ei[n] = shoup(v, f, fsh, qi);
-  }
-}
-
-// ----------------------------------------------------------------------------------- ModRaise
-// blockIdx.y = comp * (l+1) + i: out_i = SwitchModulus_{q_0 -> q_i}(x) of the coefficient-form
-// tower 0 of each component (the reference's tower-0 broadcast, ElemenwiseBatchKernels.cu:140-148).
-__global__ __launch_bounds__(kT) void k_mod_raise(const uint64_t* __restrict__ x0, uint64_t* __restrict__ out, uint32_t N, uint32_t l,
-                                                   const PrimeConst* __restrict__ prime) {
-  const uint32_t comp = blockIdx.y / (l + 1), i = blockIdx.y % (l + 1);
-  const uint64_t q0 = prime[0].q, qi = prime[i].q;
-  const uint64_t half = q0 >> 1;
-  const uint64_t diff = q0 > qi ? qi - (q0 % qi) : qi - q0;
-  const uint64_t* t = x0 + (size_t)comp * N;
-  uint64_t* o = out + ((size_t)comp * (l + 1) + i) * N;
-  for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < N; n += gridDim.x * blockDim.x) {
-    uint64_t v = t[n];
-    if (i != 0) {
-      if (v > half) v += diff;
-      if (v >= qi) v %= qi;
-    }
-    o[n] = v;
-  }
-}
-
 // ----------------------------------------------------------------------------------- automorphism
 __global__ __launch_bounds__(kT) void k_automorph(const uint64_t* __restrict__ in, uint64_t* __restrict__ out, uint32_t N, uint32_t logN,
                                                    uint32_t k) {
@@ -588,7 +538,8 @@ namespace {
 inline bool overlaps(const uint64_t* a, size_t an, const uint64_t* b, size_t bn) { return a < b + bn && b < a + an; }
 }  // namespace
 
-void moddown(Context& c, const uint64_t* x, int l, uint64_t* out, int npolys, uint64_t x_stride, uint64_t out_stride, hipStream_t st) {
+void moddown(Context& c, const uint64_t* x, int l, uint64_t* out, int npolys, uint64_t x_stride, uint64_t out_stride, hipStream_t st,
+             const uint64_t* add, uint64_t add_pair) {
   const uint32_t lq = l + 1, ext = lq + c.K, K = c.K;
   if (K > (uint32_t)kMaxK) throw Error(-3, "special prime count above kernel limit");
   if (npolys < 1) return;
@@ -598,7 +549,7 @@ void moddown(Context& c, const uint64_t* x, int l, uint64_t* out, int npolys, ui
   if (overlaps(x, xn, out, on)) {
     // the fused epilogue reads x while other blocks write out: go through a separate buffer
     DBuf tmp(c.pool, (size_t)npolys * lq * c.N);
-    moddown(c, x, l, tmp.p, npolys, x_stride, (uint64_t)lq * c.N, st);
+    moddown(c, x, l, tmp.p, npolys, x_stride, (uint64_t)lq * c.N, st, add, add_pair);
     for (int b = 0; b < npolys; ++b)
       FH_HIP(hipMemcpyAsync(out + b * out_stride, tmp.p + (size_t)b * lq * c.N, (size_t)lq * c.N * 8, hipMemcpyDeviceToDevice, st));
     return;
@@ -624,7 +575,8 @@ void moddown(Context& c, const uint64_t* x, int l, uint64_t* out, int npolys, ui
   }
   FH_HIP(hipGetLastError());
   // forward NTT of the conversion with (x_i - conv_i) * P^-1 fused into its last launch
-  ntt_fwd_moddown(c, make_set(conv.p, lq, qids.data(), npolys, (uint64_t)lq * c.N), x, x_stride, out, out_stride, st, !fused);
+  ntt_fwd_moddown(c, make_set(conv.p, lq, qids.data(), npolys, (uint64_t)lq * c.N), x, x_stride, out, out_stride, st, !fused, add,
+                  add_pair);
 }
 
 void rescale(Context& c, const uint64_t* x, int l, int ncomp, uint64_t* out, hipStream_t st) {
@@ -650,13 +602,11 @@ void rescale_core(Context& c, const uint64_t* x, int l, int ncomp, uint64_t* out
   // INTT of the top limb of every component straight into a packed buffer
   ntt_inv(c, make_set(const_cast<uint64_t*>(x) + (size_t)l * c.N, 1, &pid_top, ncomp, (uint64_t)(l + 1) * c.N),
           make_set(top, 1, &pid_top, ncomp, c.N), st);
-  RescaleParams rp{c.N, (uint32_t)l, (uint32_t)c.L1, c.d_prime, c.d_rs_qlinv, c.d_rs_qlinv_sh, c.d_rs_QlQl, c.d_rs_QlQl_sh};
-  { ProfScope ps_(c, "rescale_expand", st); k_rescale_expand<<<grid_n(c.N, ncomp * l), kT, 0, st>>>(top, e, rp); }
-  FH_HIP(hipGetLastError());
   int ids[kMaxLimbs];   // on the stack: this path makes no allocation of any kind
   for (int i = 0; i < l; ++i) ids[i] = i;
-  // forward NTT of the correction with x_i * q_l^-1 + e_i fused into its last launch
-  ntt_fwd_rescale(c, make_set(e, l, ids, ncomp, (uint64_t)l * c.N), x, (uint32_t)l, out, st);
+  // forward NTT of the correction, formed from the top limbs in its first launch, with
+  // x_i * q_l^-1 + e_i fused into its last
+  ntt_fwd_rescale(c, make_set(e, l, ids, ncomp, (uint64_t)l * c.N), top, x, (uint32_t)l, out, st);
 }
 
 void mod_raise(Context& c, const uint64_t* x, int l_in, int ncomp, int l, uint64_t* out, hipStream_t st) {
@@ -667,11 +617,9 @@ void mod_raise(Context& c, const uint64_t* x, int l_in, int ncomp, int l, uint64
   int pid0 = 0;
   // tower 0 of every component to coefficient form, packed
   ntt_inv(c, make_set(const_cast<uint64_t*>(x), 1, &pid0, ncomp, (uint64_t)(l_in + 1) * c.N), make_set(t0.p, 1, &pid0, ncomp, c.N), st);
-  { ProfScope ps_(c, "mod_raise", st); k_mod_raise<<<grid_n(c.N, ncomp * (l + 1)), kT, 0, st>>>(t0.p, out, c.N, (uint32_t)l, c.d_prime); }
-  FH_HIP(hipGetLastError());
   std::vector<int> ids(l + 1);
   for (int i = 0; i <= l; ++i) ids[i] = i;
-  ntt_fwd(c, make_set(out, l + 1, ids.data(), ncomp, (uint64_t)(l + 1) * c.N), st);
+  ntt_fwd_mod_raise(c, t0.p, make_set(out, l + 1, ids.data(), ncomp, (uint64_t)(l + 1) * c.N), st);
 }
 
 void automorph(Context& c, const uint64_t* x, int nlimbs, uint32_t k, uint64_t* out, hipStream_t st) {
@@ -681,18 +629,14 @@ void automorph(Context& c, const uint64_t* x, int nlimbs, uint32_t k, uint64_t* 
   FH_HIP(hipGetLastError());
 }
 
-// ks = ModDown(<ModUp(c2), key>); out = (c0 + ks0, c1 + ks1)
+// ks = ModDown(<ModUp(c2), key>); out = (c0 + ks0, c1 + ks1), the sum in the ModDown's epilogue
 void relinearize(Context& c, const uint64_t* ct3, int l, const uint64_t* key, uint64_t* out2, hipStream_t st) {
   const uint32_t lq = l + 1, ext = lq + c.K, beta = c.num_digits(l);
   const size_t P = (size_t)lq * c.N;
-  DBuf dig(c.pool, (size_t)beta * ext * c.N), t(c.pool, (size_t)2 * ext * c.N), ks(c.pool, 2 * P);
+  DBuf dig(c.pool, (size_t)beta * ext * c.N), t(c.pool, (size_t)2 * ext * c.N);
   modup_batch(c, ct3 + 2 * P, l, 1, 0, dig.p, st, false);
   ksk_inner(c, dig.p, l, key, t.p, t.p + (size_t)ext * c.N, nullptr, 1, st, false, ct3 + 2 * P);
-  moddown(c, t.p, l, ks.p, 2, 0, 0, st);
-  std::vector<int> ids(lq);
-  for (uint32_t i = 0; i < lq; ++i) ids[i] = i;
-  ew_binary(c, 0, make_set(const_cast<uint64_t*>(ct3), lq, ids.data(), 2, P), make_set(ks.p, lq, ids.data(), 2, P),
-            make_set(out2, lq, ids.data(), 2, P), st);
+  moddown(c, t.p, l, out2, 2, 0, 0, st, ct3, 2 * P);
 }
 
 void eval_mult(Context& c, const uint64_t* ct1, const uint64_t* ct2, int l, const uint64_t* key, uint64_t* out2, hipStream_t st) {
@@ -712,19 +656,14 @@ void eval_mult_many(Context& c, int n, const uint64_t* ct1, int limbs1, const ui
     ew_tensor(c, ct1, ct2, t.p, (int)lq, st, 1, limbs1, limbs2);
     return relinearize(c, t.p, l, key, out2, st);
   }
-  DBuf t(c.pool, (size_t)n * 3 * P), dig(c.pool, (size_t)n * beta * E), eo(c.pool, (size_t)n * 2 * E), ks(c.pool, (size_t)n * 2 * P);
+  DBuf t(c.pool, (size_t)n * 3 * P), dig(c.pool, (size_t)n * beta * E), eo(c.pool, (size_t)n * 2 * E);
   ew_tensor(c, ct1, ct2, t.p, (int)lq, st, n, limbs1, limbs2);
   // every d2 through one ModUp, one grouped key inner product (the key read once) and one ModDown
   modup_batch(c, t.p + 2 * P, l, n, 3 * P, dig.p, st, false);
   std::vector<const uint64_t*> keys(n, key);
   std::vector<uint32_t> gal(n, 1);
   ksk_items(c, n, 1, dig.p, (uint64_t)beta * E, nullptr, 0, false, false, l, keys.data(), gal.data(), eo.p, 2 * E, st, t.p + 2 * P, 3 * P);
-  moddown(c, eo.p, l, ks.p, 2 * n, E, P, st);
-  std::vector<int> ids(lq);
-  for (uint32_t i = 0; i < lq; ++i) ids[i] = i;
-  for (int b = 0; b < n; ++b)
-    ew_binary(c, 0, make_set(t.p + (size_t)b * 3 * P, lq, ids.data(), 2, P), make_set(ks.p + (size_t)b * 2 * P, lq, ids.data(), 2, P),
-              make_set(out2 + (size_t)b * 2 * P, lq, ids.data(), 2, P), st);
+  moddown(c, eo.p, l, out2, 2 * n, E, P, st, t.p, 3 * P);
 }
 
 // hoisted formulation: ext key switch of c1 (+ P c0), automorph, result over Q_l ∪ P

@@ -96,8 +96,10 @@ void linear_transform_batch(Context& c, int count, const uint64_t* cts, uint64_t
                             int offset, int slots, const uint64_t* diags, const uint64_t* const* baby_keys, const uint32_t* baby_gal,
                             const uint64_t* giant_key, uint32_t giant_gal, const uint64_t* off_key, uint32_t off_gal, uint64_t* out,
                             hipStream_t st);
-// npolys polynomials over Q_l ∪ P (x_stride words apart, 0 = packed) -> over Q_l (out_stride apart)
-void moddown(Context& c, const uint64_t* x, int l, uint64_t* out, int npolys, uint64_t x_stride, uint64_t out_stride, hipStream_t st);
+// npolys polynomials over Q_l ∪ P (x_stride words apart, 0 = packed) -> over Q_l (out_stride apart);
+// add (optional): polynomials 2 j and 2 j + 1 gain the two at add + j add_pair (l+1 limbs each)
+void moddown(Context& c, const uint64_t* x, int l, uint64_t* out, int npolys, uint64_t x_stride, uint64_t out_stride, hipStream_t st,
+             const uint64_t* add = nullptr, uint64_t add_pair = 0);
 // ncomp components over Q_l -> over Q_{l-1}
 void rescale(Context& c, const uint64_t* x, int l, int ncomp, uint64_t* out, hipStream_t st);
 // Rescale with its work buffer supplied by the caller (rescale_work_words words: the INTT of the top

@@ -1,5 +1,5 @@
-// NTT / INTT entry points over limb sets (in place and out of place, with the ModDown and Rescale
-// epilogues), and the NTT launch-shape autotuner. The kernels are in fh_ntt_impl.hpp.
+// NTT / INTT entry points over limb sets (in place and out of place, with the ModDown
+// epilogue), and the NTT launch-shape autotuner. The kernels are in fh_ntt_impl.hpp.
 #include "fh_ntt_impl.hpp"
 #include "fh_ops.hpp"
 
@@ -16,15 +16,9 @@ void ntt_inv(const Context& c, const LimbSet& in, const LimbSet& out, hipStream_
   dispatch(c, SetAddr{in}, SetAddr{out}, in.nlimbs * in.npolys, st, false);
 }
 void ntt_fwd_moddown(const Context& c, const LimbSet& conv, const uint64_t* x, uint64_t x_stride, uint64_t* out, uint64_t out_stride,
-                     hipStream_t st, bool cols) {
-  EpiModDown e{x, x_stride, out, out_stride, c.d_md_pinv, c.d_md_pinv_sh, conv.npolys, nullptr, nullptr, 0, 0, 0};
+                     hipStream_t st, bool cols, const uint64_t* add, uint64_t add_pair) {
+  EpiModDown e{x, x_stride, out, out_stride, add, add_pair, c.d_md_pinv, c.d_md_pinv_sh, conv.npolys, conv.nlimbs, nullptr, nullptr, nullptr, 0, 0, 0};
   dispatch(c, SetAddr{conv}, SetAddr{conv}, conv.nlimbs * conv.npolys, st, true, e, "ntt_fwd_rows_moddown", cols);
-}
-
-void ntt_fwd_rescale(const Context& c, const LimbSet& e, const uint64_t* x, uint32_t l, uint64_t* out, hipStream_t st) {
-  const size_t o = (size_t)l * c.L1;
-  EpiRescale ep{x, out, c.d_rs_qlinv + o, c.d_rs_qlinv_sh + o, l, e.npolys, nullptr, nullptr, 0, 0, 0};
-  dispatch(c, SetAddr{e}, SetAddr{e}, e.nlimbs * e.npolys, st, true, ep, "ntt_fwd_rows_rescale");
 }
 
 // ------------------------------------------------------------------------------- autotuner

@@ -297,6 +297,89 @@ struct OpaqueTid {
   }
 };
 
+// ------------------------------------------------------------------------------- forward prologues
+// The first launch of a forward NTT takes its inputs through a prologue, which either reads the limb
+// (ProLoad) or forms it from what it comes from: the Rescale correction from the dropped limb, a
+// raised limb from tower 0, an encoded limb from the integer coefficients. The limb's values are
+// then neither written by a launch of their own nor read back. Job y as in the epilogues.
+struct ProLoad {
+  __device__ __forceinline__ void init(uint32_t, uint32_t, const PrimeConst*) {}
+  __device__ __forceinline__ uint64_t value(const uint64_t* p, uint32_t n) const { return p[n]; }
+};
+
+// e_i = SwitchModulus_{q_l -> q_i}(top) * QlQl[l][i] (OpenFHE NativeVector::SwitchModulus: values above
+// q_l / 2 shift by the difference of the moduli; the product takes the word unreduced)
+struct SwitchMod {
+  const uint64_t* t;
+  uint64_t half, diff, qi, f, fsh;
+  __device__ __forceinline__ void set(const uint64_t* top, uint64_t ql, uint64_t q, uint64_t w, uint64_t wsh) {
+    t = top;
+    half = ql >> 1;
+    diff = ql > q ? q - (ql % q) : q - ql;
+    qi = q;
+    f = w;
+    fsh = wsh;
+  }
+  __device__ __forceinline__ uint64_t at(uint32_t n) const {
+    const uint64_t v = t[n];
+    return shoup(v > half ? v + diff : v, f, fsh, qi);
+  }
+};
+
+struct ProRescale {
+  const uint64_t* top;     // npolys limbs, coefficient form modulo q_l
+  const uint64_t* w;       // QlQl row of level l, Shoup companions
+  const uint64_t* wsh;
+  uint32_t l, npolys;
+  SwitchMod s;
+  __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime) {
+    const uint32_t i = y / npolys, b = y % npolys;
+    s.set(top + (size_t)b * N, prime[l].q, prime[i].q, w[i], wsh[i]);
+  }
+  __device__ __forceinline__ uint64_t value(const uint64_t*, uint32_t n) const { return s.at(n); }
+};
+
+// limb i of component b raised from tower 0 (centred lift modulo q_0)
+struct ProModRaise {
+  const uint64_t* x0;      // npolys limbs, coefficient form modulo q_0
+  uint32_t npolys;
+  const uint64_t* t;
+  uint64_t half, diff;
+  uint32_t i;
+  PrimeConst P;
+  __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime) {
+    i = y / npolys;
+    t = x0 + (size_t)(y % npolys) * N;
+    P = prime[i];
+    const uint64_t q0 = prime[0].q;
+    half = q0 >> 1;
+    diff = q0 > P.q ? P.q - (q0 % P.q) : P.q - q0;
+  }
+  __device__ __forceinline__ uint64_t value(const uint64_t*, uint32_t n) const {
+    const uint64_t v = t[n];
+    return i == 0 ? v : barrett128(0, v > half ? v + diff : v, P);
+  }
+};
+
+// residues of signed integer coefficients: plaintext y % npolys of N coefficients, limb y / npolys
+struct ProSigned {
+  const int64_t* m;
+  LimbSet s;
+  const int64_t* t;
+  PrimeConst P;
+  __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime) {
+    t = m + (size_t)(y % s.npolys) * N;
+    P = prime[s.pid[y / s.npolys]];
+  }
+  __device__ __forceinline__ uint64_t value(const uint64_t*, uint32_t n) const {
+    const int64_t v = t[n];
+    if (v >= 0) return barrett128(0, (uint64_t)v, P);
+    uint64_t r = barrett128(0, (uint64_t)(-(v + 1)), P) + 1;
+    if (r == P.q) r = 0;
+    return r ? P.q - r : 0;
+  }
+};
+
 // ------------------------------------------------------------------------------- forward, columns
 // The l1 stages of one column held by T = S / 16 threads, 16 elements each. First half (lo): stages
 // 0..3 on element k at row r0 + T k. Second half (hi, LS > 4): the rest on element k at row
@@ -333,10 +416,11 @@ __device__ __forceinline__ void fwd_cols_hi(const A& ar, typename A::T (&x)[16],
   for (int k = 0; k < 16; ++k) ar.settle_fwd(x[k], b[k]);
 }
 
-// First l1 stages. Input: canonical (in place or out of place), output: internal form.
-template <int LS, class Tid = PlainTid, class A, class TwT>
+// First l1 stages. Input: canonical (in place or out of place), output: internal form. pro: what
+// the inputs are, given the limb's words (ProLoad: the words).
+template <int LS, class Tid = PlainTid, class A, class TwT, class Pro>
 __device__ __forceinline__ void fwd_cols_body(const A& ar, const TwT* tw, const TwT* twsh, uint64_t* sw, uint64_t* swp, const uint64_t* p,
-                                              uint64_t* po, uint64_t* tile, uint32_t N2, int C, uint32_t bx) {
+                                              uint64_t* po, uint64_t* tile, uint32_t N2, int C, const Pro& pro, uint32_t bx) {
   constexpr int S = 1 << LS, T = S / 16, PADS = S + 1;
   const int tid = Tid::get();
   const int cc = tid % C, r0 = tid / C;
@@ -344,7 +428,7 @@ __device__ __forceinline__ void fwd_cols_body(const A& ar, const TwT* tw, const 
   typename A::T x[16];
   stage_tw(ar, sw, swp, tw, twsh, S);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) x[k] = ar.from_canon(p[(size_t)(r0 + T * k) * N2 + col]);
+  for (int k = 0; k < 16; ++k) x[k] = ar.from_canon(pro.value(p, (r0 + T * k) * N2 + col));
   __syncthreads();
   int b[16];
 #pragma unroll
@@ -366,8 +450,8 @@ __device__ __forceinline__ void fwd_cols_body(const A& ar, const TwT* tw, const 
   }
 }
 
-template <int LS, int TH, class Addr, class AddrOut>
-__global__ __launch_bounds__(TH) void k_ntt_fwd_cols(Addr ad, AddrOut ao, NttTables tb) {
+template <int LS, int TH, class Addr, class AddrOut, class Pro>
+__global__ __launch_bounds__(TH) void k_ntt_fwd_cols(Addr ad, AddrOut ao, NttTables tb, Pro pro) {
   constexpr int S = 1 << LS, T = S / 16, PADS = S + 1, CMAX = TH / T;
   __shared__ uint64_t tile[CMAX * PADS];
   __shared__ uint64_t sw[S], swp[S];
@@ -375,11 +459,12 @@ __global__ __launch_bounds__(TH) void k_ntt_fwd_cols(Addr ad, AddrOut ao, NttTab
   int pid, pido;
   ad.at(blockIdx.y, tb.N, p, pid);
   ao.at(blockIdx.y, tb.N, po, pido);
+  pro.init(blockIdx.y, tb.N, tb.prime);
   const Sel sel = select(tb, pid, false);
   const int C = blockDim.x / T;
   const uint32_t N2 = tb.N >> LS;
   with_arith(sel, [&](const auto& ar, const auto* tw, const auto* twsh) {
-    fwd_cols_body<LS>(ar, tw, twsh, sw, swp, p, po, tile, N2, C, blockIdx.x);
+    fwd_cols_body<LS>(ar, tw, twsh, sw, swp, p, po, tile, N2, C, pro, blockIdx.x);
   });
 }
 
@@ -570,25 +655,31 @@ struct EpiModDown {
   uint64_t x_stride;
   uint64_t* out;           // Q_l polys, limb i of poly b at out + b * out_stride + i * N
   uint64_t out_stride;
+  const uint64_t* add;     // optional: added to the result; polys 2 j, 2 j + 1 back to back at add + j * add_pair
+  uint64_t add_pair;
   const uint64_t* w;       // [P^-1]_{q_i}, Shoup companions
   const uint64_t* wsh;
-  uint32_t npolys;
+  uint32_t npolys, nlimbs;
   // per block
   const uint64_t* xi;
   uint64_t* oi;
+  const uint64_t* ai;
   uint64_t q, wi, wish;
   __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime) {
     const uint32_t i = y / npolys, b = y % npolys;
     xi = x + b * x_stride + (size_t)i * N;
     oi = out + b * out_stride + (size_t)i * N;
+    ai = add ? add + (size_t)(b >> 1) * add_pair + ((size_t)(b & 1) * nlimbs + i) * N : nullptr;
     q = prime[i].q;
     wi = w[i];
     wish = wsh[i];
   }
-  using In = uint64_t;
-  __device__ __forceinline__ In load(uint32_t j) const { return xi[j]; }
-  __device__ __forceinline__ void store(uint64_t*, uint32_t rbase, uint32_t j, uint64_t v, In x) const {
-    oi[rbase + j] = shoup(sub_mod(x, v, q), wi, wish, q);
+  struct In {
+    uint64_t x, a;
+  };
+  __device__ __forceinline__ In load(uint32_t j) const { return In{xi[j], ai ? ai[j] : 0}; }
+  __device__ __forceinline__ void store(uint64_t*, uint32_t rbase, uint32_t j, uint64_t v, In e) const {
+    oi[rbase + j] = add_mod(e.a, shoup(sub_mod(e.x, v, q), wi, wish, q), q);
   }
 };
 
@@ -930,8 +1021,9 @@ __device__ __forceinline__ void team_arith(const Sel& s, F&& f) {
 // of work; two limbs per team are in flight (two alternating counter slots, targets W per use).
 // One launch per arithmetic (FP: the fp64 path of the 50-bit primes, else integer Shoup): a team
 // skips the limbs of the other kind, and each kernel holds one path's registers only.
-template <int LS, int TH, bool FP, class Addr, class AddrOut, class Epi>
-__global__ __launch_bounds__(TH) __attribute__((amdgpu_waves_per_eu(3))) void k_ntt_fwd_team(Addr ad, AddrOut ao, NttTables tb, Epi epi, TeamArgs ta) {
+template <int LS, int TH, bool FP, class Addr, class AddrOut, class Epi, class Pro>
+__global__ __launch_bounds__(TH) __attribute__((amdgpu_waves_per_eu(3))) void k_ntt_fwd_team(Addr ad, AddrOut ao, NttTables tb, Epi epi, TeamArgs ta,
+                                                                                             Pro pro) {
   constexpr int S = 1 << LS, T = S / 16, CMAX = TH / T;
   constexpr int TW = CMAX * RowTile<LS>::PAD > CMAX * (S + 1) ? CMAX * RowTile<LS>::PAD : CMAX * (S + 1);
   __shared__ uint64_t tile[TW];
@@ -959,10 +1051,12 @@ __global__ __launch_bounds__(TH) __attribute__((amdgpu_waves_per_eu(3))) void k_
     int pid, pido;
     ad.at(y, tb.N, p, pid);
     ao.at(y, tb.N, po, pido);
+    Pro pr = pro;
+    pr.init(y, tb.N, tb.prime);
     const Sel sel = select(tb, pid, false);
     __syncthreads();   // earlier readers of sw / tile are done
     team_arith<FP>(sel, [&](const auto& ar, const auto* tw, const auto* twsh) {
-      fwd_cols_body<LS, OpaqueTid>(ar, tw, twsh, sw, swp, p, po, tile, N2, C, opaque(m));
+      fwd_cols_body<LS, OpaqueTid>(ar, tw, twsh, sw, swp, p, po, tile, N2, C, pr, opaque(m));
     });
     team_arrive(slot + (k & 1), formal);
   };
@@ -1139,6 +1233,28 @@ struct EpiRescaleJobs {
   }
 };
 
+struct ProRescaleJobs {
+  const EpiJob* jobs;
+  const uint64_t* w;       // [L1][L1] QlQl, Shoup companions
+  const uint64_t* wsh;
+  uint32_t L1;
+  SwitchMod s;
+  __device__ __forceinline__ void init(uint32_t y, uint32_t, const PrimeConst* prime) {
+    const EpiJob j = jobs[y];
+    const size_t o = (size_t)j.l * L1 + j.pid;
+    s.set(as_global(j.top), prime[j.l].q, prime[j.pid].q, w[o], wsh[o]);
+  }
+  __device__ __forceinline__ uint64_t value(const uint64_t*, uint32_t n) const { return s.at(n); }
+};
+
+template <class Pro>
+struct ShiftPro {
+  Pro p;
+  uint32_t base;
+  __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime) { p.init(y + base, N, prime); }
+  __device__ __forceinline__ uint64_t value(const uint64_t* x, uint32_t n) const { return p.value(x, n); }
+};
+
 template <class Epi>
 struct ShiftEpi {
   Epi e;
@@ -1157,12 +1273,12 @@ inline uint32_t chunk_limbs(const Context& c) {
 }
 
 // One launch of each pass kind, at workgroup size TH.
-template <int LS, int TH, class Addr, class AddrOut>
-void launch_fwd_cols(const Context& c, const Addr& a, const AddrOut& o, uint32_t n, const NttTables& tb, hipStream_t st) {
+template <int LS, int TH, class Addr, class AddrOut, class Pro>
+void launch_fwd_cols(const Context& c, const Addr& a, const AddrOut& o, uint32_t n, const NttTables& tb, hipStream_t st, const Pro& pro) {
   const dim3 b = col_block<LS, TH>(c.N);
   const uint32_t C = b.x / ((1 << LS) / 16);
   ProfScope ps_(c, "ntt_fwd_cols", st);
-  k_ntt_fwd_cols<LS, TH><<<dim3((c.N >> LS) / C, n), b, 0, st>>>(a, o, tb);
+  k_ntt_fwd_cols<LS, TH><<<dim3((c.N >> LS) / C, n), b, 0, st>>>(a, o, tb, pro);
 }
 template <int LS, int TH, class AddrOut, class Epi>
 void launch_fwd_rows(const Context& c, const AddrOut& o, uint32_t n, const NttTables& tb, hipStream_t st, const Epi& e, const char* name) {
@@ -1227,13 +1343,13 @@ inline const char* team_name(const char* rows_name) {
   return "ntt_fwd_team";
 }
 
-template <int LS, class Addr, class AddrOut, class Epi>
+template <int LS, class Addr, class AddrOut, class Epi, class Pro>
 bool launch_fwd_team(const Context& c, const Addr& a, const AddrOut& o, uint32_t n, const NttTables& tb, hipStream_t st, const Epi& e,
-                     const char* rows_name) {
+                     const char* rows_name, const Pro& pro) {
   constexpr int TH = kNttThreads, T = (1 << LS) / 16, C = TH / T;
   constexpr uint32_t W = (1u << LS) / C;
-  const void* fns[2] = {reinterpret_cast<const void*>(&k_ntt_fwd_team<LS, TH, true, Addr, AddrOut, Epi>),
-                        reinterpret_cast<const void*>(&k_ntt_fwd_team<LS, TH, false, Addr, AddrOut, Epi>)};
+  const void* fns[2] = {reinterpret_cast<const void*>(&k_ntt_fwd_team<LS, TH, true, Addr, AddrOut, Epi, Pro>),
+                        reinterpret_cast<const void*>(&k_ntt_fwd_team<LS, TH, false, Addr, AddrOut, Epi, Pro>)};
   static int occ[2] = {-1, -1};
   TeamArgs ta[2];
   for (int k = 0; k < 2; ++k) {
@@ -1243,7 +1359,7 @@ bool launch_fwd_team(const Context& c, const Addr& a, const AddrOut& o, uint32_t
   ProfScope ps_(c, team_name(rows_name), st);
   for (int k = 0; k < 2; ++k) {
     team_reset(c, ta[k], st);
-    void* args[] = {(void*)&a, (void*)&o, (void*)&tb, (void*)&e, (void*)&ta[k]};
+    void* args[] = {(void*)&a, (void*)&o, (void*)&tb, (void*)&e, (void*)&ta[k], (void*)&pro};
     FH_HIP(hipLaunchCooperativeKernel(fns[k], dim3(ta[k].nteams * W), dim3(TH), args, 0, st));
   }
   return true;
@@ -1298,12 +1414,12 @@ struct ChunkStreams {
 };
 
 // cols false: the limbs have had their column pass (conv_cols), only the row pass runs
-template <class Addr, class AddrOut, int L1S, int L2S, bool WIDE, class Epi>
+template <class Addr, class AddrOut, int L1S, int L2S, bool WIDE, class Epi, class Pro>
 void fwd_impl(const Context& c, const Addr& ad, const AddrOut& ao, uint32_t nlimbs, hipStream_t st0, const Epi& epi, const char* rows_name,
-              bool cols) {
+              bool cols, const Pro& pro) {
   NttTables tb = ntt_tables(c);
   if constexpr (L1S == L2S && L1S >= 6) {
-    if (cols && team_ok<L1S, L2S>(c, st0) && launch_fwd_team<L1S>(c, ad, ao, nlimbs, tb, st0, epi, rows_name)) return;
+    if (cols && team_ok<L1S, L2S>(c, st0) && launch_fwd_team<L1S>(c, ad, ao, nlimbs, tb, st0, epi, rows_name, pro)) return;
   }
   const bool wc = WIDE && c.tune.ntt_threads[0] == kNttWide, wr = WIDE && c.tune.ntt_threads[1] == kNttWide;
   const uint32_t chunk = chunk_limbs(c);
@@ -1314,13 +1430,14 @@ void fwd_impl(const Context& c, const Addr& ad, const AddrOut& ao, uint32_t nlim
     Shift<Addr> sa{ad, base};
     Shift<AddrOut> so{ao, base};
     ShiftEpi<Epi> se{epi, base};
+    ShiftPro<Pro> sp{pro, base};
     if constexpr (WIDE) {
-      if (cols && wc) launch_fwd_cols<L1S, kNttWide>(c, sa, so, n, tb, st);
-      else if (cols) launch_fwd_cols<L1S, kNttThreads>(c, sa, so, n, tb, st);
+      if (cols && wc) launch_fwd_cols<L1S, kNttWide>(c, sa, so, n, tb, st, sp);
+      else if (cols) launch_fwd_cols<L1S, kNttThreads>(c, sa, so, n, tb, st, sp);
       if (wr) launch_fwd_rows<L2S, kNttWide>(c, so, n, tb, st, se, rows_name);
       else launch_fwd_rows<L2S, kNttThreads>(c, so, n, tb, st, se, rows_name);
     } else {
-      if (cols) launch_fwd_cols<L1S, kNttThreads>(c, sa, so, n, tb, st);
+      if (cols) launch_fwd_cols<L1S, kNttThreads>(c, sa, so, n, tb, st, sp);
       launch_fwd_rows<L2S, kNttThreads>(c, so, n, tb, st, se, rows_name);
     }
   }
@@ -1354,15 +1471,16 @@ void inv_impl(const Context& c, const Addr& ad, const AddrOut& ao, uint32_t nlim
   cs.join();
 }
 
-template <class Addr, class AddrOut, class Epi = EpiStore>
+template <class Addr, class AddrOut, class Epi = EpiStore, class Pro = ProLoad>
 void dispatch(const Context& c, const Addr& ad, const AddrOut& ao, uint32_t nlimbs, hipStream_t st, bool fwd, const Epi& epi = Epi{},
-              const char* rows_name = "ntt_fwd_rows", bool cols = true) {
+              const char* rows_name = "ntt_fwd_rows", bool cols = true,
+              const Pro& pro = Pro{}) {
   if (nlimbs == 0) return;
   const int l1 = c.tune.ntt_split ? c.tune.ntt_split : ntt_default_split(c.logN);
   // (logN, l1) pairs accepted by ntt_split_ok; the default split of each logN also has wide tiles
 #define FH_NTT_CASE(LN, A, WIDE)                                                                     \
   case LN * 16 + A:                                                                                  \
-    if (fwd) fwd_impl<Addr, AddrOut, A, LN - A, WIDE, Epi>(c, ad, ao, nlimbs, st, epi, rows_name, cols); \
+    if (fwd) fwd_impl<Addr, AddrOut, A, LN - A, WIDE, Epi, Pro>(c, ad, ao, nlimbs, st, epi, rows_name, cols, pro); \
     else inv_impl<Addr, AddrOut, A, LN - A, WIDE>(c, ad, ao, nlimbs, st);                            \
     break;
   switch (c.logN * 16 + l1) {

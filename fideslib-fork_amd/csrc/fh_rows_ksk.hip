@@ -121,8 +121,8 @@ void modup_cols(const Context& c, const ModUpAddr& m, uint32_t n, hipStream_t st
   for (uint32_t base = 0; base < n; base += 65535) {
     const uint32_t cnt = std::min<uint32_t>(65535, n - base);
     const Shift<ModUpAddr> sa{m, base};
-    if (WIDE && c.tune.ntt_threads[0] == kNttWide) launch_fwd_cols<L1S, kNttWide>(c, sa, sa, cnt, tb, st);
-    else launch_fwd_cols<L1S, kNttThreads>(c, sa, sa, cnt, tb, st);
+    if (WIDE && c.tune.ntt_threads[0] == kNttWide) launch_fwd_cols<L1S, kNttWide>(c, sa, sa, cnt, tb, st, ProLoad{});
+    else launch_fwd_cols<L1S, kNttThreads>(c, sa, sa, cnt, tb, st, ProLoad{});
   }
 }
 
