@@ -159,8 +159,14 @@ void encode_slots(Context& c, const double* values, int count, uint32_t slots, d
   // this encoder rounds exactly, so it rejects every input that could reach 2^61: |re| + |im| times
   // the scale must stay below 2^61 (1 - 2^-40). One comparison per value also rejects NaN and infinity.
   const double lim = 0x1p61 * (1.0 - 0x1p-40) / scale;
-  bool bad = false;
-  for (size_t i = 0; i < (size_t)count * slots; ++i) bad |= !(std::fabs(values[2 * i]) + std::fabs(values[2 * i + 1]) < lim);
+  // four independent lanes: one flag would chain every comparison to the one before
+  uint64_t flags[4] = {0, 0, 0, 0};
+  const size_t nv = (size_t)count * slots;
+  size_t at = 0;
+  for (; at + 4 <= nv; at += 4)
+    for (int u = 0; u < 4; ++u) flags[u] |= !(std::fabs(values[2 * (at + u)]) + std::fabs(values[2 * (at + u) + 1]) < lim);
+  for (; at < nv; ++at) flags[0] |= !(std::fabs(values[2 * at]) + std::fabs(values[2 * at + 1]) < lim);
+  const bool bad = flags[0] | flags[1] | flags[2] | flags[3];
   if (bad) throw Error(-1, "encode: a slot value is not finite, or times the scale it reaches 2^61 (OpenFHE's MAX_BITS_IN_WORD)");
   ensure_ifft_tables(c);
   const uint32_t n = slots;

@@ -302,27 +302,42 @@ struct OpaqueTid {
 // (ProLoad) or forms it from what it comes from: the Rescale correction from the dropped limb, a
 // raised limb from tower 0, an encoded limb from the integer coefficients. The limb's values are
 // then neither written by a launch of their own nor read back. Job y as in the epilogues.
+// get: the value at position n in the limb's arithmetic, canonical or, for fp64, within q.
 struct ProLoad {
-  __device__ __forceinline__ void init(uint32_t, uint32_t, const PrimeConst*) {}
-  __device__ __forceinline__ uint64_t value(const uint64_t* p, uint32_t n) const { return p[n]; }
+  __device__ __forceinline__ void init(uint32_t, uint32_t, const PrimeConst*, int) {}
+  template <class A>
+  __device__ __forceinline__ typename A::T get(const A& ar, const uint64_t* p, uint32_t n) const { return ar.from_canon(p[n]); }
 };
 
 // e_i = SwitchModulus_{q_l -> q_i}(top) * QlQl[l][i] (OpenFHE NativeVector::SwitchModulus: values above
-// q_l / 2 shift by the difference of the moduli; the product takes the word unreduced)
+// q_l / 2 shift by the difference of the moduli; the product takes the word unreduced). Between two
+// fp64 primes the centred value and one fp64 product: 13 instructions instead of 35.
 struct SwitchMod {
   const uint64_t* t;
   uint64_t half, diff, qi, f, fsh;
-  __device__ __forceinline__ void set(const uint64_t* top, uint64_t ql, uint64_t q, uint64_t w, uint64_t wsh) {
+  double qld, fd;   // q_l and the factor, centred, as doubles
+  bool fp;
+  __device__ __forceinline__ void set(const uint64_t* top, const PrimeConst& l, const PrimeConst& i, uint64_t w, uint64_t wsh) {
     t = top;
-    half = ql >> 1;
-    diff = ql > q ? q - (ql % q) : q - ql;
-    qi = q;
+    qi = i.q;
+    half = l.q >> 1;
+    diff = l.q > qi ? qi - barrett128(0, l.q, i) : qi - l.q;
     f = w;
     fsh = wsh;
+    fp = l.fp64 && l.q < 4 * qi;
+    qld = l.qd;
+    fd = w > qi / 2 ? (double)w - i.qd : (double)w;
   }
-  __device__ __forceinline__ uint64_t at(uint32_t n) const {
+  template <class A>
+  __device__ __forceinline__ typename A::T at(const A& ar, uint32_t n) const {
     const uint64_t v = t[n];
-    return shoup(v > half ? v + diff : v, f, fsh, qi);
+    if constexpr (std::is_same_v<A, FpA>) {
+      if (fp) {
+        const double x = (double)v;
+        return ar.mul(v > half ? x - qld : x, fd);
+      }
+    }
+    return ar.from_canon(shoup(v > half ? v + diff : v, f, fsh, qi));
   }
 };
 
@@ -332,11 +347,12 @@ struct ProRescale {
   const uint64_t* wsh;
   uint32_t l, npolys;
   SwitchMod s;
-  __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime) {
+  __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime, int) {
     const uint32_t i = y / npolys, b = y % npolys;
-    s.set(top + (size_t)b * N, prime[l].q, prime[i].q, w[i], wsh[i]);
+    s.set(top + (size_t)b * N, prime[l], prime[i], w[i], wsh[i]);
   }
-  __device__ __forceinline__ uint64_t value(const uint64_t*, uint32_t n) const { return s.at(n); }
+  template <class A>
+  __device__ __forceinline__ typename A::T get(const A& ar, const uint64_t*, uint32_t n) const { return s.at(ar, n); }
 };
 
 // limb i of component b raised from tower 0 (centred lift modulo q_0)
@@ -347,36 +363,41 @@ struct ProModRaise {
   uint64_t half, diff;
   uint32_t i;
   PrimeConst P;
-  __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime) {
+  __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime, int) {
     i = y / npolys;
     t = x0 + (size_t)(y % npolys) * N;
     P = prime[i];
     const uint64_t q0 = prime[0].q;
     half = q0 >> 1;
-    diff = q0 > P.q ? P.q - (q0 % P.q) : P.q - q0;
+    diff = q0 > P.q ? P.q - barrett128(0, q0, P) : P.q - q0;
   }
-  __device__ __forceinline__ uint64_t value(const uint64_t*, uint32_t n) const {
+  template <class A>
+  __device__ __forceinline__ typename A::T get(const A& ar, const uint64_t*, uint32_t n) const {
     const uint64_t v = t[n];
-    return i == 0 ? v : barrett128(0, v > half ? v + diff : v, P);
+    return ar.from_canon(i == 0 ? v : barrett128(0, v > half ? v + diff : v, P));
   }
 };
 
-// residues of signed integer coefficients: plaintext y % npolys of N coefficients, limb y / npolys
+// residues of signed integer coefficients: plaintext y % npolys of N coefficients.
+// fp64 primes above 2^34: the high half's product by 2^32 and the low half, 10 instructions; others
+// through a Barrett quotient (about 45).
 struct ProSigned {
   const int64_t* m;
-  LimbSet s;
+  uint32_t npolys;
   const int64_t* t;
   PrimeConst P;
-  __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime) {
-    t = m + (size_t)(y % s.npolys) * N;
-    P = prime[s.pid[y / s.npolys]];
+  __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime, int pid) {
+    t = m + (size_t)(y % npolys) * N;
+    P = prime[pid];
   }
-  __device__ __forceinline__ uint64_t value(const uint64_t*, uint32_t n) const {
+  template <class A>
+  __device__ __forceinline__ typename A::T get(const A& ar, const uint64_t*, uint32_t n) const {
     const int64_t v = t[n];
-    if (v >= 0) return barrett128(0, (uint64_t)v, P);
-    uint64_t r = barrett128(0, (uint64_t)(-(v + 1)), P) + 1;
-    if (r == P.q) r = 0;
-    return r ? P.q - r : 0;
+    if constexpr (std::is_same_v<A, FpA>) {
+      if (P.q >> 34) return ar.mul((double)(int32_t)(v >> 32), 4294967296.0) + (double)(uint32_t)v;
+    }
+    const uint64_t r = barrett128(0, v < 0 ? 0 - (uint64_t)v : (uint64_t)v, P);
+    return ar.from_canon(v < 0 && r ? P.q - r : r);
   }
 };
 
@@ -428,7 +449,7 @@ __device__ __forceinline__ void fwd_cols_body(const A& ar, const TwT* tw, const 
   typename A::T x[16];
   stage_tw(ar, sw, swp, tw, twsh, S);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) x[k] = ar.from_canon(pro.value(p, (r0 + T * k) * N2 + col));
+  for (int k = 0; k < 16; ++k) x[k] = pro.get(ar, p, (r0 + T * k) * N2 + col);
   __syncthreads();
   int b[16];
 #pragma unroll
@@ -459,7 +480,7 @@ __global__ __launch_bounds__(TH) void k_ntt_fwd_cols(Addr ad, AddrOut ao, NttTab
   int pid, pido;
   ad.at(blockIdx.y, tb.N, p, pid);
   ao.at(blockIdx.y, tb.N, po, pido);
-  pro.init(blockIdx.y, tb.N, tb.prime);
+  pro.init(blockIdx.y, tb.N, tb.prime, pid);
   const Sel sel = select(tb, pid, false);
   const int C = blockDim.x / T;
   const uint32_t N2 = tb.N >> LS;
@@ -1052,7 +1073,7 @@ __global__ __launch_bounds__(TH) __attribute__((amdgpu_waves_per_eu(3))) void k_
     ad.at(y, tb.N, p, pid);
     ao.at(y, tb.N, po, pido);
     Pro pr = pro;
-    pr.init(y, tb.N, tb.prime);
+    pr.init(y, tb.N, tb.prime, pid);
     const Sel sel = select(tb, pid, false);
     __syncthreads();   // earlier readers of sw / tile are done
     team_arith<FP>(sel, [&](const auto& ar, const auto* tw, const auto* twsh) {
@@ -1239,20 +1260,22 @@ struct ProRescaleJobs {
   const uint64_t* wsh;
   uint32_t L1;
   SwitchMod s;
-  __device__ __forceinline__ void init(uint32_t y, uint32_t, const PrimeConst* prime) {
+  __device__ __forceinline__ void init(uint32_t y, uint32_t, const PrimeConst* prime, int) {
     const EpiJob j = jobs[y];
     const size_t o = (size_t)j.l * L1 + j.pid;
-    s.set(as_global(j.top), prime[j.l].q, prime[j.pid].q, w[o], wsh[o]);
+    s.set(as_global(j.top), prime[j.l], prime[j.pid], w[o], wsh[o]);
   }
-  __device__ __forceinline__ uint64_t value(const uint64_t*, uint32_t n) const { return s.at(n); }
+  template <class A>
+  __device__ __forceinline__ typename A::T get(const A& ar, const uint64_t*, uint32_t n) const { return s.at(ar, n); }
 };
 
 template <class Pro>
 struct ShiftPro {
   Pro p;
   uint32_t base;
-  __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime) { p.init(y + base, N, prime); }
-  __device__ __forceinline__ uint64_t value(const uint64_t* x, uint32_t n) const { return p.value(x, n); }
+  __device__ __forceinline__ void init(uint32_t y, uint32_t N, const PrimeConst* prime, int pid) { p.init(y + base, N, prime, pid); }
+  template <class A>
+  __device__ __forceinline__ typename A::T get(const A& ar, const uint64_t* x, uint32_t n) const { return p.get(ar, x, n); }
 };
 
 template <class Epi>

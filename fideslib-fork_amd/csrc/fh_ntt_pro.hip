@@ -21,7 +21,7 @@ void ntt_fwd_mod_raise(const Context& c, const uint64_t* x0, const LimbSet& out,
 void ntt_fwd_signed(const Context& c, const int64_t* m, const LimbSet& out, hipStream_t st) {
   ProSigned pr{};
   pr.m = m;
-  pr.s = out;
+  pr.npolys = out.npolys;
   dispatch(c, SetAddr{out}, SetAddr{out}, out.nlimbs * out.npolys, st, true, EpiStore{}, "ntt_fwd_rows", true, pr);
 }
 

@@ -251,7 +251,7 @@ class Context:
         v = np.asarray(values, dtype=np.complex128)
         if v.ndim == 1:
             v = v[None, :]
-        flat = np.ascontiguousarray(np.stack([v.real, v.imag], axis=-1).reshape(-1))
+        flat = np.ascontiguousarray(v)  # interleaved re, im
         _check(load().fh_encode_slots(self.h, flat.ctypes.data, v.shape[0], v.shape[1], float(scale), _i32(list(prime_ids)), len(prime_ids),
                                       out.ptr, out_stride))
 
