@@ -232,7 +232,6 @@ __global__ __launch_bounds__(kT) void k_ksk_inner(const uint64_t* __restrict__ d
 // (the dominant HBM stream of a rotation) is read once per group instead of once per ciphertext.
 constexpr int kMaxGroups = 64;
 constexpr int kMaxBatch = 256;
-constexpr int kMaxDnum = 8;
 
 struct RotGroups {
   const uint64_t* key[kMaxGroups];

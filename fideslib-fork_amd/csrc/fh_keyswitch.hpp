@@ -6,6 +6,8 @@
 
 namespace fh {
 
+constexpr int kMaxDnum = 8;   // digits the key inner products take
+
 // Conversion jobs of a mixed-level batch (device tables).
 struct ModUpJob {
   const uint64_t* coef;   // INTT of the key-switched polynomial (l+1 limbs)

@@ -8,6 +8,7 @@
 // LTdotProductPtBatch (src/CKKS/LimbPartitionBatch.cu:266-524), Ciphertext::extend
 // (src/CKKS/Ciphertext.cpp:1087-1100), contract api/CryptoContext.hpp:460-517.
 #include <algorithm>
+#include <type_traits>
 
 #include "fh_keyswitch.hpp"
 
@@ -18,46 +19,117 @@ namespace {
 constexpr int kT = 256;
 constexpr int kMaxBaby = 16;
 
-// out[comp][pos] = [P]_{q_pos} x[comp][pos] for Q limbs, 0 for the special limbs (the P-scaled
-// extended form of a ciphertext over Q_l).
-__global__ __launch_bounds__(kT) void k_extend_p(const uint64_t* __restrict__ x, uint64_t* __restrict__ out, uint32_t N, uint32_t lq,
-                                                  uint32_t ext, const PrimeConst* prime, const uint64_t* pmod, const uint64_t* pmod_sh) {
-  const uint32_t comp = blockIdx.y / ext, pos = blockIdx.y % ext;
-  uint64_t* o = out + ((size_t)comp * ext + pos) * N;
-  if (pos >= lq) {
-    for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < N; n += gridDim.x * blockDim.x) o[n] = 0;
-    return;
+// One group of rotations whose results are consumed where they are formed. Source t holds its
+// switched polynomial (EVAL, lq limbs) at own + t * own_stride, the other limbs of its digits at
+// dig + t * dig_stride ([beta][ext][N]) and its c0 at c0 + t * c0_stride.
+struct Hoist {
+  uint32_t N, lq, ext, L1, E, beta, alpha, logN;   // E = L1 + K limbs of a key polynomial
+  const PrimeConst* prime;
+  const uint64_t* pmod;
+  const uint64_t* pmod_sh;
+  const uint64_t* dig;
+  const uint64_t* own;
+  const uint64_t* c0;
+  uint64_t dig_stride, own_stride, c0_stride;
+  int c0_ext;                     // 1: c0 is given over Q_l ∪ P; 0: over Q_l, folded as P c0
+  const uint64_t* key[kMaxBaby];  // [dnum][2][E][N], Montgomery form; null: no rotation (P c0, P c1)
+  uint32_t gal[kMaxBaby];
+};
+
+// The limb a workgroup works on
+struct HoistLimb {
+  uint32_t pos, p, own_d;
+  uint64_t pm, pmsh;
+  PrimeConst P;
+  __device__ __forceinline__ HoistLimb(const Hoist& h, uint32_t pos_) : pos(pos_) {
+    const bool isq = pos < h.lq;
+    p = isq ? pos : h.L1 + (pos - h.lq);
+    own_d = isq ? pos / h.alpha : ~0u;
+    pm = isq ? h.pmod[pos] : 0;
+    pmsh = isq ? h.pmod_sh[pos] : 0;
+    P = h.prime[p];
   }
-  const uint64_t q = prime[pos].q, w = pmod[pos], wsh = pmod_sh[pos];
-  const uint64_t* xi = x + ((size_t)comp * lq + pos) * N;
-  for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < N; n += gridDim.x * blockDim.x) o[n] = shoup(xi[n], w, wsh, q);
+};
+
+// Word n of both components of source t rotated by (key, gal), over Q_l ∪ P: the key inner product
+// and c0 at the word that the automorphism brings to n. In the bit-reversed order of the transforms
+// an automorphism takes every aligned block of 2^k words to an aligned block, so the 64 words that
+// a wave gathers fill whole cache lines. Every load is issued before the first product.
+// DM bounds the digits. Memory-bound: the keys are read once; writing the rotations and reading them
+// back was a third of the traffic. N = 2^16, 50-bit primes, three digits, against key product, sum
+// and extension in launches of their own: the radix-4 fold of 256 slots 1325 -> 1022 us, 63 diagonals
+// in 16 baby steps 1495 -> 1320 us.
+template <class M, int DM>
+__device__ __forceinline__ void hoist_rot(const Hoist& h, const HoistLimb& L, const uint64_t* key, uint32_t gal, uint32_t t, uint32_t n,
+                                          uint64_t& r0, uint64_t& r1) {
+  const size_t N = h.N;
+  const uint32_t s = gal != 1 ? auto_src(n, gal, h.logN) : n;
+  const uint64_t* dg = h.dig + t * h.dig_stride + L.pos * N;
+  const uint64_t* ow = h.own + t * h.own_stride + L.pos * N;
+  const uint64_t* kp = key + L.p * N;
+  uint64_t x[DM], kb[DM], ka[DM], c = 0;
+#pragma unroll
+  for (int d = 0; d < DM; ++d) {
+    x[d] = kb[d] = ka[d] = 0;
+    if (d < (int)h.beta) {
+      x[d] = (d == (int)L.own_d ? ow : dg + (size_t)d * h.ext * N)[s];
+      kb[d] = kp[(size_t)(2 * d) * h.E * N + s];
+      ka[d] = kp[(size_t)(2 * d + 1) * h.E * N + s];
+    }
+  }
+  if (h.c0_ext || L.pos < h.lq) c = h.c0[t * h.c0_stride + L.pos * N + s];
+  M a0, a1;
+  a0.zero();
+  a1.zero();
+#pragma unroll
+  for (int d = 0; d < DM; ++d)
+    if (d < (int)h.beta) {
+      const auto xd = M::prep(x[d]);
+      a0.mac(xd, M::prep(kb[d]));
+      a1.mac(xd, M::prep(ka[d]));
+    }
+  uint64_t hi, lo;
+  a0.get(hi, lo);
+  r0 = redc(hi, lo, L.P);  // keys are in Montgomery form
+  a1.get(hi, lo);
+  r1 = redc(hi, lo, L.P);
+  r0 = add_mod(r0, h.c0_ext ? c : shoup(c, L.pm, L.pmsh, L.P.q), L.P.q);
+}
+
+// The same for a rotation by nothing: P times source t, zero on the special limbs.
+__device__ __forceinline__ void hoist_ident(const Hoist& h, const HoistLimb& L, uint32_t t, uint32_t n, uint64_t& r0, uint64_t& r1) {
+  r0 = r1 = 0;
+  if (L.pos < h.lq) {
+    r0 = shoup(h.c0[t * h.c0_stride + (size_t)L.pos * h.N + n], L.pm, L.pmsh, L.P.q);
+    r1 = shoup(h.own[t * h.own_stride + (size_t)L.pos * h.N + n], L.pm, L.pmsh, L.P.q);
+  }
 }
 
 struct MacParams {
-  uint32_t N, lq, ext, L1, rowSize, bStep, gStep;
-  const PrimeConst* prime;
+  uint32_t rowSize, bStep, gStep;
   uint32_t i0 = 0;   // first baby step of this launch (a launch covers baby steps i0 .. i0 + BB - 1)
   uint32_t acc = 0;  // 1: add into R (a later launch over the next baby steps)
 };
 
-// R[j][comp][pos] = sum_{i: bStep j + i < rowSize} fast[i][comp][pos] (.) diag[bStep j + i][pos]
-// One lane holds the bStep baby-step words of both components for its (position, coefficient)
+// R[j][comp][pos] = sum_{i: bStep j + i < rowSize} rot_i[comp][pos] (.) diag[bStep j + i][pos]
+// One lane forms the bStep rotated words of both components for its (position, coefficient)
 // and streams the diagonals once; each sum (at most 16 products) is accumulated exactly under the
-// multiply policy M and reduced once.
-template <int BB, class M>
-__global__ __launch_bounds__(kT) void k_lt_mac(const uint64_t* __restrict__ fast, const uint64_t* __restrict__ diags,
-                                                uint64_t* __restrict__ R, MacParams mp) {
+// multiply policy M and reduced once. The rotations never reach memory.
+template <int BB, class M, int DM>
+__global__ __launch_bounds__(kT) void k_lt_mac(Hoist h, const uint64_t* __restrict__ diags, uint64_t* __restrict__ R, MacParams mp) {
   using Op = typename M::Op;
-  const uint32_t pos = blockIdx.y;
-  const PrimeConst P = mp.prime[pos < mp.lq ? pos : mp.L1 + (pos - mp.lq)];
-  const size_t N = mp.N, E = (size_t)mp.ext * N;
-  for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < mp.N; n += gridDim.x * blockDim.x) {
+  const HoistLimb L(h, blockIdx.y);
+  const size_t N = h.N, E = (size_t)h.ext * N;
+  for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < h.N; n += gridDim.x * blockDim.x) {
     Op f0[BB], f1[BB];
 #pragma unroll
     for (int i = 0; i < BB; ++i) {
       if (mp.i0 + i < mp.bStep) {
-        f0[i] = M::prep(fast[((size_t)(mp.i0 + i) * 2 + 0) * E + (size_t)pos * N + n]);
-        f1[i] = M::prep(fast[((size_t)(mp.i0 + i) * 2 + 1) * E + (size_t)pos * N + n]);
+        uint64_t r0, r1;
+        if (h.key[i]) hoist_rot<M, DM>(h, L, h.key[i], h.gal[i], 0, n, r0, r1);
+        else hoist_ident(h, L, 0, n, r0, r1);
+        f0[i] = M::prep(r0);
+        f1[i] = M::prep(r1);
       }
     }
     for (uint32_t j = 0; j < mp.gStep; ++j) {
@@ -68,49 +140,102 @@ __global__ __launch_bounds__(kT) void k_lt_mac(const uint64_t* __restrict__ fast
       for (int i = 0; i < BB; ++i) {
         const uint32_t k = j * mp.bStep + mp.i0 + i;
         if (mp.i0 + i < mp.bStep && k < mp.rowSize) {
-          const Op d = M::prep(diags[(size_t)k * E + (size_t)pos * N + n]);
+          const Op d = M::prep(diags[(size_t)k * E + (size_t)L.pos * N + n]);
           a0.mac(f0[i], d);
           a1.mac(f1[i], d);
         }
       }
       uint64_t hi, lo;
-      uint64_t* r0 = R + ((size_t)j * 2 + 0) * E + (size_t)pos * N + n;
-      uint64_t* r1 = R + ((size_t)j * 2 + 1) * E + (size_t)pos * N + n;
+      uint64_t* r0 = R + ((size_t)j * 2 + 0) * E + (size_t)L.pos * N + n;
+      uint64_t* r1 = R + ((size_t)j * 2 + 1) * E + (size_t)L.pos * N + n;
       a0.get(hi, lo);
-      const uint64_t v0 = mod128(hi, lo, P);
+      const uint64_t v0 = mod128(hi, lo, L.P);
       a1.get(hi, lo);
-      const uint64_t v1 = mod128(hi, lo, P);
-      *r0 = mp.acc ? add_mod(*r0, v0, P.q) : v0;
-      *r1 = mp.acc ? add_mod(*r1, v1, P.q) : v1;
+      const uint64_t v1 = mod128(hi, lo, L.P);
+      *r0 = mp.acc ? add_mod(*r0, v0, L.P.q) : v0;
+      *r1 = mp.acc ? add_mod(*r1, v1, L.P.q) : v1;
     }
   }
 }
 
 inline dim3 grid_n(uint32_t N, uint32_t y) { return dim3(std::max(1u, std::min((N + kT - 1) / kT, 256u)), y); }
 
-// acc += sum_{t < nt} T[t] over the extended basis of both components (acc: the LimbSet's two
-// polynomials; T[t] at T + t * t_stride in the same layout): one read of each summand and one
-// read-modify-write of acc instead of nt separate additions. blockIdx.y = (comp, pos).
-__global__ __launch_bounds__(kT) void k_lt_sum(LimbSet acc, const uint64_t* __restrict__ T, uint64_t t_stride, int nt, uint32_t N,
-                                              const PrimeConst* prime) {
-  const uint32_t comp = blockIdx.y / acc.nlimbs, pos = blockIdx.y % acc.nlimbs;
-  const uint64_t q = prime[acc.pid[pos]].q;
-  const size_t off = (size_t)comp * acc.poly_stride + (size_t)pos * N;
-  uint64_t* a = acc.base + off;
-  for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < N; n += gridDim.x * blockDim.x) {
-    uint64_t s = a[n];
-    for (int t = 0; t < nt; ++t) s = add_mod(s, T[t * t_stride + off + n], q);
-    a[n] = s;
+// base + sum of n rotations, over the extended basis of both components, written to out ([2][ext][N]).
+// base: 0 P times the source, 1 what out holds, 2 the extended c0 of the source and P times its c1.
+// per_item: rotation t reads source t (base 1 only), else all read source 0. blockIdx.y = pos.
+template <class M, int DM>
+__global__ __launch_bounds__(kT) void k_hoist_sum(Hoist h, int n_rot, int base, int per_item, uint64_t* __restrict__ out) {
+  const HoistLimb L(h, blockIdx.y);
+  uint64_t* o0 = out + (size_t)L.pos * h.N;
+  uint64_t* o1 = o0 + (size_t)h.ext * h.N;
+  for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < h.N; n += gridDim.x * blockDim.x) {
+    uint64_t s0 = 0, s1 = 0;
+    if (base == 1) {
+      s0 = o0[n];
+      s1 = o1[n];
+    } else {
+      if (L.pos < h.lq) s1 = shoup(h.own[(size_t)L.pos * h.N + n], L.pm, L.pmsh, L.P.q);
+      if (base == 2 || L.pos < h.lq) s0 = h.c0[(size_t)L.pos * h.N + n];
+      if (base == 0) s0 = shoup(s0, L.pm, L.pmsh, L.P.q);
+    }
+    for (int t = 0; t < n_rot; ++t) {
+      uint64_t r0, r1;
+      hoist_rot<M, DM>(h, L, as_global(h.key[t]), h.gal[t], per_item ? t : 0, n, r0, r1);
+      s0 = add_mod(s0, r0, L.P.q);
+      s1 = add_mod(s1, r1, L.P.q);
+    }
+    o0[n] = s0;
+    o1[n] = s1;
   }
 }
 
-void lt_sum(Context& c, const LimbSet& acc, const uint64_t* T, uint64_t t_stride, int nt, hipStream_t st) {
-  ProfScope ps_(c, "lt_sum", st);
-  k_lt_sum<<<grid_n(c.N, 2 * acc.nlimbs), kT, 0, st>>>(acc, T, t_stride, nt, c.N, c.d_prime);
-  FH_HIP(hipGetLastError());
+// The parameters that every rotation of a group shares.
+Hoist hoist_group(const Context& c, int l, const uint64_t* dig, uint64_t dig_stride, const uint64_t* own, uint64_t own_stride,
+                  const uint64_t* c0, uint64_t c0_stride, bool c0_ext) {
+  const uint32_t lq = l + 1, beta = c.num_digits(l);
+  return Hoist{c.N, lq, lq + c.K, (uint32_t)c.L1, (uint32_t)(c.L1 + c.K), beta, (uint32_t)c.alpha, (uint32_t)c.logN, c.d_prime, c.d_pmod,
+               c.d_pmod_sh, dig, own, c0, dig_stride, own_stride, c0_stride, c0_ext ? 1 : 0, {}, {}};
 }
 
-// k_extend_p for B ciphertexts: blockIdx.y = (b, comp, pos)
+void hoist_check(const Context& c, const Hoist& h, const uint64_t* key, uint32_t gal) {
+  if (h.beta > (uint32_t)kMaxDnum) throw Error(-3, "dnum above kernel limit");
+  if (!key) throw Error(-1, "null key");
+  if ((gal & 1) == 0 || gal >= 2 * c.N) throw Error(-1, "galois index must be odd and < 2N");
+}
+
+// f(M, DM): the kernel for this context's multiply policy and this level's digits
+template <class F>
+void with_hoist(const Context& c, uint32_t beta, F f) {
+  if (c.split_mac_ok) beta <= 4 ? f(Mac30{}, std::integral_constant<int, 4>{}) : f(Mac30{}, std::integral_constant<int, kMaxDnum>{});
+  else beta <= 4 ? f(MacWide{}, std::integral_constant<int, 4>{}) : f(MacWide{}, std::integral_constant<int, kMaxDnum>{});
+}
+
+// out = base + the n rotations of the group (base, per_item: as in k_hoist_sum), in launches of at most
+// kMaxBaby rotations, the later ones adding to out. out is none of the group's sources.
+void hoist_sum(Context& c, Hoist h, int n, const uint64_t* const* keys, const uint32_t* gals, int base, bool per_item, uint64_t* out,
+               hipStream_t st) {
+  for (int t = 0; t < n; ++t) hoist_check(c, h, keys[t], gals[t]);
+  ProfScope ps_(c, "hoist_sum", st);
+  for (int t0 = 0; t0 < n; t0 += kMaxBaby, base = 1) {
+    const int nt = std::min(n - t0, kMaxBaby);
+    for (int t = 0; t < nt; ++t) {
+      h.key[t] = keys[t0 + t];
+      h.gal[t] = gals[t0 + t];
+    }
+    with_hoist(c, h.beta, [&](auto m, auto dm) {
+      k_hoist_sum<decltype(m), decltype(dm)::value><<<grid_n(c.N, h.ext), kT, 0, st>>>(h, nt, base, per_item ? 1 : 0, out);
+    });
+    FH_HIP(hipGetLastError());
+    if (per_item) {
+      h.dig += nt * h.dig_stride;
+      h.own += nt * h.own_stride;
+      h.c0 += nt * h.c0_stride;
+    }
+  }
+}
+
+// [P]_{q_pos} x for Q limbs, 0 for the special limbs (the P-scaled extended form of ciphertexts over
+// Q_l): blockIdx.y = (b, comp, pos)
 __global__ __launch_bounds__(kT) void k_extend_p_b(const uint64_t* __restrict__ x, uint64_t x_stride, uint64_t* __restrict__ out,
                                                     uint64_t out_stride, uint32_t N, uint32_t lq, uint32_t ext, const PrimeConst* prime,
                                                     const uint64_t* pmod, const uint64_t* pmod_sh) {
@@ -135,7 +260,10 @@ struct MacBatchParams {
   int8_t slot[kMaxBaby];   // baby step i: rotation slot (>= 0) or the P-scaled identity (-1)
 };
 
-// Giant-step partial sums for B ciphertexts sharing one diagonal set. blockIdx.y = extended
+// Giant-step partial sums for B ciphertexts sharing one diagonal set, from the rotations that
+// k_ksk_batch wrote. Forming them here, as k_lt_mac does, was measured slower for a batch: 16
+// ciphertexts, N = 2^16, 30 limbs, 8 x 8 steps, 20.5 against 16.7 ms for the transform. There the key
+// product reads its keys once for the whole batch, here once per ciphertext and wave. blockIdx.y = extended
 // position, blockIdx.x = a 64-coefficient tile: the tile of every diagonal is staged in LDS once
 // (as multiply operands, split into 30-bit halves under Mac30) and applied to all B ciphertexts
 // (four ciphertexts in flight per workgroup), so the diagonals are read once per batch.
@@ -188,64 +316,56 @@ __global__ __launch_bounds__(kT) void k_lt_mac_b(const uint64_t* __restrict__ ro
   }
 }
 
-}  // namespace
+// The keys of the baby steps i0 .. i0 + n - 1 (null for a rotation by nothing). Returns whether one of them rotates.
+bool hoist_baby(const Context& c, Hoist& h, int i0, int n, int stride, int slots, const uint64_t* const* baby_keys,
+                const uint32_t* baby_gal) {
+  bool any = false;
+  for (int i = 0; i < n; ++i) {
+    h.key[i] = nullptr;
+    if (((long long)(i0 + i) * stride) % slots == 0) continue;
+    if (!baby_keys[i0 + i]) throw Error(-1, "baby-step key missing");
+    hoist_check(c, h, baby_keys[i0 + i], baby_gal[i0 + i]);
+    h.key[i] = baby_keys[i0 + i];
+    h.gal[i] = baby_gal[i0 + i];
+    any = true;
+  }
+  return any;
+}
 
-namespace {
-
-// Baby steps (the identity in P-scaled extended form, the others from one shared ModUp) and the
-// multiply-accumulate of every giant-step partial sum: R_j, 2 x (l+1+K) limbs each, j < gStep.
+// Every giant-step partial sum from the baby steps, which share one ModUp: R_j, 2 x (l+1+K) limbs
+// each, j < gStep.
 DBuf lt_partials(Context& c, const uint64_t* ct, int l, int rowSize, int bStep, int stride, int slots, const uint64_t* diags,
                  const uint64_t* const* baby_keys, const uint32_t* baby_gal, hipStream_t st) {
-  const uint32_t lq = l + 1, ext = lq + c.K;
+  const uint32_t lq = l + 1, ext = lq + c.K, beta = c.num_digits(l);
   const size_t E = (size_t)ext * c.N;
+  const uint64_t* c1 = ct + (size_t)lq * c.N;
   const int gStep = (rowSize + bStep - 1) / bStep;
-  DBuf fast(c.pool, (size_t)bStep * 2 * E);
-  std::vector<int> rot_idx;
-  std::vector<const uint64_t*> rk;
-  std::vector<uint32_t> rg;
-  for (int i = 0; i < bStep; ++i) {
-    if (((long long)i * stride) % slots == 0) {
-      ProfScope ps_(c, "lt_extend", st);
-      k_extend_p<<<grid_n(c.N, 2 * ext), kT, 0, st>>>(ct, fast.p + (size_t)i * 2 * E, c.N, lq, ext, c.d_prime, c.d_pmod, c.d_pmod_sh);
-      FH_HIP(hipGetLastError());
-    } else {
-      if (!baby_keys[i]) throw Error(-1, "baby-step key missing");
-      rot_idx.push_back(i);
-      rk.push_back(baby_keys[i]);
-      rg.push_back(baby_gal[i]);
-    }
+  DBuf dig, R(c.pool, (size_t)gStep * 2 * E);
+  Hoist h = hoist_group(c, l, nullptr, 0, c1, 0, ct, 0, false);
+  if (hoist_baby(c, h, 0, bStep, stride, slots, baby_keys, baby_gal)) {
+    dig = DBuf(c.pool, (size_t)beta * E);
+    h.dig = dig.p;
+    modup_batch(c, c1, l, 1, 0, dig.p, st, false);
   }
-  if (!rot_idx.empty()) {
-    bool contiguous = true;
-    for (size_t t = 1; t < rot_idx.size(); ++t) contiguous &= rot_idx[t] == rot_idx[t - 1] + 1;
-    if (contiguous) {
-      rotate_hoisted(c, ct, l, (int)rot_idx.size(), rk.data(), rg.data(), true, false, fast.p + (size_t)rot_idx[0] * 2 * E, st);
-    } else {
-      DBuf tmp(c.pool, rot_idx.size() * 2 * E);
-      rotate_hoisted(c, ct, l, (int)rot_idx.size(), rk.data(), rg.data(), true, false, tmp.p, st);
-      for (size_t t = 0; t < rot_idx.size(); ++t)
-        FH_HIP(hipMemcpyAsync(fast.p + (size_t)rot_idx[t] * 2 * E, tmp.p + t * 2 * E, 2 * E * 8, hipMemcpyDeviceToDevice, st));
+  MacParams mp{(uint32_t)rowSize, (uint32_t)bStep, (uint32_t)gStep};
+  ProfScope ps_(c, "lt_mac", st);
+  const dim3 g = grid_n(c.N, ext);
+  with_hoist(c, beta, [&](auto m, auto dm) {
+    using M = decltype(m);
+    constexpr int DM = decltype(dm)::value;
+    if (bStep <= 4) {
+      k_lt_mac<4, M, DM><<<g, kT, 0, st>>>(h, diags, R.p, mp);
+      return;
     }
-  }
-  DBuf R(c.pool, (size_t)gStep * 2 * E);
-  MacParams mp{c.N, lq, ext, (uint32_t)c.L1, (uint32_t)rowSize, (uint32_t)bStep, (uint32_t)gStep, c.d_prime};
-  {
-    ProfScope ps_(c, "lt_mac", st);
-    const dim3 g = grid_n(c.N, ext);
     // more than 8 baby steps: launches of 8 each, the later ones adding into R (the sums are
     // exact residues, so the split result is the same word); 16 per lane would hold 3 waves per
     // SIMD instead of 5
-    if (c.split_mac_ok) {
-      if (bStep <= 4) k_lt_mac<4, Mac30><<<g, kT, 0, st>>>(fast.p, diags, R.p, mp);
-      else
-        for (mp.i0 = 0; mp.i0 < (uint32_t)bStep; mp.i0 += 8, mp.acc = 1) k_lt_mac<8, Mac30><<<g, kT, 0, st>>>(fast.p, diags, R.p, mp);
-    } else {
-      if (bStep <= 4) k_lt_mac<4, MacWide><<<g, kT, 0, st>>>(fast.p, diags, R.p, mp);
-      else
-        for (mp.i0 = 0; mp.i0 < (uint32_t)bStep; mp.i0 += 8, mp.acc = 1) k_lt_mac<8, MacWide><<<g, kT, 0, st>>>(fast.p, diags, R.p, mp);
+    for (mp.i0 = 0; mp.i0 < (uint32_t)bStep; mp.i0 += 8, mp.acc = 1) {
+      hoist_baby(c, h, mp.i0, std::min(8, bStep - (int)mp.i0), stride, slots, baby_keys, baby_gal);
+      k_lt_mac<8, M, DM><<<g, kT, 0, st>>>(h, diags, R.p, mp);
     }
-    FH_HIP(hipGetLastError());
-  }
+  });
+  FH_HIP(hipGetLastError());
   return R;
 }
 
@@ -328,12 +448,12 @@ void linear_transform_flat(Context& c, const uint64_t* ct, int l, int rowSize, i
   for (uint32_t p = 0; p < ext; ++p) epids[p] = c.ext_prime(l, p);
   const LimbSet acc = make_set(R.p, ext, epids.data(), 2, E);
   if (!rot.empty()) {
-    // the rotated partial sums side by side: one ModDown of their c1, one ModUp, one key inner
-    // product with each item's own key (the extended c0 folded directly, as a Horner step does)
+    // the rotated partial sums side by side: one ModDown of their c1, one ModUp, and one launch that
+    // adds every item's key inner product (the extended c0 folded directly, as a Horner step does)
     const int nr = (int)rot.size();
     bool contiguous = true;
     for (int t = 1; t < nr; ++t) contiguous &= rot[t] == rot[0] + t;
-    DBuf gathered, c1q(c.pool, (size_t)nr * lq * N), dig(c.pool, (size_t)nr * beta * E), T(c.pool, (size_t)nr * 2 * E);
+    DBuf gathered, c1q(c.pool, (size_t)nr * lq * N), dig(c.pool, (size_t)nr * beta * E);
     const uint64_t* src = R.p + (size_t)rot[0] * 2 * E;
     if (!contiguous) {
       gathered = DBuf(c.pool, (size_t)nr * 2 * E);
@@ -343,9 +463,8 @@ void linear_transform_flat(Context& c, const uint64_t* ct, int l, int rowSize, i
     }
     moddown(c, src + E, l, c1q.p, nr, 2 * E, (uint64_t)lq * N, st);
     modup_batch(c, c1q.p, l, nr, (uint64_t)lq * N, dig.p, st, false);
-    ksk_items(c, nr, 1, dig.p, (uint64_t)beta * E, src, 2 * E, true, true, l, keys.data(), gals.data(), T.p, 2 * E, st, c1q.p,
-              (uint64_t)lq * N);
-    lt_sum(c, acc, T.p, 2 * E, nr, st);
+    hoist_sum(c, hoist_group(c, l, dig.p, (uint64_t)beta * E, c1q.p, (uint64_t)lq * N, src, 2 * E, true), nr, keys.data(), gals.data(), 1,
+              true, R.p, st);
   }
   for (int j = 1; j < gStep; ++j)
     if (((long long)j * bStep * stride) % slots == 0) ew_binary(c, 0, acc, make_set(R.p + (size_t)j * 2 * E, ext, epids.data(), 2, E), acc, st);
@@ -478,26 +597,17 @@ void accumulate_cascade(Context& c, const uint64_t* ct, int l, int radix, int si
   const size_t E = (size_t)ext * N, Q = (size_t)lq * N;
   if (out != ct) FH_HIP(hipMemcpyAsync(out, ct, 2 * Q * 8, hipMemcpyDeviceToDevice, st));
   if (start <= 0 || size <= 0 || start >= size) return;
-  std::vector<int> epids(ext);
-  for (uint32_t p = 0; p < ext; ++p) epids[p] = c.ext_prime(l, p);
-  DBuf fast(c.pool, (size_t)radix * 2 * E);
+  DBuf sum(c.pool, 2 * E), dig(c.pool, (size_t)c.num_digits(l) * E);
   int used = 0;
   for (long long s = start; s < size; s *= radix) {
     int n = 0;
     while (n + 1 < radix && (long long)(n + 1) * s < size) ++n;
-    {
-      ProfScope ps_(c, "lt_extend", st);
-      k_extend_p<<<grid_n(N, 2 * ext), kT, 0, st>>>(out, fast.p, N, lq, ext, c.d_prime, c.d_pmod, c.d_pmod_sh);
-      FH_HIP(hipGetLastError());
-    }
-    rotate_hoisted(c, out, l, n, keys + used, galois + used, true, false, fast.p + 2 * E, st);
-    LimbSet a = make_set(fast.p, ext, epids.data(), 2, E);
-    lt_sum(c, a, fast.p + 2 * E, 2 * E, n, st);
-    moddown(c, fast.p, l, out, 2, 0, 0, st);
+    modup_batch(c, out + Q, l, 1, 0, dig.p, st, false);
+    hoist_sum(c, hoist_group(c, l, dig.p, 0, out + Q, 0, out, 0, false), n, keys + used, galois + used, 0, false, sum.p, st);
+    moddown(c, sum.p, l, out, 2, 0, 0, st);
     used += n;
   }
 }
-
 
 // The lazy rotation-fold sum (CKKS::Accumulate(ct, bStep, stride, size),
 // src/CKKS/AccumulateBroadcast.cu:122-160). Per fold level s = 1, radix, ... < size: one ModUp of c1
@@ -505,42 +615,31 @@ void accumulate_cascade(Context& c, const uint64_t* ct, int l, int radix, int si
 // c0 is folded as P*c0 on the first level and afterwards stays in Q_l ∪ P, where it is added on
 // every limb before the automorphism (the c0_modup branch of hoistedRotateDotKSK_2_,
 // src/CKKS/ElemenwiseBatchKernels.cu:302-307). The rotations are summed into (c0, P*c1); c1 takes a
-// ModDown at the end of each level and c0 one ModDown after the last. Buffer fast: slot 0 holds the
-// accumulators (extended c0, extended c1), slots 1..radix-1 the level's rotations.
+// ModDown at the end of each level and c0 one ModDown after the last. The levels' sums alternate
+// between two buffers, since a level's rotations gather from the last level's c0.
 void accumulate_sum(Context& c, const uint64_t* ct, int l, int radix, int size, const uint64_t* const* keys, const uint32_t* galois,
                     uint64_t* out, hipStream_t st) {
   const uint32_t N = c.N, lq = l + 1, ext = lq + c.K, beta = c.num_digits(l);
   const size_t E = (size_t)ext * N, Q = (size_t)lq * N;
   if (out != ct) FH_HIP(hipMemcpyAsync(out, ct, 2 * Q * 8, hipMemcpyDeviceToDevice, st));
   if (size <= 1 || radix < 2) return;
-  std::vector<int> epids(ext);
-  for (uint32_t p = 0; p < ext; ++p) epids[p] = c.ext_prime(l, p);
-  DBuf fast(c.pool, (size_t)radix * 2 * E);
-  DBuf dig(c.pool, (size_t)beta * E);
-  bool c0_ext = false;
+  DBuf sum(c.pool, 4 * E), dig(c.pool, (size_t)beta * E);
+  uint64_t* cur = nullptr;   // the last level's sums: extended c0, extended c1
+  uint64_t* next = sum.p;
   int used = 0;
   for (long long s = 1; s < size; s *= radix) {
     int n = 0;
     while (n + 1 < radix && (long long)(n + 1) * s < size) ++n;
     // the level's rotations, all from the level's input (c0 or its extension, and c1)
     modup_batch(c, out + Q, l, 1, 0, dig.p, st, false);
-    ksk_items(c, n, n, dig.p, 0, c0_ext ? fast.p : out, 0, true, c0_ext, l, keys + used, galois + used, fast.p + 2 * E, 2 * E, st,
-              out + Q, 0);
-    {
-      // accumulators: P*c1 (and P*c0 on the first level; afterwards slot 0 already holds c0)
-      ProfScope ps_(c, "lt_extend", st);
-      const uint32_t comps = c0_ext ? 1 : 2;
-      k_extend_p<<<grid_n(N, comps * ext), kT, 0, st>>>(c0_ext ? out + Q : out, c0_ext ? fast.p + E : fast.p, N, lq, ext, c.d_prime,
-                                                       c.d_pmod, c.d_pmod_sh);
-      FH_HIP(hipGetLastError());
-    }
-    LimbSet a = make_set(fast.p, ext, epids.data(), 2, E);
-    lt_sum(c, a, fast.p + 2 * E, 2 * E, n, st);
-    moddown(c, fast.p + E, l, out + Q, 1, 0, 0, st);
-    c0_ext = true;
+    hoist_sum(c, hoist_group(c, l, dig.p, 0, out + Q, 0, cur ? cur : out, 0, cur != nullptr), n, keys + used, galois + used, cur ? 2 : 0,
+              false, next, st);
+    moddown(c, next + E, l, out + Q, 1, 0, 0, st);
+    cur = next;
+    next = cur == sum.p ? sum.p + 2 * E : sum.p;
     used += n;
   }
-  moddown(c, fast.p, l, out, 1, 0, 0, st);
+  moddown(c, cur, l, out, 1, 0, 0, st);
 }
 
 }  // namespace fh
