@@ -58,7 +58,7 @@ struct HoistLimb {
 // DM bounds the digits. Memory-bound: the keys are read once; writing the rotations and reading them
 // back was a third of the traffic. N = 2^16, 50-bit primes, three digits, against key product, sum
 // and extension in launches of their own: the radix-4 fold of 256 slots 1325 -> 1022 us, 63 diagonals
-// in 16 baby steps 1495 -> 1320 us.
+// in 16 baby steps 1495 -> 1270 us.
 template <class M, int DM>
 __device__ __forceinline__ void hoist_rot(const Hoist& h, const HoistLimb& L, const uint64_t* key, uint32_t gal, uint32_t t, uint32_t n,
                                           uint64_t& r0, uint64_t& r1) {
@@ -115,8 +115,11 @@ struct MacParams {
 // One lane forms the bStep rotated words of both components for its (position, coefficient)
 // and streams the diagonals once; each sum (at most 16 products) is accumulated exactly under the
 // multiply policy M and reduced once. The rotations never reach memory.
+// Up to four digits four waves a SIMD are asked for: left alone the compiler takes 133 registers for
+// eight baby steps, which is three waves (28 bytes spilled; 63 diagonals in 16 baby steps 1319 -> 1270
+// us); with more digits that would spill 156 bytes.
 template <int BB, class M, int DM>
-__global__ __launch_bounds__(kT) void k_lt_mac(Hoist h, const uint64_t* __restrict__ diags, uint64_t* __restrict__ R, MacParams mp) {
+__global__ __launch_bounds__(kT, DM <= 4 ? 4 : 1) void k_lt_mac(Hoist h, const uint64_t* __restrict__ diags, uint64_t* __restrict__ R, MacParams mp) {
   using Op = typename M::Op;
   const HoistLimb L(h, blockIdx.y);
   const size_t N = h.N, E = (size_t)h.ext * N;
@@ -262,7 +265,8 @@ struct MacBatchParams {
 
 // Giant-step partial sums for B ciphertexts sharing one diagonal set, from the rotations that
 // k_ksk_batch wrote. Forming them here, as k_lt_mac does, was measured slower for a batch: 16
-// ciphertexts, N = 2^16, 30 limbs, 8 x 8 steps, 20.5 against 16.7 ms for the transform. There the key
+// ciphertexts, N = 2^16, 30 limbs, 8 x 8 steps, 20.5 (two waves a SIMD) and 18.9 ms (four, with spills)
+// against 16.7 for the transform. There the key
 // product reads its keys once for the whole batch, here once per ciphertext and wave. blockIdx.y = extended
 // position, blockIdx.x = a 64-coefficient tile: the tile of every diagonal is staged in LDS once
 // (as multiply operands, split into 30-bit halves under Mac30) and applied to all B ciphertexts
@@ -358,8 +362,8 @@ DBuf lt_partials(Context& c, const uint64_t* ct, int l, int rowSize, int bStep, 
       return;
     }
     // more than 8 baby steps: launches of 8 each, the later ones adding into R (the sums are
-    // exact residues, so the split result is the same word); 16 per lane would hold 3 waves per
-    // SIMD instead of 5
+    // exact residues, so the split result is the same word). 16 rotations a lane keep too few waves in
+    // flight: 63 diagonals, 16 baby steps, N = 2^16, 30 limbs: 1463 us for the transform against 1319 (1270 with the bound above)
     for (mp.i0 = 0; mp.i0 < (uint32_t)bStep; mp.i0 += 8, mp.acc = 1) {
       hoist_baby(c, h, mp.i0, std::min(8, bStep - (int)mp.i0), stride, slots, baby_keys, baby_gal);
       k_lt_mac<8, M, DM><<<g, kT, 0, st>>>(h, diags, R.p, mp);
