@@ -78,9 +78,9 @@ def algorithmic_bytes(family, N, lq, ext, beta, B, groups):
         digits = B * beta * ext
         keys = groups * 2 * beta * ext
         return limb * (digits + keys + B * lq + 2 * B * ext)
-    if family == "modup_conv":
-        return limb * B * (2 * lq + beta * ext - lq)
-    if family == "moddown_conv":
+    if family in ("modup_conv_cols", "modup_conv"):   # sources read once, every digit's other limbs written
+        return limb * B * (lq + beta * ext - lq)
+    if family in ("moddown_conv_cols", "moddown_conv"):
         return limb * 2 * B * (K + lq)
     return None
 
@@ -225,8 +225,9 @@ def main():
         ctx.rotate_batch(cts, B, lvl, ks, gs, out_b)
     ctx.sync()
     t_batched = time.perf_counter() - t0
-    fams = ["ntt_inv_rows", "ntt_inv_cols", "ntt_fwd_cols", "ntt_fwd_rows", "modup_conv", "ksk_batch",
-            "moddown_conv", "ntt_fwd_rows_moddown", "ntt_rows_ksk"]
+    # *_conv_cols: a basis conversion and its targets' column pass in one launch
+    fams = ["ntt_inv_rows", "ntt_inv_cols", "modup_conv_cols", "ntt_fwd_rows", "ksk_batch", "moddown_conv_cols",
+            "ntt_fwd_rows_moddown", "ntt_rows_ksk"]
     prof = {f: ctx.profile_read(f) for f in fams}
     ctx.profile(False)
     ms_per_step = 1000.0 * t_batched / a.steps

@@ -32,6 +32,7 @@ struct PrimeConst {
 };
 
 __device__ __forceinline__ uint64_t mulhi(uint64_t a, uint64_t b) { return __umul64hi(a, b); }
+__device__ __forceinline__ uint32_t mulhi32(uint32_t a, uint32_t b) { return (uint32_t)(((uint64_t)a * b) >> 32); }
 
 // a*w mod q in [0, 2q) for any a < 2^64 and w < q, with wp = floor(w 2^64 / q).
 __device__ __forceinline__ uint64_t shoup_lazy(uint64_t a, uint64_t w, uint64_t wp, uint64_t q) {
@@ -43,7 +44,7 @@ __device__ __forceinline__ uint64_t shoup_lazy(uint64_t a, uint64_t w, uint64_t 
 // two below the exact one; 13 instructions, where the exact product above takes 22.
 __device__ __forceinline__ uint64_t shoup_lazy4(uint64_t a, uint64_t w, uint64_t wp, uint64_t nq) {
   const uint32_t al = (uint32_t)a, ah = (uint32_t)(a >> 32), pl = (uint32_t)wp, ph = (uint32_t)(wp >> 32);
-  const uint64_t h = (uint64_t)ah * ph + ((uint64_t)__umulhi(ah, pl) + __umulhi(al, ph));
+  const uint64_t h = (uint64_t)ah * ph + ((uint64_t)mulhi32(ah, pl) + mulhi32(al, ph));
   const uint32_t hl = (uint32_t)h, hh = (uint32_t)(h >> 32), wl = (uint32_t)w, wh = (uint32_t)(w >> 32);
   const uint32_t ql = (uint32_t)nq, qh = (uint32_t)(nq >> 32);
   const uint64_t p = (uint64_t)al * wl + (uint64_t)hl * ql;

@@ -56,9 +56,13 @@ struct EpiJob {
 // well, wait on both counters and take no scalar base. The pointer must be uniform over the wave.
 template <class T>
 __device__ __forceinline__ T* as_global(T* p) {
+#ifdef __HIP_DEVICE_COMPILE__
   const uint64_t v = (uint64_t)p;
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
   return (T*)(__attribute__((address_space(1))) T*)((uint64_t)hi << 32 | lo);
+#else
+  return p;
+#endif
 }
 
 struct SetAddr {

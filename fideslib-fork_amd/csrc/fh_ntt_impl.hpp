@@ -10,12 +10,12 @@
 //  * N = S1 * S2 (S1 = 2^l1 "column" points, S2 = 2^l2 "row" points). The first
 //    l1 stages only couple elements of one column (stride S2), the last l2
 //    stages only elements of one row (contiguous), so a limb is transformed by
-//    two launches: the column launch with the table's first S1 twiddles in LDS, the row launch with
-//    each row's own twiddles straight from the table. Each lane owns 16 elements of one sub-transform: four radix-2
-//    stages run in registers, one LDS exchange re-partitions the sub-transform,
-//    the remaining stages run in registers again. Global loads and stores are
-//    coalesced in both passes (rows are staged through LDS where the register
-//    layout is not).
+//    two launches: the column launch with the table's first S1 twiddles in LDS,
+//    the row launch with each row's own twiddles straight from the table. Each
+//    lane owns 16 elements of one sub-transform: four radix-2 stages run in
+//    registers, one LDS exchange re-partitions the sub-transform, the remaining
+//    stages run in registers again. Global loads and stores are coalesced in both
+//    passes (rows are staged through LDS where the register layout is not).
 //  * Two exact arithmetics, chosen per limb by its prime:
 //      - fp64 (q < 2^50.2, the 50-bit scaling primes): residues are doubles in a
 //        signed lazy range; a product is split exactly with FMA (h = yw,
