@@ -108,6 +108,43 @@ __global__ __launch_bounds__(kEncThreads) void k_encode_round(const D2* __restri
   for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < N; j += gridDim.x * blockDim.x) o[j] = coeff_at(wk, j, N, n, logn, loggap, scale);
 }
 
+// Uploads from the caller's host memory, which is the caller's again when the encoder returns. From
+// pageable memory hipMemcpyAsync returns once the memory has been read; from page-locked or managed
+// memory the copy may still wait behind earlier work of the stream, so it is waited for here (the
+// copy alone: the kernels behind it stay queued). Not under stream capture, where nothing has run yet.
+class HostReads {
+ public:
+  explicit HostReads(hipStream_t st) : st_(st) {}
+  HostReads(const HostReads&) = delete;
+  HostReads& operator=(const HostReads&) = delete;
+  ~HostReads() {
+    if (!ev_) return;
+    if (hipEventSynchronize(ev_) != hipSuccess) (void)hipGetLastError();
+    (void)hipEventDestroy(ev_);
+  }
+  void copy(void* dst, const void* src, size_t bytes) {
+    if (returns_early(src) && !ev_) FH_HIP(hipEventCreateWithFlags(&ev_, hipEventDisableTiming));
+    FH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st_));
+    if (!ev_) return;
+    const hipError_t e = hipEventRecord(ev_, st_);
+    if (e != hipSuccess) (void)hipStreamSynchronize(st_);
+    FH_HIP(e);
+  }
+
+ private:
+  bool returns_early(const void* p) const {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    FH_HIP(hipStreamIsCapturing(st_, &cs));
+    if (cs != hipStreamCaptureStatusNone) return false;
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();   // pageable memory may be unknown to the runtime
+    return false;
+  }
+  hipStream_t st_;
+  hipEvent_t ev_ = nullptr;
+};
+
 inline dim3 enc_grid(uint32_t N, uint32_t jobs) {
   uint32_t gx = (N + kEncThreads - 1) / kEncThreads;
   if (gx > 64) gx = 64;
@@ -178,11 +215,12 @@ void encode_slots(Context& c, const double* values, int count, uint32_t slots, d
   // chunks of about 8 MB of slot values: the upload of one chunk (synchronous for pageable host
   // memory) overlaps the transforms of the previous one
   const int chunk = std::max(1, std::min(count, (int)((8u << 20) / (16u * n))));
+  HostReads reads(st);
   for (int b0 = 0; b0 < count; b0 += chunk) {
     const int nb = std::min(chunk, count - b0);
     double* v = reinterpret_cast<double*>(vals.p) + (size_t)b0 * n * 2;
     D2* wk = reinterpret_cast<D2*>(work.p) + (size_t)b0 * n;
-    FH_HIP(hipMemcpyAsync(v, values + (size_t)b0 * n * 2, (size_t)nb * n * 2 * sizeof(double), hipMemcpyHostToDevice, st));
+    reads.copy(v, values + (size_t)b0 * n * 2, (size_t)nb * n * 2 * sizeof(double));
     ProfScope ps_(c, "encode", st);
     k_ifft_load<<<dim3((n + kEncThreads - 1) / kEncThreads, nb), kEncThreads, 0, st>>>(v, wk, n);
     FH_HIP(hipGetLastError());
@@ -208,7 +246,8 @@ void encode_coeffs(Context& c, const int64_t* coeffs, int count, const LimbSet& 
   if ((uint32_t)count != out.npolys) throw Error(-1, "encode: output set and count differ");
   if (count > 65535 || (size_t)out.nlimbs * count > 65535) throw Error(-1, "encode: too many plaintexts in one call");
   DBuf m(c.pool, (size_t)count * c.N);
-  FH_HIP(hipMemcpyAsync(m.p, coeffs, (size_t)count * c.N * sizeof(int64_t), hipMemcpyHostToDevice, st));
+  HostReads reads(st);
+  reads.copy(m.p, coeffs, (size_t)count * c.N * sizeof(int64_t));
   ntt_fwd_signed(c, reinterpret_cast<const int64_t*>(m.p), out, st);
 }
 

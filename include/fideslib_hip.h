@@ -109,12 +109,14 @@ int fh_ntt_inverse(fh_context* ctx, uint64_t* polys, const int32_t* prime_ids, i
  * (every product and sum rounded once), / slots, * scale, llround, the gap scatter (real parts at
  * i * N/(2 slots), imaginary parts N/2 above), residues modulo prime_ids[0..num_limbs), forward NTT:
  * out holds count polynomials of num_limbs limbs, out_stride words apart (0 = packed), equal bit
- * for bit to the host encoder. (|re| + |im|) * scale must stay below 2^63. Replaces
- * EncodeChunkSlots / loadSlotsBatch (src/CKKS/DeviceEncodeBatch.cu:435-665, 766-860). */
+ * for bit to the host encoder. (|re| + |im|) * scale must stay below 2^61 (1 - 2^-40), for every
+ * value, or nothing is written. values has been read when the call returns, page-locked or not; the
+ * result is complete behind the context stream. Replaces EncodeChunkSlots / loadSlotsBatch
+ * (src/CKKS/DeviceEncodeBatch.cu:435-665, 766-860). */
 int fh_encode_slots(fh_context* ctx, const double* values, int count, int slots, double scale, const int32_t* prime_ids, int num_limbs,
                     uint64_t* out, size_t out_stride);
-/* The same from signed integer coefficients (count x N, host): residues and forward NTT. Replaces
- * fit_to_native_batch_ / EncodeChunk / loadCoefficientsBatch
+/* The same from signed integer coefficients (count x N, host; read when the call returns): residues
+ * and forward NTT. Replaces fit_to_native_batch_ / EncodeChunk / loadCoefficientsBatch
  * (src/CKKS/DeviceEncodeBatch.cu:143-390, 665-760). */
 int fh_encode_coeffs(fh_context* ctx, const int64_t* coeffs, int count, const int32_t* prime_ids, int num_limbs, uint64_t* out,
                      size_t out_stride);

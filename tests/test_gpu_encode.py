@@ -1,6 +1,8 @@
 """Device CKKS encoding (fh_encode_slots / fh_encode_coeffs) against the oracle's encoder, bit for
 bit: the special inverse FFT in fp64 with the host encoder's rounding sequence, the gap scatter,
 the residues and the forward NTT; batched plaintexts; Q and Q-and-P prime sets."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -84,3 +86,35 @@ def test_encode_at_the_2_61_boundary(gctx2, octx2):
     with pytest.raises(ValueError):
         o.encode(np.array([8.0 + 0j]), 2.0 ** 58, 2)
     out.free()
+
+
+@pytest.mark.parametrize("form", ["slots", "coeffs"])
+def test_input_is_read_when_the_call_returns(form, gctx2, fh):
+    """The caller's array is the caller's again on return, page-locked memory (which a copy engine reads
+    after the call is queued) included: here the upload is queued behind transforms on the stream."""
+    g = gctx2
+    pids, count = [0, 1, g.L1], 20          # more than one chunk of slot values
+    if form == "slots":
+        src = _values(g.N // 2, 12, count)
+        encode = lambda v, out: g.encode_slots(v, 2.0 ** 50, pids, out)
+    else:
+        src = np.random.default_rng(11).integers(-(1 << 50), 1 << 50, (count, g.N), dtype=np.int64)
+        encode = lambda v, out: g.encode_coeffs(v, pids, out)
+    hip, p = fh.load(), ctypes.c_void_p()   # the runtime's symbols are found through the library's dependencies
+    assert hip.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(src.nbytes), ctypes.c_uint(0)) == 0
+    pinned = np.frombuffer((ctypes.c_char * src.nbytes).from_address(p.value), dtype=src.dtype).reshape(src.shape)
+    ids = list(range(g.L1 + g.K))
+    ref, got, busy = g.array((count * len(pids), g.N)), g.array((count * len(pids), g.N)), g.array((32 * len(ids), g.N))
+    g.fill_uniform(busy, ids, num_polys=32)
+    encode(src, ref)
+    g.sync()
+    for _ in range(2):
+        pinned[...] = src
+        for _ in range(8):
+            g.ntt_forward(busy, ids, num_polys=32)
+        encode(pinned, got)
+        pinned[...] = 0
+        assert np.array_equal(got.download(), ref.download())
+    for a in (ref, got, busy):
+        a.free()
+    assert hip.hipHostFree(p) == 0
