@@ -1,5 +1,6 @@
 // NTT / INTT entry points over limb sets (in place and out of place, with the ModDown
 // epilogue), and the NTT launch-shape autotuner. The kernels are in fh_ntt_impl.hpp.
+#include "fh_keyswitch.hpp"
 #include "fh_ntt_impl.hpp"
 #include "fh_ops.hpp"
 
@@ -79,7 +80,11 @@ AutotuneResult autotune_ntt(Context& c, int polys) {
     // a candidate replaces the current choice only when it is clearly faster: timing noise and the
     // difference between this synthetic set and a workload's launches are a few percent
     constexpr double kGain = 0.95;
-    for (int l1 = 4; l1 <= 8; ++l1) {
+    // The conversions fused with the column pass (conv_cols) are built for the default split: another
+    // one would turn them off in every ModUp and ModDown, which the transforms timed here do not show
+    // (16 rotations at N = 2^15, 24 limbs: 882 us, at split 8 1037). Where they run the split stays.
+    const bool fixed = conv_cols_usable(c, std::max(c.alpha, c.K));
+    for (int l1 = 4; l1 <= 8 && !fixed; ++l1) {
       if (l1 == l1d || !ntt_split_ok(c.logN, l1)) continue;
       c.tune.ntt_split = l1;
       const double t = measure();

@@ -423,7 +423,9 @@ int fh_profile_read(fh_context* ctx, const char* name, int* launches, double* to
  *   "ntt_chunk_mb"          limb data per NTT launch pair (MB, >= 1)
  *   "ntt_mix"               0/1: spread the NTT jobs of 60-bit primes among the 50-bit ones
  *   "ntt_split"             log2 of the column-pass length: 0 (floor(logN/2)) or a split with both
- *                           factors in [2^4, 2^8] and within a factor 4 of each other
+ *                           factors in [2^4, 2^8] and within a factor 4 of each other; at a split
+ *                           other than the default a basis conversion and its targets' column
+ *                           pass are separate launches
  *   "ntt_fwd_cols_threads", "ntt_fwd_rows_threads", "ntt_inv_rows_threads", "ntt_inv_cols_threads"
  *                           workgroup size of each pass, 256 or 512 (512: default split only)
  *   "rot_streams"           1/2: fh_rotate_batch of 8 or more ciphertexts as two halves on two
@@ -436,7 +438,8 @@ int fh_profile_read(fh_context* ctx, const char* name, int* launches, double* to
  *   "ntt_streams"           1/2: the chunks of a chunked NTT alternate between two streams
  *   "ntt_team"              0/1: NTTs over N = S x S run as one cooperative launch of workgroup
  *                           teams, one HBM round trip per limb (the intermediate stays in the L2 of
- *                           the team's XCD); outside HIP graph capture
+ *                           the team's XCD); outside HIP graph capture; basis conversions are
+ *                           launches of their own then
  *   "ntt_team_per_xcd"      teams per XCD of such a launch (1..64) */
 int fh_tune_set(fh_context* ctx, const char* name, int value);
 int fh_tune_get(const fh_context* ctx, const char* name, int* value);
@@ -444,7 +447,9 @@ int fh_tune_get(const fh_context* ctx, const char* name, int* value);
 /* NTT autotuner (no reference counterpart). Times forward + inverse NTTs of `polys` synthetic
  * polynomials over every prime of the context (resident in HBM) under candidate radix splits,
  * per-pass workgroup sizes and limbs per launch pair, and keeps the fastest as the context's
- * tunables. Synchronizes the context stream. */
+ * tunables. The split stays the default where key switching then runs its basis conversions fused
+ * with the column pass (three sources or more, primes in (2^48, 2^60), N >= 2^12, neither
+ * ReducedNoise nor ntt_team on: set those before). Synchronizes the context stream. */
 typedef struct fh_autotune_report {
   int split;              /* chosen log2 column-pass length */
   int threads[4];         /* forward cols, forward rows, inverse rows, inverse cols */

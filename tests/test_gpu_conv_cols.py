@@ -82,3 +82,25 @@ def test_many_polynomials(fh, oracle_mod):
         kk.free()
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("logN,L1,K,splits", [(13, 6, 3, 0), (12, 6, 1, 0), (12, 2, 3, 0), (13, 4, 2, 1), (11, 6, 3, 1)])
+def test_autotuned_context_keeps_the_fused_conversions(fh, oracle_mod, logN, L1, K, splits):
+    """The autotuner times transforms alone, so it may not choose a split that the fused conversions are not
+    built for: it tries other splits only where no conversion of the context is fused."""
+    g = fh.Context(logN, L1, K, 2)
+    try:
+        o = oracle_mod.Ctx(logN, [int(q) for q in g.moduli], L1, K, 2)
+        r = g.autotune(2)
+        assert r["candidates"] == 1 + splits + 4, r     # the default, other splits, four workgroup sizes
+        key = np.concatenate([o.random_poly(10 + i, list(range(L1 + K))) for i in range(4)])
+        ct = np.concatenate([o.random_poly(30 + i, list(range(L1))) for i in range(2)])
+        kk, gal, d, out = g.key(key), g.galois_index(1), g.to_device(ct), g.array((2 * L1, o.N))
+        g.profile()
+        g.profile_reset()
+        g.eval_rotate(d, L1 - 1, kk, gal, out)
+        assert np.array_equal(out.download(), o.eval_rotate(ct, L1 - 1, key, gal))
+        assert g.profile_read("modup_conv_cols")[0] == (logN >= 12 and L1 // 2 > 2)
+        assert g.profile_read("moddown_conv_cols")[0] == (logN >= 12 and K > 2)
+    finally:
+        g.close()
