@@ -6,20 +6,20 @@
 
 namespace fh {
 
-void ntt_fwd(const Context& c, const LimbSet& s, hipStream_t st) { dispatch(c, SetAddr{s}, SetAddr{s}, s.nlimbs * s.npolys, st, true); }
-void ntt_inv(const Context& c, const LimbSet& s, hipStream_t st) { dispatch(c, SetAddr{s}, SetAddr{s}, s.nlimbs * s.npolys, st, false); }
+void ntt_fwd(const Context& c, const LimbSet& s, hipStream_t st) { dispatch_fwd(c, SetAddr{s}, SetAddr{s}, s.nlimbs * s.npolys, st); }
+void ntt_inv(const Context& c, const LimbSet& s, hipStream_t st) { dispatch_inv(c, SetAddr{s}, SetAddr{s}, s.nlimbs * s.npolys, st); }
 void ntt_fwd(const Context& c, const LimbSet& in, const LimbSet& out, hipStream_t st) {
   if (in.nlimbs * in.npolys != out.nlimbs * out.npolys) throw Error(-1, "NTT in/out shapes differ");
-  dispatch(c, SetAddr{in}, SetAddr{out}, in.nlimbs * in.npolys, st, true);
+  dispatch_fwd(c, SetAddr{in}, SetAddr{out}, in.nlimbs * in.npolys, st);
 }
 void ntt_inv(const Context& c, const LimbSet& in, const LimbSet& out, hipStream_t st) {
   if (in.nlimbs * in.npolys != out.nlimbs * out.npolys) throw Error(-1, "NTT in/out shapes differ");
-  dispatch(c, SetAddr{in}, SetAddr{out}, in.nlimbs * in.npolys, st, false);
+  dispatch_inv(c, SetAddr{in}, SetAddr{out}, in.nlimbs * in.npolys, st);
 }
 void ntt_fwd_moddown(const Context& c, const LimbSet& conv, const uint64_t* x, uint64_t x_stride, uint64_t* out, uint64_t out_stride,
                      hipStream_t st, bool cols, const uint64_t* add, uint64_t add_pair) {
   EpiModDown e{x, x_stride, out, out_stride, add, add_pair, c.d_md_pinv, c.d_md_pinv_sh, conv.npolys, conv.nlimbs, nullptr, nullptr, nullptr, 0, 0, 0};
-  dispatch(c, SetAddr{conv}, SetAddr{conv}, conv.nlimbs * conv.npolys, st, true, e, "ntt_fwd_rows_moddown", cols);
+  dispatch_fwd(c, SetAddr{conv}, SetAddr{conv}, conv.nlimbs * conv.npolys, st, e, "ntt_fwd_rows_moddown", cols);
 }
 
 // ------------------------------------------------------------------------------- autotuner

@@ -7,7 +7,7 @@ namespace fh {
 void ntt_fwd_modup(const Context& c, const ModUpAddr& a, uint32_t n, hipStream_t st, bool cols) {
   ModUpAddr m = a;
   m.mix = c.tune.ntt_mix ? 1u : 0u;
-  dispatch(c, m, m, n, st, true, EpiStore{}, "ntt_fwd_rows", cols);
+  dispatch_fwd(c, m, m, n, st, EpiStore{}, "ntt_fwd_rows", cols);
 }
 
 }  // namespace fh

@@ -8,21 +8,21 @@ void ntt_fwd_rescale(const Context& c, const LimbSet& e, const uint64_t* top, co
   const size_t o = (size_t)l * c.L1;
   EpiRescale ep{x, out, c.d_rs_qlinv + o, c.d_rs_qlinv_sh + o, l, e.npolys, nullptr, nullptr, 0, 0, 0};
   ProRescale pr{top, c.d_rs_QlQl + o, c.d_rs_QlQl_sh + o, l, e.npolys, {}};
-  dispatch(c, SetAddr{e}, SetAddr{e}, e.nlimbs * e.npolys, st, true, ep, "ntt_fwd_rows_rescale", true, pr);
+  dispatch_fwd(c, SetAddr{e}, SetAddr{e}, e.nlimbs * e.npolys, st, ep, "ntt_fwd_rows_rescale", true, pr);
 }
 
 void ntt_fwd_mod_raise(const Context& c, const uint64_t* x0, const LimbSet& out, hipStream_t st) {
   ProModRaise pr{};
   pr.x0 = x0;
   pr.npolys = out.npolys;
-  dispatch(c, SetAddr{out}, SetAddr{out}, out.nlimbs * out.npolys, st, true, EpiStore{}, "ntt_fwd_rows", true, pr);
+  dispatch_fwd(c, SetAddr{out}, SetAddr{out}, out.nlimbs * out.npolys, st, EpiStore{}, "ntt_fwd_rows", true, pr);
 }
 
 void ntt_fwd_signed(const Context& c, const int64_t* m, const LimbSet& out, hipStream_t st) {
   ProSigned pr{};
   pr.m = m;
   pr.npolys = out.npolys;
-  dispatch(c, SetAddr{out}, SetAddr{out}, out.nlimbs * out.npolys, st, true, EpiStore{}, "ntt_fwd_rows", true, pr);
+  dispatch_fwd(c, SetAddr{out}, SetAddr{out}, out.nlimbs * out.npolys, st, EpiStore{}, "ntt_fwd_rows", true, pr);
 }
 
 }  // namespace fh

@@ -43,3 +43,14 @@ def test_no_cpu_fallback_in_binding():
     """The Python binding only forwards to the shared library; it never imports the oracle."""
     src = open(os.path.join(ROOT, "fideslib-fork_amd", "fides_hip.py")).read()
     assert "oracle" not in src.replace("oracle/", "")
+
+
+@pytest.mark.skipif(not os.path.exists(LIB), reason="libfideslib_hip.so not built")
+def test_inverse_transform_kernels_are_built_once():
+    """Units that only transform forward (ModUp targets, limbs formed in the first launch) hold no inverse
+    kernels: each one is in the library once, and none is over ModUp targets, which nothing transforms back."""
+    out = subprocess.run(["nm", "--defined-only", LIB], capture_output=True, text=True, check=True).stdout
+    syms = [line.split()[-1] for line in out.splitlines() if "__device_stub__k_ntt_inv_" in line]
+    assert syms
+    assert len(syms) == len(set(syms))
+    assert not [s for s in syms if "ModUpAddr" in s]
