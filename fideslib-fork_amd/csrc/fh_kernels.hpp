@@ -222,6 +222,10 @@ void ntt_fwd_rescale(const Context& c, const LimbSet& e, const uint64_t* top, co
 void ntt_fwd_mod_raise(const Context& c, const uint64_t* x0, const LimbSet& out, hipStream_t st);
 // forward NTT of npolys x N signed integer coefficients modulo every limb of out
 void ntt_fwd_signed(const Context& c, const int64_t* m, const LimbSet& out, hipStream_t st);
+// Load the code objects of the transforms over limb sets and of the three forms above on the current
+// device, which the runtime would do at the first launch of one of their kernels.
+void ntt_load();
+void ntt_pro_load();
 void ntt_inv_jobs(const Context& c, const LimbJob* d_jobs, uint32_t njobs, hipStream_t st);
 // out-of-place job forms: job y reads in[y].ptr and writes out[y].ptr (same prime)
 void ntt_fwd_jobs(const Context& c, const LimbJob* d_in, const LimbJob* d_out, uint32_t njobs, hipStream_t st);

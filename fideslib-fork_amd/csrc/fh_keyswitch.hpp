@@ -109,7 +109,8 @@ void rescale(Context& c, const uint64_t* x, int l, int ncomp, uint64_t* out, hip
 inline size_t rescale_work_words(const Context& c, int l, int ncomp) { return (size_t)ncomp * (l + 1) * c.N; }
 void rescale_core(Context& c, const uint64_t* x, int l, int ncomp, uint64_t* out, uint64_t* work, hipStream_t st);
 // fh_noalloc.hip: Rescale through a fixed per-device array (no allocation); noalloc_init looks the
-// array's device address up for the current device and records the device in the context.
+// array's device address up for the current device, loads the kernels and records the device in the
+// context.
 void noalloc_init(Context& c);
 size_t noalloc_scratch_words();
 void rescale_noalloc(Context& c, const uint64_t* x, int l, int ncomp, uint64_t* out, hipStream_t st);

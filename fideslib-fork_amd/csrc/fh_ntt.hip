@@ -6,6 +6,8 @@
 
 namespace fh {
 
+void ntt_load() { load_unit(); }
+
 void ntt_fwd(const Context& c, const LimbSet& s, hipStream_t st) { dispatch_fwd(c, SetAddr{s}, SetAddr{s}, s.nlimbs * s.npolys, st); }
 void ntt_inv(const Context& c, const LimbSet& s, hipStream_t st) { dispatch_inv(c, SetAddr{s}, SetAddr{s}, s.nlimbs * s.npolys, st); }
 void ntt_fwd(const Context& c, const LimbSet& in, const LimbSet& out, hipStream_t st) {

@@ -1330,6 +1330,12 @@ __global__ void k_zero_u32(uint32_t* p, uint32_t n) {
   for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
 }
 
+// loads the code object of the unit that includes this on the current device
+inline void load_unit() {
+  hipFuncAttributes a;
+  FH_HIP(hipFuncGetAttributes(&a, reinterpret_cast<const void*>(&k_zero_u32)));
+}
+
 // the team form applies to N = S x S with whole columns per tile (S >= 64), outside graph capture
 // (the launch is cooperative)
 template <int L1S, int L2S>

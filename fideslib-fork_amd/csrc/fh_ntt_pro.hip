@@ -4,6 +4,8 @@
 
 namespace fh {
 
+void ntt_pro_load() { load_unit(); }
+
 void ntt_fwd_rescale(const Context& c, const LimbSet& e, const uint64_t* top, const uint64_t* x, uint32_t l, uint64_t* out, hipStream_t st) {
   const size_t o = (size_t)l * c.L1;
   EpiRescale ep{x, out, c.d_rs_qlinv + o, c.d_rs_qlinv_sh + o, l, e.npolys, nullptr, nullptr, 0, 0, 0};

@@ -1,6 +1,10 @@
 """fh_rescale_noalloc (Rescale through the library's fixed per-device array, no allocation) against
 fh_rescale and the oracle, bit for bit, on two calls in a row (the second smaller, so it runs over
 the first call's leftovers in the shared array), plus its size and overlap contract."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -46,3 +50,42 @@ def test_rescale_noalloc_contract(gctx1, gctx2, octx1, fh):
     gctx1.rescale_noalloc(d1, 3, 2, out1)
     assert np.array_equal(out1.download(), o.rescale_ct(x, 3, 2))
     d1.free(); out1.free()
+
+
+FIRST_CALL = """
+import ctypes, sys
+sys.path.insert(0, sys.argv[1])
+import fides_hip as fh
+
+class Map(ctypes.Structure):
+    pass
+Map._fields_ = [("addr", ctypes.c_uint64), ("name", ctypes.c_char_p), ("dyn", ctypes.c_void_p), ("next", ctypes.POINTER(Map)), ("prev", ctypes.POINTER(Map))]
+class Debug(ctypes.Structure):
+    _fields_ = [("version", ctypes.c_int), ("map", ctypes.POINTER(Map))]
+
+def loaded():
+    # the code objects on the device, by the list the HSA runtime keeps for debuggers (laid out as the ELF r_debug)
+    p, n = Debug.in_dll(ctypes.CDLL("libhsa-runtime64.so.1"), "_amdgpu_r_debug").map, 0
+    while p:
+        p, n = p.contents.next, n + 1
+    return n
+
+g = fh.Context(13, 4, 2, 2)
+x, out = g.array((8, g.N)), g.array((8, g.N))
+g.fill_uniform(x, [0, 1, 2, 3], num_polys=2)
+g.sync()
+print(loaded())
+for f in (lambda: g.rescale_noalloc(x, 3, 2, out), lambda: g.rescale(x, 3, 2, out), lambda: g.mod_raise(x, 0, 2, 3, out), lambda: g.ntt_forward(out, [0, 1, 2, 3])):
+    f()
+    g.sync()
+    print(loaded())
+"""
+
+
+def test_first_rescale_loads_no_code(fh):
+    """In a fresh process the first allocation-free Rescale finds its kernels on the device (loading a code
+    object allocates device memory), and so do the first Rescale, ModRaise and transform."""
+    r = subprocess.run([sys.executable, "-c", FIRST_CALL, os.path.dirname(fh.__file__)], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr
+    counts = [int(v) for v in r.stdout.split()]
+    assert len(counts) == 5 and counts[0] > 0 and len(set(counts)) == 1, counts
