@@ -124,3 +124,53 @@ def test_team_ntt_other_ring_sizes(fh, oracle_mod, logN):
         d.free()
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("logN", [12, 16])
+def test_team_limbs_formed_in_the_first_launch(fh, oracle_mod, logN):
+    """Raised towers, residues of signed coefficients and the Rescale correction (one ciphertext and a
+    batch's job tables), formed in the first pass of a team launch."""
+    L1, K = 5, 1
+    g = fh.Context(logN, L1, K, 2)
+    try:
+        o = oracle_mod.Ctx(logN, [int(q) for q in g.moduli], L1, K, 2)
+        l, ids = L1 - 1, list(range(L1))
+        ct, ct2 = (np.concatenate([o.random_poly(s + i, ids) for i in range(2)]) for s in (500, 510))
+        rng = np.random.default_rng(6)
+        m = rng.integers(-(1 << 62), 1 << 62, (3, o.N))
+        z = rng.uniform(-1, 1, o.N // 2) + 1j * rng.uniform(-1, 1, o.N // 2)
+        pt = o.random_poly(520, ids)
+        g.tune_set("ntt_team", 1)
+        g.profile()
+        g.profile_reset()
+        d, up, enc, slots = g.to_device(ct), g.array((2 * L1, o.N)), g.array((3 * (L1 + K), o.N)), g.array((L1, o.N))
+        for what in ("mod_raise", "coeffs", "slots", "rescale", "batch"):
+            print(f"[team ntt logN={logN}] {what}", flush=True)
+            if what == "mod_raise":
+                g.mod_raise(d, l, 2, l, up)
+                assert np.array_equal(up.download(), o.mod_raise(ct, l, l, 2))
+            elif what == "coeffs":
+                pids = list(range(L1 + K))
+                g.encode_coeffs(m, pids, enc)
+                res = np.array([[[int(v) % int(q) for v in row] for q in g.moduli] for row in m], dtype=np.uint64)
+                assert np.array_equal(enc.download().reshape(res.shape), np.stack([o.ntt(r, pids) for r in res]))
+            elif what == "slots":
+                g.encode_slots(z, 2.0 ** 50, ids, slots)
+                assert np.array_equal(slots.download(), o.encode(z, 2.0 ** 50, l))
+            elif what == "rescale":
+                out = g.array((2 * l, o.N))
+                g.rescale(d, l, 2, out)
+                assert np.array_equal(out.download(), o.rescale_ct(ct, l, 2))
+            else:
+                b, d2, dp, o1, o2 = fh.Batch(g), g.to_device(ct2), g.to_device(pt), g.array((2 * l, o.N)), g.array((2 * l, o.N))
+                b.mult_plain(d.addr(), dp.addr(), l, True, o1.addr())
+                b.mult_plain(d2.addr(), dp.addr(), l, True, o2.addr())
+                b.run()
+                for src, got in ((ct, o1), (ct2, o2)):
+                    prod = np.concatenate([o.mul(src[:L1], pt), o.mul(src[L1:], pt)])
+                    assert np.array_equal(got.download(), o.rescale_ct(prod, l, 2))
+                b.free()
+        assert g.profile_read("ntt_fwd_team")[0] == 3 and g.profile_read("ntt_fwd_team_rescale")[0] == 2
+        assert g.profile_read("ntt_fwd_cols")[0] == 0
+    finally:
+        g.close()
