@@ -1337,11 +1337,13 @@ inline void load_unit() {
 }
 
 // the team form applies to N = S x S with whole columns per tile (S >= 64), outside graph capture
-// (the launch is cooperative)
+// (the launch is cooperative) and on the context's own stream alone: every launch of a context uses its
+// one set of arrival counters, which a launch on the second stream (half of a batched rotation) would
+// reset and count on while the first is running
 template <int L1S, int L2S>
 inline bool team_ok(const Context& c, hipStream_t st) {
   if constexpr (L1S != L2S || L1S < 6) return false;
-  if (!c.tune.ntt_team) return false;
+  if (!c.tune.ntt_team || st != c.stream) return false;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   FH_HIP(hipStreamIsCapturing(st, &cs));
   return cs == hipStreamCaptureStatusNone;

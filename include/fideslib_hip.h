@@ -438,8 +438,9 @@ int fh_profile_read(fh_context* ctx, const char* name, int* launches, double* to
  *   "ntt_streams"           1/2: the chunks of a chunked NTT alternate between two streams
  *   "ntt_team"              0/1: NTTs over N = S x S run as one cooperative launch of workgroup
  *                           teams, one HBM round trip per limb (the intermediate stays in the L2 of
- *                           the team's XCD); outside HIP graph capture; basis conversions are
- *                           launches of their own then
+ *                           the team's XCD); outside HIP graph capture and on the context
+ *                           stream (not in the second half of a rotation under rot_streams 2);
+ *                           basis conversions are launches of their own then
  *   "ntt_team_per_xcd"      teams per XCD of such a launch (1..64) */
 int fh_tune_set(fh_context* ctx, const char* name, int value);
 int fh_tune_get(const fh_context* ctx, const char* name, int* value);

@@ -174,3 +174,33 @@ def test_team_limbs_formed_in_the_first_launch(fh, oracle_mod, logN):
         assert g.profile_read("ntt_fwd_cols")[0] == 0
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("B", [9, 20])
+def test_team_rotations_on_two_streams(fh, oracle_mod, B):
+    """Half of the batch is on the context's second stream: it takes the two-launch form, since the context
+    has one set of team counters and a team launch of the first half may be running."""
+    logN, L1, K, dnum = 12, 6, 3, 2
+    g = fh.Context(logN, L1, K, dnum)
+    try:
+        o = oracle_mod.Ctx(logN, [int(q) for q in g.moduli], L1, K, dnum)
+        l, ids = L1 - 1, list(range(L1))
+        key = o.random_poly(700, list(range(L1 + K)) * (2 * dnum))
+        cts = [np.concatenate([o.random_poly(710 + i % 3, ids), o.random_poly(720 + i % 3, ids)]) for i in range(B)]
+        k, dk, d, out = o.rot_index(3), g.key(key), g.to_device(np.concatenate(cts)), g.array((B * 2 * L1, o.N))
+        exp = [o.eval_rotate(cts[i], l, key, k) for i in range(3)]
+        g.tune_set("ntt_team", 1)
+        g.tune_set("rot_streams", 2)
+        g.profile()
+        for rep in range(2):
+            print(f"[team ntt] {B} rotations on two streams, run {rep}", flush=True)
+            g.profile_reset()
+            g.rotate_batch(d, B, l, [dk] * B, [k] * B, out)
+            g.sync()
+            got = out.download().reshape(B, 2 * L1, o.N)
+            for i in range(B):
+                assert np.array_equal(got[i], exp[i % 3]), (rep, i)
+            # the inverse transforms of ModUp and ModDown, once per half
+            assert (g.profile_read("ntt_inv_team")[0], g.profile_read("ntt_inv_rows")[0]) == (2, 2)
+    finally:
+        g.close()
