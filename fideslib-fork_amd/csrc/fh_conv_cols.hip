@@ -23,10 +23,19 @@
 //    One workgroup of 8 waves per CU: the loop is bound by vector instructions and stores, has eight
 //    independent butterflies in flight per lane and two barriers per group.
 //
-// Measured at N=2^16, 9 sources: 64 rotations (4928 ModUp and 3200 ModDown targets) 2.75 ms for what
-// took 3.70 ms in four launches (two conversions, two column passes); one rotation 70 us against 92.
-// Vector instructions issue in 64% of the cycles, matrix instructions in 15%; 5.7 GB move instead of
-// 14.2. Each spilled register or wait for an earlier store in the loop showed (3.3 ms at first).
+// Measured at N=2^16, 9 sources: 64 rotations (4928 ModUp and 3200 ModDown targets) 2.69 ms (1671 and
+// 1017 us); two conversions and two column passes took 3.77 ms before the column passes' present 60-bit
+// arithmetic. 5.7 GB move instead of 14.2: 1.1 ms at the copy rate. Vector instructions issue in 61% of
+// the cycles (113 and 100 per target word, the column stages among them), matrix instructions in 15%.
+// Each spilled register or wait for an earlier store in the loop showed (3.3 ms at first). With 13 to 16
+// sources 35 registers spill at N=2^16 (11 at 2^14, 9 at 2^15, none below).
+//
+// Against the separate launches by number of sources (both in one build, N = 2^12 .. 2^16, two digits,
+// 50-bit targets): one rotation, and 16 in one batch, are faster by the factors
+//   2: 0.86-0.92, 0.88-1.02    5: 1.00-1.09, 1.03-1.09    9: 1.06-1.13, 1.05-1.11    13: 1.12-1.27, 1.16-1.30
+//   3: 0.91-0.99, 0.92-1.02    6: 1.02-1.07, 1.04-1.10   12: 1.08-1.27, 1.08-1.19    16: 1.12-1.39, 1.16-1.33
+//   4: 0.93-1.01, 0.98-1.05    8: 1.08-1.15, 1.07-1.12
+// (59-bit targets, 2 .. 4 sources: 0.93-0.98 and 0.97-1.10, 0.98-1.04 and 0.97-1.06, 1.00-1.07 and 1.04-1.10.)
 #include "fh_keyswitch.hpp"
 #include "fh_ntt_impl.hpp"
 
@@ -474,9 +483,10 @@ ConvJobs conv_jobs(const Context& c, bool down) {
 }  // namespace
 
 bool conv_cols_usable(const Context& c, int sources) {
-  // Two sources cost the plain conversion four products per output, and its two launches at N=2^13
-  // take 11.7 us where this one takes 15.8 (a single small ciphertext); from four sources on (N=2^15,
-  // digits of 4) one launch is the faster.
+  // Two sources cost the plain conversion four products per output, and a rotation is up to 14% faster
+  // with its two launches (N=2^13: 64 us against 75). Five and more gain. At three and four it depends on
+  // the launch: a single call loses up to 9% (N=2^13, three sources: 68 us against 74), most batches and
+  // all of 59-bit targets gain up to 6%; they run fused. Figures above.
   return sources > 2 && c.conv_cols_ok && !c.reduced_noise && !c.tune.ntt_team && (!c.tune.ntt_split || c.tune.ntt_split == ntt_default_split(c.logN));
 }
 

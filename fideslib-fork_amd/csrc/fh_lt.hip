@@ -117,7 +117,9 @@ struct MacParams {
 // multiply policy M and reduced once. The rotations never reach memory.
 // Up to four digits four waves a SIMD are asked for: left alone the compiler takes 133 registers for
 // eight baby steps, which is three waves (28 bytes spilled; 63 diagonals in 16 baby steps 1319 -> 1270
-// us); with more digits that would spill 156 bytes.
+// us). With more digits that would spill 156 bytes, and the compiler's own choice is the faster one: 32
+// diagonals in 16 baby steps, N = 2^16, 24 limbs, six digits 1094 us (four waves: 1445), eight digits 1230
+// (1685).
 template <int BB, class M, int DM>
 __global__ __launch_bounds__(kT, DM <= 4 ? 4 : 1) void k_lt_mac(Hoist h, const uint64_t* __restrict__ diags, uint64_t* __restrict__ R, MacParams mp) {
   using Op = typename M::Op;

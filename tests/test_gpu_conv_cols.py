@@ -56,6 +56,32 @@ def test_modup_moddown(fh, oracle_mod, shape):
         g.close()
 
 
+# the operand sizes at the rings that the shapes above leave out (at N=2^14 and more the largest keeps
+# some of its operands in scratch memory)
+@pytest.mark.parametrize("shape", [(13, 26, 13, 2), (14, 18, 9, 2), (15, 18, 9, 2), (15, 29, 15, 2), (16, 24, 12, 2), (16, 31, 16, 2)],
+                         ids=lambda s: f"n{s[0]}-q{s[1]}-p{s[2]}-d{s[3]}")
+def test_modup_moddown_at_the_top_level(fh, oracle_mod, shape):
+    logN, L1, K, dnum = shape
+    g = fh.Context(logN, L1, K, dnum)
+    try:
+        o = oracle_mod.Ctx(logN, [int(q) for q in g.moduli], L1, K, dnum)
+        qs, l = np.array([int(m) for m in g.moduli], dtype=np.uint64), L1 - 1
+        ids, eids, ext = list(range(L1)), o.ext_pids(l), L1 + K
+        top = lambda pids: np.ascontiguousarray(np.broadcast_to(qs[pids][:, None] - np.uint64(1), (len(pids), o.N)))
+        for i, (x, xe) in enumerate([(o.random_poly(50, ids), o.random_poly(70, eids)), (o.ntt(top(ids), ids), o.ntt(top(eids), eids))]):
+            print(f"[conv cols] {shape} input {i}", flush=True)
+            d, dig = g.to_device(x), g.array((o.num_digits(l) * ext, o.N))
+            g.modup(d, l, dig)
+            assert np.array_equal(dig.download(), o.modup(x, l)), i
+            de, out = g.to_device(xe), g.array((L1, o.N))
+            g.moddown(de, l, 1, out)
+            assert np.array_equal(out.download(), o.moddown(xe, l)), i
+            for a in (d, dig, de, out):
+                a.free()
+    finally:
+        g.close()
+
+
 def test_many_polynomials(fh, oracle_mod):
     """Launches of one chunk of targets per workgroup and of several, and the job tables of a mixed-level
     batch, give the same rotation."""
