@@ -210,7 +210,8 @@ void encode_slots(Context& c, const double* values, int count, uint32_t slots, d
   int logn = 0;
   while ((1u << logn) < n) ++logn;
   const int logM = c.logN + 1, loggap = c.logN - 1 - logn;
-  DBuf vals(c.pool, (size_t)count * n * 2), work(c.pool, (size_t)count * n * 2), coef(c.pool, (size_t)count * c.N);
+  // coef: a chunk's slot values (at most N words a plaintext), once they are in `work` its coefficients
+  DBuf work(c.pool, (size_t)count * n * 2), coef(c.pool, (size_t)count * c.N);
   const double2* tw = reinterpret_cast<const double2*>(c.d_ifft_w);
   // chunks of about 8 MB of slot values: the upload of one chunk (synchronous for pageable host
   // memory) overlaps the transforms of the previous one
@@ -218,7 +219,7 @@ void encode_slots(Context& c, const double* values, int count, uint32_t slots, d
   HostReads reads(st);
   for (int b0 = 0; b0 < count; b0 += chunk) {
     const int nb = std::min(chunk, count - b0);
-    double* v = reinterpret_cast<double*>(vals.p) + (size_t)b0 * n * 2;
+    double* v = reinterpret_cast<double*>(coef.p) + (size_t)b0 * c.N;
     D2* wk = reinterpret_cast<D2*>(work.p) + (size_t)b0 * n;
     reads.copy(v, values + (size_t)b0 * n * 2, (size_t)nb * n * 2 * sizeof(double));
     ProfScope ps_(c, "encode", st);

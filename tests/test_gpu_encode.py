@@ -118,3 +118,30 @@ def test_input_is_read_when_the_call_returns(form, gctx2, fh):
     for a in (ref, got, busy):
         a.free()
     assert hip.hipHostFree(p) == 0
+
+
+def test_encode_scratch(fh, oracle_mod):
+    """Full-slot values take two buffers of N words a plaintext: the values, where their coefficients follow,
+    and the transform's."""
+    logN, count = 13, 512
+    g = fh.Context(logN, 1, 1, 1)
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert fh.load().hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    try:
+        o = oracle_mod.Ctx(logN, [int(q) for q in g.moduli], 1, 1, 1)
+        z = _values(g.N // 2, 3, count)
+        out = g.array((count, g.N))
+        g.encode_slots(z[:1], 2.0 ** 40, [0], out)      # tables and code of the encoder
+        g.sync()
+        before = free()
+        g.encode_slots(z, 2.0 ** 40, [0], out)
+        got = out.download()
+        assert before - free() <= 2 * 8 * g.N * count + (4 << 20)
+        for b in (0, 63, 64, count - 1):
+            assert np.array_equal(got[b:b + 1], o.encode(z[b], 2.0 ** 40, 0)), b
+    finally:
+        g.close()
