@@ -225,9 +225,10 @@ def main():
         ctx.rotate_batch(cts, B, lvl, ks, gs, out_b)
     ctx.sync()
     t_batched = time.perf_counter() - t0
-    # *_conv_cols: a basis conversion and its targets' column pass in one launch
+    # *_conv_cols: a basis conversion and its targets' column pass in one launch; under tunables that turn
+    # that off, *_conv and ntt_fwd_cols
     fams = ["ntt_inv_rows", "ntt_inv_cols", "modup_conv_cols", "ntt_fwd_rows", "ksk_batch", "moddown_conv_cols",
-            "ntt_fwd_rows_moddown", "ntt_rows_ksk"]
+            "ntt_fwd_rows_moddown", "ntt_rows_ksk", "modup_conv", "moddown_conv", "ntt_fwd_cols"]
     prof = {f: ctx.profile_read(f) for f in fams}
     ctx.profile(False)
     ms_per_step = 1000.0 * t_batched / a.steps
